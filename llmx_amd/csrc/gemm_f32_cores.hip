@@ -1,0 +1,401 @@
+// The true 32-bit path's products on the matrix cores: C[M,N] (+)= A[M,K] * W[N,K]^T, all float32, dense or grouped, with the
+// universal product's epilogues (v_mfma_f32_16x16x4_f32 multiplies and adds full float32 values; it has no reduced-precision mode).
+//
+// Two forms give an element the same bits.  K is cut into `ks` runs of whole steps of 16 (a function of N and K alone), a run is
+// one accumulator walked over its steps in order, W as the instruction's A operand, and the runs' sums are added in order; so a
+// row's bits depend on its own values and the weights only, not on the rows beside it or on the form.
+//
+//  * stream: few rows.  The weights' way from memory bounds it: a workgroup's `ks` waves share a strip of 16 features, one run of
+//    K each, and ask for a round of steps while the round before is multiplied.  1 row: 32,768 features of 2,048 values 56 us (4.8
+//    TB/s), 8,192 of 3,072 22 us, 3,072 of 2,048 12.8 us; the universal product takes 0.2-0.5 ms for the smallest of these.
+//  * tiles: many rows.  The instruction's rate bounds it (140 TFLOP/s measured alone): 64 rows x 128 (64) features a workgroup,
+//    operands staged through LDS 32 values of k at a time, a wave 32 x 32, its runs folded in registers.  2,048 rows: 8,192 features
+//    of 3,072 values 0.78 ms (132 TFLOP/s); 333 rows of 2,048 values: 32,768 features 0.44 ms (102 TFLOP/s), where the universal
+//    product reaches 8 TFLOP/s.  Chunks asked for two ahead instead of one: 0.84 -> 0.78 ms and 0.47 -> 0.44 ms.
+#include "gemm_args.h"
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// What an output element gets; `up` counts for the gated epilogue only.
+template <int EPI>
+__device__ __forceinline__ void f32_store_quad(const GemmArgs& g, const ActFn& act, int row, int n, f32x4_t v, f32x4_t up) {
+    const GluRow glu(g.glu, EPI == EPI_SWIGLU ? row : 0);
+    float* c = (float*)g.C + (size_t)row * g.ldc + n;
+    const bool whole = n + 3 < g.N && g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;
+    f32x4_t old = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (EPI == EPI_ADD && whole) old = *reinterpret_cast<const f32x4_t*>(c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (EPI == EPI_SWIGLU) {
+            v[i] = glu(v[i], up[i]);
+            continue;
+        }
+        v[i] = llmx_act_reads_vector(act.kind) ? biased_act(act.kind, v[i], act_feature(act.kind, g.act_params, n + i, g.N)) : act(v[i]);
+        if (EPI == EPI_ADD) v[i] = (whole ? old[i] : n + i < g.N ? c[i] : 0.0f) + v[i];
+    }
+    if (whole) {
+        *reinterpret_cast<f32x4_t*>(c) = v;
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n + i < g.N) c[i] = v[i];
+}
+
+// Grid: dense (strips, chunks of 16 MT rows); grouped (strips, groups, row chunks of a group).
+template <int KS, int MT, int EPI>
+__global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
+    constexpr int NS = EPI == EPI_SWIGLU ? 2 : 1;                  // weight strips: the features', and the up rows' of the same features
+    constexpr int UN = NS * MT == 1 ? 8 : NS * MT == 2 ? 4 : 2;    // steps of a round: its loads travel together
+    __shared__ __attribute__((aligned(16))) float red[KS > 1 ? KS : 1][NS * MT][256];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = lane & 15, kg = lane >> 4;
+    const int n0 = blockIdx.x * 16, K = g.K;
+    const float* A = (const float*)g.A;
+    const float* W = (const float*)g.W;
+    int row_end = g.M, m0 = blockIdx.y * 16 * MT, m_step = gridDim.y * 16 * MT;
+    if (g.group_offsets) {
+        m0 = g.group_offsets[blockIdx.y] + blockIdx.z * 16 * MT;
+        row_end = g.group_offsets[blockIdx.y + 1];
+        m_step = gridDim.z * 16 * MT;
+        W += (size_t)blockIdx.y * g.w_group_stride;
+    }
+    const int steps = (K + 15) >> 4, per = (steps + KS - 1) / KS, ranges = (steps + per - 1) / per;
+    const int s_begin = min(steps, wave * per), s_end = min(steps, s_begin + per);
+    const int whole_end = min(s_end, K >> 4);                      // steps before this one are whole
+    const float* wp[NS];
+#pragma unroll
+    for (int ns = 0; ns < NS; ++ns) wp[ns] = W + (size_t)(min(n0 + r, g.N - 1) + (ns ? g.up_offset : 0)) * g.ldw + kg * 4;
+    const ActFn act(EPI != EPI_SWIGLU ? g.act : LLMX_ACT_NONE, g.act_params);
+
+    for (; m0 < row_end; m0 += m_step) {
+        // a row past the last reads the last one: what its column of the product gives is never stored
+        const float* ap[MT];
+        int row_c[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const int m = min(m0 + 16 * t + r, row_end - 1);
+            row_c[t] = g.group_offsets ? g.list[m] : m;
+            ap[t] = A + (size_t)(g.group_offsets ? row_c[t] / g.a_div : m) * g.lda + kg * 4;
+        }
+        f32x4_t acc[NS][MT];
+#pragma unroll
+        for (int ns = 0; ns < NS; ++ns)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        struct Round {
+            f32x4_t w[UN][NS], a[UN][MT];
+        };
+        auto fetch = [&](Round& f, int s) {
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const size_t at = (size_t)max(min(s + u, whole_end - 1), 0) * 16;      // past the end: a step fetched before, not multiplied
+#pragma unroll
+                for (int ns = 0; ns < NS; ++ns) f.w[u][ns] = *reinterpret_cast<const f32x4_t*>(wp[ns] + at);
+#pragma unroll
+                for (int t = 0; t < MT; ++t) f.a[u][t] = *reinterpret_cast<const f32x4_t*>(ap[t] + at);
+            }
+        };
+        auto multiply = [&](const f32x4_t (&w)[NS], const f32x4_t (&a)[MT]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int ns = 0; ns < NS; ++ns)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) acc[ns][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[ns][i], a[t][i], acc[ns][t], 0, 0, 0);
+        };
+        auto round = [&](const Round& f, int s) {
+#pragma unroll
+            for (int u = 0; u < UN; ++u)
+                if (s + u < whole_end) multiply(f.w[u], f.a[u]);
+        };
+        if (s_begin < whole_end) {
+            Round first, second;
+            fetch(first, s_begin);
+            for (int s = s_begin; s < whole_end; s += 2 * UN) {
+                fetch(second, s + UN);
+                round(first, s);
+                fetch(first, s + 2 * UN);
+                round(second, s + UN);
+            }
+        }
+        if (s_end > whole_end) {       // K's last step holds 4, 8 or 12 values
+            const bool in = whole_end * 16 + 4 * kg < K;
+            f32x4_t w[NS], a[MT];
+#pragma unroll
+            for (int ns = 0; ns < NS; ++ns) w[ns] = in ? *reinterpret_cast<const f32x4_t*>(wp[ns] + (size_t)whole_end * 16) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int t = 0; t < MT; ++t) a[t] = in ? *reinterpret_cast<const f32x4_t*>(ap[t] + (size_t)whole_end * 16) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            multiply(w, a);
+        }
+        if (KS > 1) {
+#pragma unroll
+            for (int ns = 0; ns < NS; ++ns)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4_t*>(&red[wave][ns * MT + t][lane * 4]) = acc[ns][t];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            if (t % KS != wave) continue;
+            f32x4_t v[NS];
+#pragma unroll
+            for (int ns = 0; ns < NS; ++ns) {
+                v[ns] = acc[ns][t];
+                if (KS > 1) {
+                    v[ns] = *reinterpret_cast<f32x4_t*>(&red[0][ns * MT + t][lane * 4]);
+                    for (int w = 1; w < ranges; ++w) {
+                        const f32x4_t o = *reinterpret_cast<f32x4_t*>(&red[w][ns * MT + t][lane * 4]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[ns][i] += o[i];
+                    }
+                }
+            }
+            if (m0 + 16 * t + r < row_end) f32_store_quad<EPI>(g, act, row_c[t], n0 + 4 * kg, v[0], v[NS - 1]);
+        }
+        if (KS > 1) __syncthreads();
+    }
+}
+
+// K a multiple of 16.  A workgroup takes 64 rows and BN weight rows (gated: BN / 2 features' gate and up rows); grid (feature tiles,
+// row tiles), grouped: the row tiles of the groups that have rows, in order.  A staged row takes 32 values of k and 4 of padding, so
+// that 8 rows' 16-byte pieces fall into different banks; the next chunk travels while this one is multiplied.
+#define FT_ROWS 64
+#define FT_PITCH 36
+template <int EPI, int BN>
+__global__ void __launch_bounds__(4 * BN) gemm_f32_tiles_kernel(GemmArgs g, int ks, int n_groups) {
+    constexpr int THREADS = 4 * BN, WAVES = THREADS / 64;
+    constexpr int A_PIECES = FT_ROWS * 8 / THREADS, ROWS_A_PASS = THREADS / 8;       // 16-byte pieces of a chunk a thread brings: 2 of W's
+    __shared__ __attribute__((aligned(16))) float Ws[2][BN * FT_PITCH];
+    __shared__ __attribute__((aligned(16))) float As[2][FT_ROWS * FT_PITCH];
+    __shared__ int rows_a[FT_ROWS], rows_c[FT_ROWS], tile_info[3], scan_waves[WAVES];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int r = lane & 15, kg = lane >> 4;
+    const int wn = wave % (BN / 32), wm = wave / (BN / 32);
+    constexpr int FEATS = EPI == EPI_SWIGLU ? BN / 2 : BN;
+    const int n0 = blockIdx.x * FEATS, K = g.K;
+    const float* W = (const float*)g.W;
+    int row_begin = blockIdx.y * FT_ROWS, row_end = g.M;
+    if (g.group_offsets) {
+        // which group's which tile: the groups' tile counts scanned by all threads together
+        if (tid == 0) tile_info[0] = -1;
+        int base = 0;
+        for (int e0 = 0; e0 < n_groups; e0 += THREADS) {
+            const int e = e0 + tid;
+            const int begin = e < n_groups ? g.group_offsets[e] : 0, end = e < n_groups ? g.group_offsets[e + 1] : 0;
+            const int tiles = (end - begin + FT_ROWS - 1) / FT_ROWS;
+            int incl = tiles;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(incl, d, 64);
+                if (lane >= d) incl += o;
+            }
+            if (lane == 63) scan_waves[wave] = incl;
+            __syncthreads();
+            int before = base;
+            for (int w = 0; w < WAVES; ++w) {
+                if (w < wave) before += scan_waves[w];
+                base += scan_waves[w];
+            }
+            const int first = before + incl - tiles;
+            if ((int)blockIdx.y >= first && (int)blockIdx.y < first + tiles) {
+                tile_info[0] = e;
+                tile_info[1] = begin + ((int)blockIdx.y - first) * FT_ROWS;
+                tile_info[2] = end;
+            }
+            __syncthreads();
+            if ((int)blockIdx.y < base) break;
+        }
+        if (tile_info[0] < 0) return;
+        row_begin = tile_info[1];
+        row_end = tile_info[2];
+        W += (size_t)tile_info[0] * g.w_group_stride;
+    }
+    if (tid < FT_ROWS) {
+        const int m = min(row_begin + tid, row_end - 1);
+        const int p = g.group_offsets ? g.list[m] : m;
+        rows_a[tid] = g.group_offsets ? p / g.a_div : m;      // a row past the last reads the last one and is not stored
+        rows_c[tid] = row_begin + tid < row_end ? p : -1;
+    }
+    __syncthreads();
+    const int piece = tid & 7, prow = tid >> 3;
+    const float* w_src[2];
+    const float* a_src[A_PIECES];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int w = prow + ROWS_A_PASS * j;
+        // gated: rows 32 q .. + 15 of the tile are features 16 q .. + 15's gate rows, the next 16 their up rows
+        const int f = EPI == EPI_SWIGLU ? n0 + 16 * (w >> 5) + (w & 15) : n0 + w;
+        w_src[j] = W + (size_t)(min(f, g.N - 1) + (EPI == EPI_SWIGLU && (w & 16) ? g.up_offset : 0)) * g.ldw + 4 * piece;
+    }
+#pragma unroll
+    for (int j = 0; j < A_PIECES; ++j) a_src[j] = (const float*)g.A + (size_t)rows_a[prow + ROWS_A_PASS * j] * g.lda + 4 * piece;
+    struct Fetched {
+        f32x4_t w[2], a[A_PIECES];
+    };
+    auto fetch = [&](int c, Fetched& f) {
+        const int kk = min(32 * c, K - 16 - 16 * (piece >> 2));      // K's last chunk may hold one step: the second is fetched from inside K and not multiplied
+#pragma unroll
+        for (int j = 0; j < 2; ++j) f.w[j] = *reinterpret_cast<const f32x4_t*>(w_src[j] + kk);
+#pragma unroll
+        for (int j = 0; j < A_PIECES; ++j) f.a[j] = *reinterpret_cast<const f32x4_t*>(a_src[j] + kk);
+    };
+    auto stage = [&](const Fetched& f, int buf) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<f32x4_t*>(&Ws[buf][(prow + ROWS_A_PASS * j) * FT_PITCH + 4 * piece]) = f.w[j];
+#pragma unroll
+        for (int j = 0; j < A_PIECES; ++j) *reinterpret_cast<f32x4_t*>(&As[buf][(prow + ROWS_A_PASS * j) * FT_PITCH + 4 * piece]) = f.a[j];
+    };
+    const int steps = K >> 4, per = (steps + ks - 1) / ks, chunks = (steps + 1) / 2;
+    f32x4_t total[2][2], acc[2][2];
+#pragma unroll
+    for (int ns = 0; ns < 2; ++ns)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[ns][t] = total[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    bool first_run = true;
+    int in_run = 0;
+    auto multiply = [&](int c, int buf) {
+        f32x4_t wf[2][2], af[2][2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int ns = 0; ns < 2; ++ns) wf[u][ns] = *reinterpret_cast<const f32x4_t*>(&Ws[buf][(32 * wn + 16 * ns + r) * FT_PITCH + 16 * u + 4 * kg]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) af[u][t] = *reinterpret_cast<const f32x4_t*>(&As[buf][(32 * wm + 16 * t + r) * FT_PITCH + 16 * u + 4 * kg]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int s = 2 * c + u;
+            if (s >= steps) break;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int ns = 0; ns < 2; ++ns)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) acc[ns][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][ns][i], af[u][t][i], acc[ns][t], 0, 0, 0);
+            if (++in_run == per || s + 1 == steps) {
+#pragma unroll
+                for (int ns = 0; ns < 2; ++ns)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) total[ns][t][i] = first_run ? acc[ns][t][i] : total[ns][t][i] + acc[ns][t][i];
+                        acc[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+                first_run = false;
+                in_run = 0;
+            }
+        }
+    };
+    const ActFn act(EPI != EPI_SWIGLU ? g.act : LLMX_ACT_NONE, g.act_params);
+    // two chunks are on their way through two register sets while a third is multiplied (one ahead: 8% slower, a chunk's
+    // multiplications being shorter than the way to memory); past the end the last one again
+    Fetched even, odd;
+    fetch(0, even);
+    fetch(min(1, chunks - 1), odd);
+    stage(even, 0);
+    fetch(min(2, chunks - 1), even);
+    __syncthreads();
+    for (int c = 0; c < chunks; c += 2) {
+        multiply(c, 0);
+        stage(odd, 1);
+        fetch(min(c + 3, chunks - 1), odd);
+        __syncthreads();
+        if (c + 1 >= chunks) break;
+        multiply(c + 1, 1);
+        stage(even, 0);
+        fetch(min(c + 4, chunks - 1), even);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int row = rows_c[32 * wm + 16 * t + r];
+        if (row < 0) continue;
+        if (EPI == EPI_SWIGLU) {
+            const int n = n0 + 16 * wn + 4 * kg;
+            if (n < g.N) f32_store_quad<EPI>(g, act, row, n, total[0][t], total[1][t]);
+        } else {
+#pragma unroll
+            for (int ns = 0; ns < 2; ++ns) {
+                const int n = n0 + 32 * wn + 16 * ns + 4 * kg;
+                if (n < g.N) f32_store_quad<EPI>(g, act, row, n, total[ns][t], total[ns][t]);
+            }
+        }
+    }
+}
+
+// Runs K is cut into: enough strips x runs to keep the chip's waves streaming, at least 12 steps of 16 a run.  N and K only.
+static int f32_runs(int N, int K) {
+    const int strips = (N + 15) / 16, steps = K >> 4;
+    int ks = 1;
+    while (ks < 8 && strips * ks < 2048 && steps / (ks * 2) >= 12) ks *= 2;
+    return ks;
+}
+
+bool llmx_gemm_f32_cores_take(const GemmArgs& g, int n_groups) {
+    return g.K % 4 == 0 && g.lda % 4 == 0 && g.ldw % 4 == 0 && ((uintptr_t)g.A & 15) == 0 && ((uintptr_t)g.W & 15) == 0 &&
+           (n_groups == 0 || g.w_group_stride % 4 == 0);
+}
+
+template <int EPI>
+static int launch_stream(const GemmArgs& g, int n_groups, int ks, int rows_a_group, hipStream_t stream) {
+    const int mt = rows_a_group <= 16 ? 1 : rows_a_group <= 32 || EPI == EPI_SWIGLU ? 2 : 4;
+    int chunks = (rows_a_group + 16 * mt - 1) / (16 * mt);
+    const dim3 grid = n_groups ? dim3((g.N + 15) / 16, n_groups, chunks > 64 ? 64 : chunks) : dim3((g.N + 15) / 16, chunks > 4096 ? 4096 : chunks);
+#define F32_STREAM(KS, MT) hipLaunchKernelGGL((gemm_f32_stream_kernel<KS, MT, EPI>), grid, dim3(64 * KS), 0, stream, g)
+#define F32_STREAM_MT(KS)               \
+    do {                                \
+        if (mt == 1) F32_STREAM(KS, 1); \
+        else if (mt == 2) F32_STREAM(KS, 2); \
+        else if constexpr (EPI != EPI_SWIGLU) F32_STREAM(KS, 4); \
+    } while (0)
+    switch (ks) {
+        case 1: F32_STREAM_MT(1); break;
+        case 2: F32_STREAM_MT(2); break;
+        case 4: F32_STREAM_MT(4); break;
+        default: F32_STREAM_MT(8); break;
+    }
+#undef F32_STREAM_MT
+#undef F32_STREAM
+    return LLMX_CHECK_LAUNCH();
+}
+
+template <int EPI>
+static int launch_tiles(const GemmArgs& g, int n_groups, int ks, int row_tiles, hipStream_t stream) {
+    // 128 weight rows a workgroup read the activations half as often, 64 fill the chip with fewer rows.  Measured at K 2,048, 256
+    // CUs: with n workgroups a CU the narrow form takes about 22 + 33 n us (1: 56, 2: 87, 3: 121), the wide one 12 + 60 n (1: 72, 2: 131).
+    const int wide = EPI == EPI_SWIGLU ? 64 : 128, narrow = wide / 2;
+    const long n_wide = ((long)((g.N + wide - 1) / wide) * row_tiles + 255) / 256, n_narrow = ((long)((g.N + narrow - 1) / narrow) * row_tiles + 255) / 256;
+    if (12 + 60 * n_wide <= 22 + 33 * n_narrow)
+        hipLaunchKernelGGL((gemm_f32_tiles_kernel<EPI, 128>), dim3((g.N + wide - 1) / wide, row_tiles), dim3(512), 0, stream, g, ks, n_groups);
+    else
+        hipLaunchKernelGGL((gemm_f32_tiles_kernel<EPI, 64>), dim3((g.N + narrow - 1) / narrow, row_tiles), dim3(256), 0, stream, g, ks, n_groups);
+    return LLMX_CHECK_LAUNCH();
+}
+
+// Which form: the stream form multiplies at about 50 TFLOP/s beyond 16 rows (every strip reads the rows again), the tiles at 100 to
+// 130 but, at K 2,048, never in less than 56 us: they meet at rows x features of about 680,000 (3,072 features: 128 rows 47 against
+// 57 us, 256 rows 71 against 58; 8,192: 64 rows 73 against 82, 96 rows 120 against 86; 32,768: 16 rows 69 against 78, 48 rows 142
+// against 80).  Groups of at most half a tile of rows on average stay with the stream form, the tiles being mostly padding.
+template <int EPI>
+static int launch_f32(const GemmArgs& g, int n_groups, hipStream_t stream) {
+    const int ks = f32_runs(g.N, g.K);
+    const int rows = n_groups ? (g.M + n_groups - 1) / n_groups : g.M;      // grouped: a group's on average (the counts are on the device; both forms take any)
+    const int row_tiles = n_groups ? (n_groups < g.M ? n_groups : g.M) + g.M / FT_ROWS : (g.M + FT_ROWS - 1) / FT_ROWS;
+    const bool few = rows <= (n_groups ? FT_ROWS / 2 : 16) || (long)g.M * g.N <= 680000;
+    if (!few && g.K % 16 == 0 && row_tiles <= 65535) {
+        llmx_note_launch(LK_GEMM_GENERIC_TILES);
+        return launch_tiles<EPI>(g, n_groups, ks, row_tiles, stream);
+    }
+    llmx_note_launch(LK_GEMM_GENERIC_STREAM);
+    return launch_stream<EPI>(g, n_groups, ks, rows, stream);
+}
+
+int llmx_gemm_f32_cores(const GemmArgs& g, int epi, int n_groups, hipStream_t stream) {
+    switch (epi) {
+        case EPI_STORE: return launch_f32<EPI_STORE>(g, n_groups, stream);
+        case EPI_ADD: return launch_f32<EPI_ADD>(g, n_groups, stream);
+        case EPI_SWIGLU: return launch_f32<EPI_SWIGLU>(g, n_groups, stream);
+        default: return -1;
+    }
+}

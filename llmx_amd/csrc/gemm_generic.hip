@@ -3,33 +3,14 @@
 // Every output element is one accumulator walked over k = 0..K-1 with fmaf, so its bits depend only on its own
 // row of A and row of W: not on M, on the tile it falls in, or on its neighbours.  It takes any M, N, K, any of
 // f32/bf16 for A, W and C, rows of A gathered and rows of C scattered through index lists, and groups of rows
-// that each use their own weight matrix (routed experts).  It is the true 32-bit path's product and the
-// fallback of the bf16 path for shapes the MFMA kernels refuse.
-#include "common.h"
+// that each use their own weight matrix (routed experts).  It is the product of the shapes that the matrix-core kernels
+// refuse: rows of a length that is no multiple of 4, mixed types, misaligned operands.  Products of float32 operands that
+// allow 16-byte loads go to the 32-bit matrix instruction instead (gemm_f32_cores.hip).
+#include "gemm_args.h"
 
 #define GT_BM 64
 #define GT_BN 64
 #define GT_BK 16
-
-enum : int { EPI_STORE = 0, EPI_ADD = 1, EPI_SWIGLU = 2 };
-
-struct GemmArgs {
-    const void* A;
-    const void* W;
-    void* C;
-    int M, N, K;
-    int lda, ldw, ldc;
-    // Grouped mode (group_offsets != null): blockIdx.y is the group g; its rows are list[group_offsets[g] .. group_offsets[g+1]).
-    // A's row for list entry p is p / a_div, C's row is p.  Weights of group g start at W + g * w_group_stride elements.
-    const int* group_offsets;
-    const int* list;
-    int a_div;
-    long w_group_stride;
-    int up_offset;  // EPI_SWIGLU: W row n is the gate row, W row n + up_offset the up row
-    int act;        // EPI_STORE, EPI_ADD: an activation applied to the product (LLMX_ACT_*), with its parameters on the device
-    const float* act_params;
-    GluArgs glu;    // EPI_SWIGLU: the gated unit and its per-row values
-};
 
 template <typename TA, typename TW, typename TC, int EPI>
 __global__ void __launch_bounds__(256) gemm_generic_kernel(GemmArgs g) {
@@ -174,6 +155,8 @@ extern "C" int llmx_gemm_generic(const void* A, int a_dtype, const void* W, int 
                GluArgs{epi == EPI_SWIGLU ? glu_kind : LLMX_GLU_SILU, glu_limit, epi == EPI_SWIGLU ? glu_row_scale : nullptr,
                        epi == EPI_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld}};
     if (!llmx_act_fits(act, act_params, epi == EPI_STORE, epi == EPI_ADD)) return -2;
+    if (a_dtype == LLMX_F32 && w_dtype == LLMX_F32 && c_dtype == LLMX_F32 && llmx_gemm_f32_cores_take(g, n_groups))
+        return llmx_gemm_f32_cores(g, epi, n_groups, stream);
     dim3 grid;
     grid.x = (N + GT_BN - 1) / GT_BN;
     if (n_groups) {

@@ -13,6 +13,8 @@
     X(MOE_COMBINE, "moe_combine")                                                                                         \
     X(GEMM_GENERIC, "gemm_generic")                                                                                       \
     X(GEMM_GENERIC_GROUPED, "gemm_generic.grouped")                                                                       \
+    X(GEMM_GENERIC_STREAM, "gemm_generic.stream")                                                                         \
+    X(GEMM_GENERIC_TILES, "gemm_generic.tiles")                                                                           \
     X(GEMM_SKINNY, "gemm_skinny")                                                                                         \
     X(GEMM_SKINNY_TWO_STRIPS, "gemm_skinny.two_strips")                                                                   \
     X(GEMM_SKINNY_NORMED, "gemm_skinny.normed")                                                                           \
