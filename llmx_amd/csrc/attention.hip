@@ -1,5 +1,5 @@
 // Attention-side kernels: QK RMSNorm + partial rotary + KV page write, and the universal paged attention kernel.
-#include "common.h"
+#include "attention_args.h"
 
 // Per-step row plan shared by the attention kernels (device arrays made once a step):
 //   pos[t]        absolute position of row t in its request
@@ -434,26 +434,6 @@ extern "C" int llmx_gate_heads(void* o, int dtype, const float* gate, int ldg, i
 // `sink` (a logit a head) enters the softmax's denominator only.  `maps` > 1: a head has several score maps over one set of
 // values: q holds [head][map][D], the key cache [kv head][map] heads, and the output [head][map][VD].
 // A row's arithmetic depends on its own position and request only.  Values may have a width of their own (v_dim).
-struct AttnArgs {
-    const void* q;  // [T, n_heads * maps, head_dim]
-    const void* k_cache;
-    const void* v_cache;
-    const int* pos;
-    const int* row_entry;
-    const int* tables;
-    void* out;  // [T, n_heads * maps * v_dim]
-    float scale;
-    int n_heads, n_kv_heads, head_dim, page_tokens, max_blocks, window;
-    int v_dim;   // width of a value head (the output's too); keys and queries have head_dim
-    const float* gate;  // null, or float32 logits, row stride gate_ld: the output is multiplied by their sigmoid
-    int gate_ld;
-    int gate_wide;       // 0: a logit a (row, head); 1: a logit a (row, head, value dim)
-    int keep_first, chunk, maps;
-    float softcap;
-    const float* slopes;   // [n_heads] or null
-    const float* sink;     // [n_heads] or null
-};
-
 #define ATT_MAX_D 256
 
 template <typename T, typename TO>
@@ -548,12 +528,13 @@ __global__ void __launch_bounds__(64) paged_attention_generic_kernel(AttnArgs a)
     }
 }
 
+// `scratch` (may be null): what llmx_attention_f32_scratch asks for, for float32 rows whose contexts are shared out.
 // `out_dtype`: the output's type where it differs from the cache's (several maps are joined in float32 by a later kernel).
 extern "C" int llmx_paged_attention_generic(const void* q, const void* k_cache, const void* v_cache, const int* pos, const int* row_entry,
                                             const int* tables, void* out, int dtype, float scale, int rows, int n_heads, int n_kv_heads,
                                             int head_dim, int page_tokens, int max_blocks, int window, int v_dim, const float* gate, int gate_ld,
                                             int gate_wide, int keep_first, int chunk, int maps, float softcap, const float* slopes,
-                                            const float* sink, int out_dtype, hipStream_t stream) {
+                                            const float* sink, int out_dtype, float* scratch, long scratch_floats, hipStream_t stream) {
     if (rows <= 0) return 0;
     if (head_dim > ATT_MAX_D || v_dim > ATT_MAX_D || v_dim < 1 || n_heads % n_kv_heads) return -2;
     if (gate && gate_ld < (gate_wide ? n_heads * v_dim : n_heads)) return -2;
@@ -561,6 +542,8 @@ extern "C" int llmx_paged_attention_generic(const void* q, const void* k_cache, 
     AttnArgs a{q, k_cache, v_cache, pos, row_entry, tables, out, scale, n_heads, n_kv_heads, head_dim, page_tokens, max_blocks, window, v_dim,
                gate, gate_ld, gate_wide, keep_first, chunk, maps, softcap, slopes, sink};
     llmx_note_launch(LK_ATTENTION_GENERIC);
+    // plain float32 attention whose sizes allow 16-byte loads goes to the float32 matrix instruction
+    if (dtype == LLMX_F32 && out_dtype == LLMX_F32 && llmx_attention_f32_takes(a)) return llmx_attention_f32(a, rows, scratch, scratch_floats, stream);
     const dim3 grid(rows, n_heads * maps);
     if (dtype == LLMX_F32)
         hipLaunchKernelGGL((paged_attention_generic_kernel<float, float>), grid, dim3(64), 0, stream, a);

@@ -35,6 +35,8 @@
     X(QKNORM_ROPE_KVWRITE, "qknorm_rope_kvwrite")                                                                         \
     X(QKNORM_ROPE_KVWRITE_ROWS, "qknorm_rope_kvwrite.rows")                                                               \
     X(ATTENTION_GENERIC, "attention.generic")                                                                             \
+    X(ATTENTION_F32, "attention_f32")                                                                                     \
+    X(ATTENTION_F32_MERGE, "attention_f32.merge")                                                                         \
     X(ATTENTION_TILES128, "attention.tiles128")                                                                           \
     X(ATTENTION_TILES, "attention.tiles")                                                                                 \
     X(ATTENTION_DIRECT, "attention.direct")                                                                               \

@@ -78,7 +78,7 @@ def _declare(h) -> None:
         "llmx_attention_partial_pad": [],
         "llmx_gemm_generic": [P, I, P, I, P, I, I, I, I, I, I, I, I, I, P, P, I, L, I, I, P, I, F, P, P, I, P],
         "llmx_qknorm_rope_kvwrite": [P, P, P, P, P, P, P, P, P, P, I, F, I, I, I, I, I, I, I, I, I, I, I, I, P],
-        "llmx_paged_attention_generic": [P, P, P, P, P, P, P, I, F, I, I, I, I, I, I, I, I, P, I, I, I, I, I, F, P, P, I, P],
+        "llmx_paged_attention_generic": [P, P, P, P, P, P, P, I, F, I, I, I, I, I, I, I, I, P, I, I, I, I, I, F, P, P, I, P, L, P],
         "llmx_head_norm_rope_kvwrite": [P, P, P, P, P, P, P, P, P, P, P, I, F, I, I, I, I, I, I, I, I, I, I, I, P, I, I, I, I, P],
         "llmx_gate_heads": [P, I, P, I, I, I, I, P],
         "llmx_rmsnorm_add_norm": [P, P, P, F, P, F, P, I, P, I, I, P],
@@ -138,6 +138,8 @@ def _declare(h) -> None:
     h.llmx_sample_ranked_scratch.restype = c_long
     h.llmx_gemm_tile_runs_scratch.argtypes = [I, I, I, I, I, I]
     h.llmx_gemm_tile_runs_scratch.restype = c_long
+    h.llmx_attention_f32_scratch.argtypes = [I, I, I, I, I, I]
+    h.llmx_attention_f32_scratch.restype = c_long
     h.llmx_launch_name.restype = ctypes.c_char_p
     h.llmx_note_launch.restype = None
 
@@ -1602,10 +1604,12 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                                           _dev(r.sink, "sink", torch.float32, (n_heads,)), gate_at, gate_ld, gate_wide, rules_plan.hpc, _stream()),
                "attention_rules")
         return
+    need = 0 if scratch is None or q.dtype != torch.float32 else lib().llmx_attention_f32_scratch(rows, n_heads, n_kv_heads, v_dim, page_tokens, tables.shape[1])
+    parts = scratch("attention.f32_parts", (need,), torch.float32) if need else None      # float32 contexts shared out over workgroups; the same bits without
     _check(lib().llmx_paged_attention_generic(*common, _dev(out, "out"), _code(q.dtype), float(scale), rows, n_heads, n_kv_heads,
                                               head_dim, page_tokens, tables.shape[1], int(window), v_dim, gate_at, gate_ld, gate_wide,
                                               r.keep_first, r.chunk, r.maps, r.softcap, _dev(r.slopes, "slopes", torch.float32, (n_heads,)),
-                                              _dev(r.sink, "sink", torch.float32, (n_heads,)), _code(out.dtype), _stream()), "paged_attention")
+                                              _dev(r.sink, "sink", torch.float32, (n_heads,)), _code(out.dtype), _dev(parts, "parts"), need, _stream()), "paged_attention")
 
 
 def _parts_args(z: torch.Tensor, parts: Optional[torch.Tensor]):
