@@ -229,10 +229,14 @@ extern "C" int llmx_sigmoid_root(const float* z, const float* bias, float inv_ta
 
 // ---------------------------------------------------------------------------
 // The scan.  Grid (H * ceil(V / 8), entries), four waves a block: 32 lanes (two rows of 16) own value channel
-// 8 * tile + c together, lane s of them the key channels s, 32 + s, ... of its head (R of them).  q and k are read head h / share (several heads may share one), with row
-// strides of their own, so they may be columns of a wider projection.  A lane's sums over its R channels run in up to four
-// chains (channels i, i + 4, ...: (c0 + c1) + (c2 + c3)); sums over a column's lanes are a butterfly over each row of 16,
-// then the two rows' sums added.
+// 8 * tile + c together, lane s of them the key channels s, 32 + s, 64 + s, ... of its head (2 R of them).  q and k are read head h /
+// share (several heads may share one), with row strides of their own, so they may be columns of a wider projection.
+// A sum over the key channels has one order: channels 64 apart in up to four chains ((c0 + c1) + (c2 + c3)), then the sums of
+// channels 32 apart (in a lane), 16 apart (between the column's rows of lanes) and 8, 4, 2, 1 apart (a butterfly over a row).
+// What bounds a prompt is the chain from a token's state to the next one's, a wave's instructions a token one after the other: with
+// a whole wave a column, two channels a lane, a wave spent as many instructions on a column's sums as on its channels and two waves
+// shared a SIMD (a prompt of 1,999 rows, heads of 128 x 128, mean over layers of 16 and of 4 heads: 552 us; this form 330 us, without a
+// branch a token on whether there is a correction 284 us: 0.14 us a token).
 // An entry's blocks also hand on the convolution tail, each a share of its channels: the entry's last taps - 1 inputs, from
 // this step's rows of `tail_src` and, where the step brought fewer, from the old tail.
 struct StateScanArgs {
@@ -257,22 +261,38 @@ struct StateScanArgs {
     StateOperands operands;
 };
 
-// Rows are worked on in chunks of CH: the block brings a chunk's q, k and decay values (its head's D of each, padded to
-// 16 R) and its 8 values of v and beta through registers into LDS while the chunk before is worked on, so the chain from
+// Rows are worked on in chunks of CH: the block brings a chunk's k, q and decay values (its head's D of each, padded to
+// 64 R) and its 8 values of v and beta through registers into LDS while the chunk before is worked on, so the chain from
 // token to token waits for LDS, not for memory; a token's operands are read from LDS while the token before is worked on.
 // Every load is asked for whatever the index (addresses are clamped, the value is chosen afterwards), so none sits behind
-// a branch.
-__device__ __forceinline__ float column_sum(float v) { return wave_sum(v); }     // over a column's lanes, the same bits in each
+// a branch.  QUADS: plain operands whose heads, strides and starts are multiples of four floats are brought 16 bytes at a time.
 
 #define SCAN_COLS 8     // value channels a block of four waves owns
-#define SCAN_LANES 64   // lanes that share a column: a wave
+#define SCAN_LANES 32   // lanes that share a column
 #define SCAN_THREADS (SCAN_COLS * SCAN_LANES)
-template <int R, int CH, int KIND>
+
+// The last levels of a column's sum: the values of its 32 lanes, channels 16 apart first; the same bits in each lane.
+__device__ __forceinline__ float row_sum16(float v) {
+    v += row_rotate<8>(v);
+    v += row_rotate<4>(v);
+    v += row_rotate<2>(v);
+    v += row_rotate<1>(v);
+    return v;
+}
+__device__ __forceinline__ float column_sum(float v) {
+    uint32_t even, odd;
+    rows_pair16(__float_as_uint(v), even, odd);
+    return row_sum16(__uint_as_float(even) + __uint_as_float(odd));
+}
+
+template <int R, int CH, int KIND, bool QUADS, bool DELTA>
 __global__ void __launch_bounds__(SCAN_THREADS) state_scan_kernel(StateScanArgs a) {
-    constexpr int DP = SCAN_LANES * R;              // a head's key channels, padded
+    static_assert(KIND == STATE_OPERANDS_PLAIN || !QUADS, "only plain operands are brought as they lie");
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    constexpr int DP = 64 * R, J = 2 * R;           // a head's key channels, padded; a lane's
     constexpr int PER_TOKEN = 3 * DP;               // k | q | decay
-    constexpr int STAGE = (CH * PER_TOKEN + SCAN_THREADS - 1) / SCAN_THREADS;   // values a thread brings a chunk
-    constexpr int NC = R >= 4 ? 4 : R;              // chains a lane's sums run in
+    constexpr int UNIT = QUADS ? 4 : 1;             // floats of a load
+    constexpr int STAGE = (CH * PER_TOKEN / UNIT + SCAN_THREADS - 1) / SCAN_THREADS;   // loads a thread makes a chunk
     __shared__ __attribute__((aligned(16))) float rows[2][CH][PER_TOKEN];
     __shared__ float vals[2][CH][SCAN_COLS];
     __shared__ float betas[2][CH];
@@ -284,7 +304,6 @@ __global__ void __launch_bounds__(SCAN_THREADS) state_scan_kernel(StateScanArgs 
     if (a.max_rows_here > 0 && n > a.max_rows_here) return;     // its tail is the other kernel's too
     const int j = tile * SCAN_COLS + c;
     const bool col = j < a.V;
-    const int d0 = s * R;           // where the lane's operands lie in a staged row; its i-th key channel is 32 i + s
     const size_t slot_r = (size_t)a.slot_read[e] * a.state_stride, slot_w = (size_t)a.slot_write[e] * a.state_stride;
 
     if (a.taps > 1) {       // the entry's blocks share the tail's channels out among themselves
@@ -305,44 +324,52 @@ __global__ void __launch_bounds__(SCAN_THREADS) state_scan_kernel(StateScanArgs 
     const float* qp = a.q + (size_t)hq * a.D;
     const float* gp = a.decay + (size_t)h * (a.head_decay ? 1 : a.D);
     const float* vp = a.v + (size_t)h * a.V + tile * SCAN_COLS;
-    float stage[STAGE], vstage = 0.0f, bstage = 0.0f;
+    float stage[STAGE][UNIT], vstage = 0.0f, bstage = 0.0f;
     auto fetch = [&](int t0) {
 #pragma unroll
         for (int u = 0; u < STAGE; ++u) {
-            const int idx = min(tid + SCAN_THREADS * u, CH * PER_TOKEN - 1);
-            const int tt = idx / PER_TOKEN, rem = idx % PER_TOKEN, which = rem / DP, d = rem % DP;
+            const int idx = min(tid + SCAN_THREADS * u, CH * PER_TOKEN / UNIT - 1);
+            const int tt = idx / (PER_TOKEN / UNIT), rem = idx % (PER_TOKEN / UNIT) * UNIT, which = rem / DP, d = rem % DP;
             const size_t row = (size_t)(row0 + min(t0 + tt, n - 1));
             const int dd = d < a.D ? d : 0;
             const float* src = which == 0 ? kp + row * a.ldk : which == 1 ? qp + row * a.ldq : gp + row * a.ldg;
-            const int at = which == 2 && a.head_decay ? 0 : dd;
-            const float x = KIND == STATE_OPERANDS_PLAIN || which == 2 ? src[at] : state_key<KIND>(a.operands, src, row, dd);
-            stage[u] = d < a.D ? x : 0.0f;
+            if constexpr (QUADS) {
+                const f32x4_t x = *reinterpret_cast<const f32x4_t*>(src + dd);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) stage[u][i] = d < a.D ? x[i] : 0.0f;
+            } else {
+                const int at = which == 2 && a.head_decay ? 0 : dd;
+                const float x = KIND == STATE_OPERANDS_PLAIN || which == 2 ? src[at] : state_key<KIND>(a.operands, src, row, dd);
+                stage[u][0] = d < a.D ? x : 0.0f;
+            }
         }
         if (tid < CH * SCAN_COLS) {
             const int tt = min(tid / SCAN_COLS, CH - 1), cc = tid % SCAN_COLS;
             vstage = state_value<KIND>(vp[(size_t)(row0 + min(t0 + tt, n - 1)) * a.ldv + min(cc, a.V - 1 - tile * SCAN_COLS)]);
         }
-        if (a.beta) bstage = a.beta[(size_t)(row0 + min(t0 + min(tid, CH - 1), n - 1)) * a.H + h];
+        if (DELTA) bstage = a.beta[(size_t)(row0 + min(t0 + min(tid, CH - 1), n - 1)) * a.H + h];
     };
-    // a staged row holds channel d at (d % 32) * R + d / 32, so that a lane's R values (channels s, 32 + s, ...) lie together
     auto put = [&](int b) {
 #pragma unroll
         for (int u = 0; u < STAGE; ++u) {
             const int idx = tid + SCAN_THREADS * u;
-            const int tt = idx / PER_TOKEN, rem = idx % PER_TOKEN, which = rem / DP, d = rem % DP;
-            if (idx < CH * PER_TOKEN) rows[b][tt][which * DP + (d % SCAN_LANES) * R + d / SCAN_LANES] = stage[u];
+            if (idx < CH * PER_TOKEN / UNIT) {
+                float* to = &rows[b][0][0] + idx * UNIT;
+                if constexpr (QUADS) *reinterpret_cast<f32x4_t*>(to) = f32x4_t{stage[u][0], stage[u][1], stage[u][2], stage[u][3]};
+                else *to = stage[u][0];
+            }
         }
         if (tid < CH * SCAN_COLS) (&vals[b][0][0])[tid] = vstage;
         if (tid < CH) betas[b][tid] = bstage;
     };
 
     // the state is asked for before the first chunk, whose values may wait for arithmetic of their own
-    float S[R];
+    float S[J];
     const size_t tile_at = ((size_t)h * tiles + tile) * a.D * SCAN_COLS + c;
     {
         const float* src = a.state + slot_r + tile_at;
 #pragma unroll
-        for (int i = 0; i < R; ++i) {
+        for (int i = 0; i < J; ++i) {
             const int d = SCAN_LANES * i + s;
             const float x = src[(size_t)(d < a.D ? d : 0) * SCAN_COLS];
             S[i] = (col && d < a.D) ? x : 0.0f;
@@ -351,52 +378,49 @@ __global__ void __launch_bounds__(SCAN_THREADS) state_scan_kernel(StateScanArgs 
     fetch(0);
     put(0);
     __syncthreads();
-    const bool delta = a.beta != nullptr;
     // a token's operands as the lane reads them from the staged chunk; two sets take turns, so that a token's are read while
     // the token before is worked on and nothing is copied from set to set
     struct Operands {
-        float k[R], q[R], g[R], v, beta;
+        float k[J], q[J], g[J], v, beta;
     };
     auto read = [&](Operands& x, int b, int tt) {
-        const float* kr = &rows[b][tt][d0];
+        const float* kr = &rows[b][tt][s];
 #pragma unroll
-        for (int i = 0; i < R; ++i) {
-            x.k[i] = kr[i];
-            x.q[i] = kr[DP + i];
-            x.g[i] = kr[2 * DP + i];
+        for (int i = 0; i < J; ++i) {
+            x.k[i] = kr[SCAN_LANES * i];
+            x.q[i] = kr[DP + SCAN_LANES * i];
+            x.g[i] = kr[2 * DP + SCAN_LANES * i];
         }
         x.v = vals[b][tt][c];
-        x.beta = betas[b][tt];
+        x.beta = DELTA ? betas[b][tt] : 0.0f;
+    };
+    // a lane's share of a column's sum: channels s, 64 + s, ... and 32 + s, 96 + s, ..., then the two
+    auto lane_sum = [&](const float (&p)[J]) {
+        auto chains = [&](int first) {
+            if constexpr (R == 4) return (p[first] + p[first + 2]) + (p[first + 4] + p[first + 6]);
+            else if constexpr (R == 2) return p[first] + p[first + 2];
+            else return p[first];
+        };
+        return chains(0) + chains(1);
     };
     const size_t out_ld = (size_t)a.H * a.V;
     // one token: the state's update, and the lane's share of the read-out (summed over the column's lanes later, for a whole
     // chunk at once: only the delta correction's sum lies on the way from a token's state to the next one's)
     auto token = [&](const Operands& x) -> float {
-        float u = x.v;
-        if (delta) {
-            float p[NC];
+        float u = x.v, p[J];
 #pragma unroll
-            for (int y = 0; y < NC; ++y) p[y] = 0.0f;
+        for (int i = 0; i < J; ++i) S[i] = S[i] * x.g[i];
+        if constexpr (DELTA) {
 #pragma unroll
-            for (int i = 0; i < R; ++i) {
-                S[i] = S[i] * x.g[i];
-                p[i % NC] = fmaf(x.k[i], S[i], p[i % NC]);
-            }
-            const float dot = NC == 4 ? (p[0] + p[1]) + (p[2] + p[3]) : NC == 2 ? p[0] + p[1] : p[0];
-            u = x.beta * (u - column_sum(dot));
-        } else {
-#pragma unroll
-            for (int i = 0; i < R; ++i) S[i] = S[i] * x.g[i];
+            for (int i = 0; i < J; ++i) p[i] = fmaf(x.k[i], S[i], 0.0f);
+            u = x.beta * (u - column_sum(lane_sum(p)));
         }
-        float o[NC];
 #pragma unroll
-        for (int y = 0; y < NC; ++y) o[y] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
+        for (int i = 0; i < J; ++i) {
             S[i] = fmaf(x.k[i], u, S[i]);
-            o[i % NC] = fmaf(x.q[i], S[i], o[i % NC]);
+            p[i] = fmaf(x.q[i], S[i], 0.0f);
         }
-        return NC == 4 ? (o[0] + o[1]) + (o[2] + o[3]) : NC == 2 ? o[0] + o[1] : o[0];
+        return lane_sum(p);
     };
     Operands first, second;
     float* out_at = a.out + (size_t)row0 * out_ld + (size_t)h * a.V + (col ? j : 0);
@@ -408,20 +432,34 @@ __global__ void __launch_bounds__(SCAN_THREADS) state_scan_kernel(StateScanArgs 
         const int m = min(CH, n - t0);
         read(first, b, 0);
         float share[CH];
+        if (m == CH) {
 #pragma unroll
-        for (int tt = 0; tt < CH; ++tt) {
-            if (tt < m) {
+            for (int tt = 0; tt < CH; ++tt) {
                 read((tt & 1) ? first : second, b, tt + 1 < CH ? tt + 1 : tt);
                 share[tt] = token((tt & 1) ? second : first);
             }
-        }
+        } else {
 #pragma unroll
-        for (int tt = 0; tt < CH; ++tt) {
-            if (tt < m) {
-                const float sum = column_sum(share[tt]);
-                if (s == 0 && col) out_at[(size_t)tt * out_ld] = sum * a.out_scale;
+            for (int tt = 0; tt < CH; ++tt) {
+                share[tt] = 0.0f;
+                if (tt < m) {
+                    read((tt & 1) ? first : second, b, tt + 1 < CH ? tt + 1 : tt);
+                    share[tt] = token((tt & 1) ? second : first);
+                }
             }
         }
+        // the read-outs' sums: the two rows of a column take half of the chunk's tokens each, the halves' values changing
+        // places between them; then a lane picks one of its row's tokens and stores it
+        float picked = 0.0f;
+#pragma unroll
+        for (int tt = 0; tt < CH / 2; ++tt) {
+            const auto swapped = __builtin_amdgcn_permlane16_swap(__float_as_uint(share[tt]), __float_as_uint(share[tt + CH / 2]), false, false);
+            const uint32_t w0 = swapped[0], w1 = swapped[1];       // an even row: its own and the odd row's share of token tt; an odd row: of token tt + CH / 2
+            const float sum = row_sum16(__uint_as_float(w0) + __uint_as_float(w1));
+            picked = (s & 15) == tt ? sum : picked;
+        }
+        const int tt = (s & 15) + (s >> 4) * (CH / 2);
+        if ((s & 15) < CH / 2 && tt < m && col) out_at[(size_t)tt * out_ld] = picked * a.out_scale;
         out_at += (size_t)CH * out_ld;
         if (more) put(b ^ 1);
         __syncthreads();
@@ -429,7 +467,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) state_scan_kernel(StateScanArgs 
     {
         float* dst = a.state + slot_w + tile_at;
 #pragma unroll
-        for (int i = 0; i < R; ++i)
+        for (int i = 0; i < J; ++i)
             if (col && SCAN_LANES * i + s < a.D) dst[(size_t)(SCAN_LANES * i + s) * SCAN_COLS] = S[i];
     }
 }
@@ -728,27 +766,36 @@ extern "C" int llmx_state_scan(const float* q, int ldq, const float* k, int ldk,
         return LLMX_CHECK_LAUNCH();
     }
     llmx_note_launch(LK_STATE_SCAN);
-    const int per_lane = (D + SCAN_LANES - 1) / SCAN_LANES;
+    const int chains = (D + 63) / 64;
     // steps of single decoded tokens stage chunks of two rows (a quarter of the LDS, so more blocks a compute unit); a
     // row's arithmetic does not depend on the chunk it came in
-#define LLMX_SCAN_KIND(R_, CH_, KIND_) \
+    const bool quads = operands == STATE_OPERANDS_PLAIN && !head_decay && D % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ldg % 4 == 0 &&
+                       (((uintptr_t)q | (uintptr_t)k | (uintptr_t)decay) & 15) == 0;
+#define LLMX_SCAN_FORM(R_, CH_, KIND_, QUADS_) \
     do { \
-        if (max_rows > 0 && max_rows <= 2) hipLaunchKernelGGL((state_scan_kernel<R_, 2, KIND_>), grid, dim3(SCAN_THREADS), 0, stream, a); \
-        else hipLaunchKernelGGL((state_scan_kernel<R_, CH_, KIND_>), grid, dim3(SCAN_THREADS), 0, stream, a); \
+        if (beta) hipLaunchKernelGGL((state_scan_kernel<R_, CH_, KIND_, QUADS_, true>), grid, dim3(SCAN_THREADS), 0, stream, a); \
+        else hipLaunchKernelGGL((state_scan_kernel<R_, CH_, KIND_, QUADS_, false>), grid, dim3(SCAN_THREADS), 0, stream, a); \
     } while (0)
-#define LLMX_SCAN(R_, CH_) \
+#define LLMX_SCAN_KIND(R_, CH_, KIND_, QUADS_) \
     do { \
-        if (operands == STATE_OPERANDS_SILU) LLMX_SCAN_KIND(R_, CH_, STATE_OPERANDS_SILU); \
-        else if (operands == STATE_OPERANDS_ROTATED) LLMX_SCAN_KIND(R_, CH_, STATE_OPERANDS_ROTATED); \
-        else LLMX_SCAN_KIND(R_, CH_, STATE_OPERANDS_PLAIN); \
+        if (max_rows > 0 && max_rows <= 2) LLMX_SCAN_FORM(R_, 2, KIND_, QUADS_); \
+        else LLMX_SCAN_FORM(R_, CH_, KIND_, QUADS_); \
+    } while (0)
+#define LLMX_SCAN(R_, CH_, CH_SINGLE_) \
+    do { \
+        if (operands == STATE_OPERANDS_SILU) LLMX_SCAN_KIND(R_, CH_SINGLE_, STATE_OPERANDS_SILU, false); \
+        else if (operands == STATE_OPERANDS_ROTATED) LLMX_SCAN_KIND(R_, CH_SINGLE_, STATE_OPERANDS_ROTATED, false); \
+        else if (quads) LLMX_SCAN_KIND(R_, CH_, STATE_OPERANDS_PLAIN, true); \
+        else LLMX_SCAN_KIND(R_, CH_SINGLE_, STATE_OPERANDS_PLAIN, false); \
     } while (0)
     // chunks of 16 rows where LDS holds two of them (heads of at most 128 key channels): a chunk's work then outlasts the
-    // next chunk's way from memory
-    if (per_lane <= 1) LLMX_SCAN(1, 16);
-    else if (per_lane <= 2) LLMX_SCAN(2, 16);
-    else LLMX_SCAN(4, 8);
+    // next chunk's way from memory; operands that come one value a load take chunks whose loads a thread has registers for
+    if (chains <= 1) LLMX_SCAN(1, 16, 8);
+    else if (chains <= 2) LLMX_SCAN(2, 16, 8);
+    else LLMX_SCAN(4, 8, 4);
 #undef LLMX_SCAN
 #undef LLMX_SCAN_KIND
+#undef LLMX_SCAN_FORM
     return LLMX_CHECK_LAUNCH();
 }
 
