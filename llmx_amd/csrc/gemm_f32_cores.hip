@@ -9,10 +9,11 @@
 //    K each, and ask for a round of steps while the round before is multiplied.  1 row: 32,768 features of 2,048 values 56 us (4.8
 //    TB/s), 8,192 of 3,072 22 us, 3,072 of 2,048 12.8 us; the universal product takes 0.2-0.5 ms for the smallest of these.
 //  * tiles: many rows.  The instruction's rate bounds it (140 TFLOP/s measured alone): 64 rows x 128 (64) features a workgroup,
-//    operands staged through LDS 32 values of k at a time, a wave 32 x 32, its runs folded in registers.  2,048 rows: 8,192 features
-//    of 3,072 values 0.78 ms (132 TFLOP/s); 333 rows of 2,048 values: 32,768 features 0.44 ms (102 TFLOP/s), where the universal
+//    operands staged through LDS 32 values of k at a time, its runs folded in registers.  2,048 rows: 8,192 features
+//    of 3,072 values 0.80 ms (130 TFLOP/s); 333 rows of 2,048 values: 32,768 features 0.44 ms (102 TFLOP/s), where the universal
 //    product reaches 8 TFLOP/s.  Chunks asked for two ahead instead of one: 0.84 -> 0.78 ms and 0.47 -> 0.44 ms.
 #include "gemm_args.h"
+#include <type_traits>
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -162,10 +163,13 @@ __global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
 // that 8 rows' 16-byte pieces fall into different banks; the next chunk travels while this one is multiplied.
 #define FT_ROWS 64
 #define FT_PITCH 36
+#define FT_AHEAD 2      // (4: the same)
 template <int EPI, int BN>
-__global__ void __launch_bounds__(4 * BN) gemm_f32_tiles_kernel(GemmArgs g, int ks, int n_groups) {
-    constexpr int THREADS = 4 * BN, WAVES = THREADS / 64;
-    constexpr int A_PIECES = FT_ROWS * 8 / THREADS, ROWS_A_PASS = THREADS / 8;       // 16-byte pieces of a chunk a thread brings: 2 of W's
+__global__ void __launch_bounds__(512) gemm_f32_tiles_kernel(GemmArgs g, int ks, int n_groups) {
+    // eight waves of 32 weight rows by TT tiles of 16 rows: also a tile that has its CU to itself gives a SIMD two waves, so that one's
+    // operand reads hide behind the other's multiplications (64 weight rows, 2,048 values, four waves of 32 x 32: 55 us a tile)
+    constexpr int TT = BN / 64, THREADS = 512, WAVES = 8;
+    constexpr int W_PIECES = BN * 8 / THREADS, ROWS_A_PASS = THREADS / 8;       // 16-byte pieces of a chunk a thread brings: these of W's, one of A's
     __shared__ __attribute__((aligned(16))) float Ws[2][BN * FT_PITCH];
     __shared__ __attribute__((aligned(16))) float As[2][FT_ROWS * FT_PITCH];
     __shared__ int rows_a[FT_ROWS], rows_c[FT_ROWS], tile_info[3], scan_waves[WAVES];
@@ -219,49 +223,48 @@ __global__ void __launch_bounds__(4 * BN) gemm_f32_tiles_kernel(GemmArgs g, int 
     }
     __syncthreads();
     const int piece = tid & 7, prow = tid >> 3;
-    const float* w_src[2];
-    const float* a_src[A_PIECES];
+    const float* w_src[W_PIECES];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < W_PIECES; ++j) {
         const int w = prow + ROWS_A_PASS * j;
         // gated: rows 32 q .. + 15 of the tile are features 16 q .. + 15's gate rows, the next 16 their up rows
         const int f = EPI == EPI_SWIGLU ? n0 + 16 * (w >> 5) + (w & 15) : n0 + w;
         w_src[j] = W + (size_t)(min(f, g.N - 1) + (EPI == EPI_SWIGLU && (w & 16) ? g.up_offset : 0)) * g.ldw + 4 * piece;
     }
-#pragma unroll
-    for (int j = 0; j < A_PIECES; ++j) a_src[j] = (const float*)g.A + (size_t)rows_a[prow + ROWS_A_PASS * j] * g.lda + 4 * piece;
+    const float* a_src = (const float*)g.A + (size_t)rows_a[prow] * g.lda + 4 * piece;
     struct Fetched {
-        f32x4_t w[2], a[A_PIECES];
+        f32x4_t w[W_PIECES], a;
     };
     auto fetch = [&](int c, Fetched& f) {
         const int kk = min(32 * c, K - 16 - 16 * (piece >> 2));      // K's last chunk may hold one step: the second is fetched from inside K and not multiplied
 #pragma unroll
-        for (int j = 0; j < 2; ++j) f.w[j] = *reinterpret_cast<const f32x4_t*>(w_src[j] + kk);
-#pragma unroll
-        for (int j = 0; j < A_PIECES; ++j) f.a[j] = *reinterpret_cast<const f32x4_t*>(a_src[j] + kk);
+        for (int j = 0; j < W_PIECES; ++j) f.w[j] = *reinterpret_cast<const f32x4_t*>(w_src[j] + kk);
+        f.a = *reinterpret_cast<const f32x4_t*>(a_src + kk);
     };
     auto stage = [&](const Fetched& f, int buf) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) *reinterpret_cast<f32x4_t*>(&Ws[buf][(prow + ROWS_A_PASS * j) * FT_PITCH + 4 * piece]) = f.w[j];
-#pragma unroll
-        for (int j = 0; j < A_PIECES; ++j) *reinterpret_cast<f32x4_t*>(&As[buf][(prow + ROWS_A_PASS * j) * FT_PITCH + 4 * piece]) = f.a[j];
+        for (int j = 0; j < W_PIECES; ++j) *reinterpret_cast<f32x4_t*>(&Ws[buf][(prow + ROWS_A_PASS * j) * FT_PITCH + 4 * piece]) = f.w[j];
+        *reinterpret_cast<f32x4_t*>(&As[buf][prow * FT_PITCH + 4 * piece]) = f.a;
     };
     const int steps = K >> 4, per = (steps + ks - 1) / ks, chunks = (steps + 1) / 2;
-    f32x4_t total[2][2], acc[2][2];
+    f32x4_t total[2][TT], acc[2][TT];
 #pragma unroll
     for (int ns = 0; ns < 2; ++ns)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[ns][t] = total[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < TT; ++t) acc[ns][t] = total[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     bool first_run = true;
     int in_run = 0;
-    auto multiply = [&](int c, int buf) {
-        f32x4_t wf[2][2], af[2][2];
+    auto multiply = [&](auto live, int c, int buf) {
+        constexpr int LIVE = decltype(live)::value;      // 16-row tiles of the wave that hold rows
+        f32x4_t wf[2][2], af[2][TT];
+        if constexpr (LIVE > 0) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < 2; ++u) {
 #pragma unroll
-            for (int ns = 0; ns < 2; ++ns) wf[u][ns] = *reinterpret_cast<const f32x4_t*>(&Ws[buf][(32 * wn + 16 * ns + r) * FT_PITCH + 16 * u + 4 * kg]);
+                for (int ns = 0; ns < 2; ++ns) wf[u][ns] = *reinterpret_cast<const f32x4_t*>(&Ws[buf][(32 * wn + 16 * ns + r) * FT_PITCH + 16 * u + 4 * kg]);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) af[u][t] = *reinterpret_cast<const f32x4_t*>(&As[buf][(32 * wm + 16 * t + r) * FT_PITCH + 16 * u + 4 * kg]);
+                for (int t = 0; t < LIVE; ++t) af[u][t] = *reinterpret_cast<const f32x4_t*>(&As[buf][(16 * (TT * wm + t) + r) * FT_PITCH + 16 * u + 4 * kg]);
+            }
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -272,12 +275,12 @@ __global__ void __launch_bounds__(4 * BN) gemm_f32_tiles_kernel(GemmArgs g, int 
 #pragma unroll
                 for (int ns = 0; ns < 2; ++ns)
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) acc[ns][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][ns][i], af[u][t][i], acc[ns][t], 0, 0, 0);
+                    for (int t = 0; t < LIVE; ++t) acc[ns][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][ns][i], af[u][t][i], acc[ns][t], 0, 0, 0);
             if (++in_run == per || s + 1 == steps) {
 #pragma unroll
                 for (int ns = 0; ns < 2; ++ns)
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) {
+                    for (int t = 0; t < LIVE; ++t) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) total[ns][t][i] = first_run ? acc[ns][t][i] : total[ns][t][i] + acc[ns][t][i];
                         acc[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -288,28 +291,33 @@ __global__ void __launch_bounds__(4 * BN) gemm_f32_tiles_kernel(GemmArgs g, int 
         }
     };
     const ActFn act(EPI != EPI_SWIGLU ? g.act : LLMX_ACT_NONE, g.act_params);
-    // two chunks are on their way through two register sets while a third is multiplied (one ahead: 8% slower, a chunk's
-    // multiplications being shorter than the way to memory); past the end the last one again
-    Fetched even, odd;
-    fetch(0, even);
-    fetch(min(1, chunks - 1), odd);
-    stage(even, 0);
-    fetch(min(2, chunks - 1), even);
-    __syncthreads();
-    for (int c = 0; c < chunks; c += 2) {
-        multiply(c, 0);
-        stage(odd, 1);
-        fetch(min(c + 3, chunks - 1), odd);
-        __syncthreads();
-        if (c + 1 >= chunks) break;
-        multiply(c + 1, 1);
-        stage(even, 0);
-        fetch(min(c + 4, chunks - 1), even);
-        __syncthreads();
-    }
+    // FT_AHEAD chunks are on their way, a register set each, while another is multiplied: a chunk's multiplications are far shorter than
+    // the way to memory; past the end the last one again
+    Fetched f[FT_AHEAD];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int row = rows_c[32 * wm + 16 * t + r];
+    for (int d = 0; d < FT_AHEAD; ++d) fetch(min(d, chunks - 1), f[d]);
+    stage(f[0], 0);
+    fetch(min(FT_AHEAD, chunks - 1), f[0]);
+    __syncthreads();
+    auto walk = [&](auto live) {
+        for (int c = 0; c < chunks; c += FT_AHEAD)
+#pragma unroll
+            for (int d = 0; d < FT_AHEAD; ++d) {
+                if (c + d >= chunks) break;
+                multiply(live, c + d, d & 1);
+                stage(f[(d + 1) % FT_AHEAD], (d & 1) ^ 1);
+                fetch(min(c + d + 1 + FT_AHEAD, chunks - 1), f[(d + 1) % FT_AHEAD]);
+                __syncthreads();
+            }
+    };
+    // a wave whose rows are past the last ones (a group's last tile) leaves the matrix cores to the others; every wave meets every barrier
+    const int held = min(row_end - row_begin, FT_ROWS) - 16 * TT * wm;
+    if (TT > 1 && held > 16) walk(std::integral_constant<int, TT>());
+    else if (held > 0) walk(std::integral_constant<int, 1>());
+    else walk(std::integral_constant<int, 0>());
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+        const int row = rows_c[16 * (TT * wm + t) + r];
         if (row < 0) continue;
         if (EPI == EPI_SWIGLU) {
             const int n = n0 + 16 * wn + 4 * kg;
@@ -363,26 +371,28 @@ static int launch_stream(const GemmArgs& g, int n_groups, int ks, int rows_a_gro
 template <int EPI>
 static int launch_tiles(const GemmArgs& g, int n_groups, int ks, int row_tiles, hipStream_t stream) {
     // 128 weight rows a workgroup read the activations half as often, 64 fill the chip with fewer rows.  Measured at K 2,048, 256
-    // CUs: with n workgroups a CU the narrow form takes about 22 + 33 n us (1: 56, 2: 87, 3: 121), the wide one 12 + 60 n (1: 72, 2: 131).
+    // CUs: with n workgroups a CU the narrow form takes about 10 + 33 n us (1: 43, 2: 76, 3: 106), the wide one 12 + 61 n (1: 73,
+    // 2: 136); rows count in sixteens, as the last tile's absent ones take no time (a group's last sixteen is half full on average).
     const int wide = EPI == EPI_SWIGLU ? 64 : 128, narrow = wide / 2;
-    const long n_wide = ((long)((g.N + wide - 1) / wide) * row_tiles + 255) / 256, n_narrow = ((long)((g.N + narrow - 1) / narrow) * row_tiles + 255) / 256;
-    if (12 + 60 * n_wide <= 22 + 33 * n_narrow)
+    const long sixteens = n_groups ? (g.M + 8 * (n_groups < g.M ? n_groups : g.M) + 15) / 16 : (g.M + 15) / 16;
+    const long n_wide = ((g.N + wide - 1) / wide * sixteens + 4 * 256 - 1) / (4 * 256), n_narrow = ((g.N + narrow - 1) / narrow * sixteens + 4 * 256 - 1) / (4 * 256);
+    if (12 + 61 * n_wide <= 10 + 33 * n_narrow)
         hipLaunchKernelGGL((gemm_f32_tiles_kernel<EPI, 128>), dim3((g.N + wide - 1) / wide, row_tiles), dim3(512), 0, stream, g, ks, n_groups);
     else
-        hipLaunchKernelGGL((gemm_f32_tiles_kernel<EPI, 64>), dim3((g.N + narrow - 1) / narrow, row_tiles), dim3(256), 0, stream, g, ks, n_groups);
+        hipLaunchKernelGGL((gemm_f32_tiles_kernel<EPI, 64>), dim3((g.N + narrow - 1) / narrow, row_tiles), dim3(512), 0, stream, g, ks, n_groups);
     return LLMX_CHECK_LAUNCH();
 }
 
-// Which form: the stream form multiplies at about 50 TFLOP/s beyond 16 rows (every strip reads the rows again), the tiles at 100 to
-// 130 but, at K 2,048, never in less than 56 us: they meet at rows x features of about 680,000 (3,072 features: 128 rows 47 against
-// 57 us, 256 rows 71 against 58; 8,192: 64 rows 73 against 82, 96 rows 120 against 86; 32,768: 16 rows 69 against 78, 48 rows 142
-// against 80).  Groups of at most half a tile of rows on average stay with the stream form, the tiles being mostly padding.
+// Which form: the stream form multiplies at about 45 TFLOP/s beyond 16 rows (every strip reads the rows again), the tiles at 100 to
+// 130 but, at K 2,048, never in less than 43 us: they meet at rows x features of about 380,000 (3,072 features: 96 rows 40 against
+// 43 us, 128 rows 47 against 44; 2,048: 128 rows 26 against 43, 192 rows 46 against 43; 8,192 of K 3,072: 48 rows 62 against 63).
+// Groups of at most half a tile of rows on average stay with the stream form, the tiles being mostly padding.
 template <int EPI>
 static int launch_f32(const GemmArgs& g, int n_groups, hipStream_t stream) {
     const int ks = f32_runs(g.N, g.K);
     const int rows = n_groups ? (g.M + n_groups - 1) / n_groups : g.M;      // grouped: a group's on average (the counts are on the device; both forms take any)
     const int row_tiles = n_groups ? (n_groups < g.M ? n_groups : g.M) + g.M / FT_ROWS : (g.M + FT_ROWS - 1) / FT_ROWS;
-    const bool few = rows <= (n_groups ? FT_ROWS / 2 : 16) || (long)g.M * g.N <= 680000;
+    const bool few = rows <= (n_groups ? FT_ROWS / 2 : 16) || (long)g.M * g.N <= 380000;
     if (!few && g.K % 16 == 0 && row_tiles <= 65535) {
         llmx_note_launch(LK_GEMM_GENERIC_TILES);
         return launch_tiles<EPI>(g, n_groups, ks, row_tiles, stream);
