@@ -90,7 +90,8 @@ struct TileArgs {
     GluArgs glu;            // TL_SWIGLU: the gated unit and its per-row values
 };
 
-// Whether the groups' rows fill tiles of 128 rows well enough: the tiles hold at most 1.6 times the rows (measured on
+// Whether the groups' rows fill tiles of 128 rows well enough.  The grouping's own choice comes as a count of 0 or 2^30; for a caller
+// that brings the bare count: the tiles hold at most 1.6 times the rows (measured on
 // the prompt's routing on one machine: a 2,048-token step takes 30.9 ms with the bound at 1.25, 30.3 ms at 1.6, 30.2 ms at 2).  The launcher
 // cannot know (the counts are on the device), so it launches the form for either case and one of them leaves at once.
 __device__ __forceinline__ bool tile_launch_runs(const TileArgs& g) {
@@ -832,7 +833,8 @@ static int form_feats(int form, int epi) { return (epi == TL_SWIGLU ? 64 : 128) 
 // Which form runs (every form gives an output element the same bits):
 //   dense: the wide form (8 waves, 128 x 256, three tiles deep) where it has at least 192 tiles for the 256 CUs
 //     (measured on 2,048 rows: 8,192 features 113 against 165 us, 3,072 features 100 against 108 us), else 64-row
-//     tiles (three workgroups a CU; more, smaller tiles fill the chip better when there are few).
+//     tiles (three workgroups a CU; more, smaller tiles fill the chip better when there are few, and up to 64 rows half
+//     of a 128-row tile is padding: 200,064 features of 3,072, 48 rows 265 -> 257 us, 64 rows 276 -> 268).
 //     With `runs_scratch` (llmx_gemm_tile_runs_scratch floats) a product of few tiles and several runs of K gives each
 //     run a workgroup of its own and adds the runs' sums in a second kernel, in the order the one kernel adds them.
 //   grouped with tile_stats: both a 128-row form (wide for long K, 4 waves for short K) and the 64-row form are
@@ -905,7 +907,7 @@ extern "C" int llmx_gemm_tile(const void* A, const void* W, void* C, int c_dtype
         rc = 0;
     } else if (!grouped) {
         const long wide_tiles = (long)((M + WD_BM - 1) / WD_BM) * ((N + form_feats(FORM_WIDE, epi) - 1) / form_feats(FORM_WIDE, epi));
-        rc = launch(wide_tiles >= 192 ? FORM_WIDE : FORM_64, 0);
+        rc = launch(wide_tiles >= 192 && M > 64 ? FORM_WIDE : FORM_64, 0);
     } else if (tile_stats) {
         // 128-row tiles: each group adds at most one partial tile
         const int big_tiles = (n_groups < M ? n_groups : M) + M / 128;

@@ -350,40 +350,80 @@ __global__ void __launch_bounds__(64) moe_place_kernel(const int* __restrict__ i
     }
 }
 
-// Few pairs (a decode step): one workgroup of 1024 threads does it all.  The pairs' experts sit in LDS; thread p owns
-// pair p: the experts' counts come from LDS atomics (a count does not depend on their order), the offsets from a scan
-// over the experts, and a pair's place in its expert's run is the number of earlier pairs of that expert (counted by
-// the thread itself), so each expert's pairs stay in increasing pair order.
+// The pairs p < 1,024 of a workgroup grouped by expert, thread p holding pair p's expert (-1: none).  Places follow pair order: a pair's
+// rank within its expert's run is the number of its wave's earlier lanes with the same expert (found by ballots over the expert
+// numbers' bits) plus what the waves before counted, a byte a wave and expert in LDS, read 16 bytes at once.  (Counting a pair's
+// predecessors one after the other took 10 us of the 13 for 666 pairs, 12 of the 16 for a chunk of 1,024.)
 #define ALIGN_SMALL_PAIRS 1024
-__device__ void align_in_block(const int* pair_expert, int n_pairs, int n_experts, int* cnt, int* offs, int* __restrict__ counts,
+struct PairTable {
+    uint32_t counts[1024][4];       // expert, then a byte for each of 16 waves
+};
+// The lanes of the wave that hold the same expert.
+__device__ __forceinline__ unsigned long long same_expert(int mine, int n_experts) {
+    unsigned long long peers = __ballot(mine >= 0);
+    for (int bit = 1; bit < n_experts; bit <<= 1) {
+        const unsigned long long set = __ballot((mine & bit) != 0);
+        peers &= (mine & bit) ? set : ~set;
+    }
+    return peers;
+}
+__device__ __forceinline__ int byte_sum(uint32_t x, int sum) { return (int)__builtin_amdgcn_sad_u8(x, 0u, (uint32_t)sum); }
+// The pair's rank in its expert's run (meaningless for a thread without a pair); the table then holds every expert's counts.  Every
+// thread of the workgroup calls it; it ends behind a barrier.
+__device__ __forceinline__ int rank_in_block(PairTable& table, int mine, int n_experts) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    if (tid < n_experts) *reinterpret_cast<uint4*>(table.counts[tid]) = make_uint4(0u, 0u, 0u, 0u);
+    const unsigned long long peers = same_expert(mine, n_experts), before = peers & ((1ull << lane) - 1ull);
+    __syncthreads();
+    if (mine >= 0 && before == 0ull) reinterpret_cast<uint8_t*>(table.counts[mine])[wave] = (uint8_t)__popcll(peers);
+    __syncthreads();
+    int rank = __popcll(before);
+    if (mine >= 0) {
+        const uint4 c = *reinterpret_cast<const uint4*>(table.counts[mine]);
+        const uint32_t words[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {      // of word w the bytes of the waves before this one
+            const int bytes = min(max(wave - 4 * w, 0), 4);
+            rank = byte_sum(bytes == 4 ? words[w] : words[w] & ((1u << (8 * bytes)) - 1u), rank);
+        }
+    }
+    return rank;
+}
+__device__ __forceinline__ int expert_pairs(const PairTable& table, int e) {
+    const uint4 c = *reinterpret_cast<const uint4*>(table.counts[e]);
+    return byte_sum(c.w, byte_sum(c.z, byte_sum(c.y, byte_sum(c.x, 0))));
+}
+// Over the wave's lanes before this one: the sum of c (at most `most`), bit by bit; the wave's sum in `all`.
+__device__ __forceinline__ int lanes_before(int c, int most, int lane, int& all) {
+    const unsigned long long earlier = (1ull << lane) - 1ull;
+    int sum = 0;
+    all = 0;
+    for (int bit = 0; (most >> bit) > 0; ++bit) {
+        const unsigned long long set = __ballot((c >> bit) & 1);
+        sum += __popcll(set & earlier) << bit;
+        all += __popcll(set) << bit;
+    }
+    return sum;
+}
+
+__device__ void align_in_block(const int* pair_expert, int n_pairs, int n_experts, PairTable& table, int* offs, int* __restrict__ counts,
                                int* __restrict__ offsets, int* __restrict__ list, int* __restrict__ active, int* __restrict__ n_active) {
     __shared__ int wave_total[16], wave_active[16];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    if (tid < n_experts) cnt[tid] = 0;
-    __syncthreads();
     int mine = tid < n_pairs ? pair_expert[tid] : -1;
     if (mine >= n_experts) mine = -1;   // an id outside the experts belongs to no run
-    if (mine >= 0) atomicAdd(&cnt[mine], 1);
-    __syncthreads();
+    const int rank = rank_in_block(table, mine, n_experts);
     // exclusive scan of the counts (and of "has rows") over the experts: within each wave, then over the waves before it
     {
         const int e = tid;
-        const int c = e < n_experts ? cnt[e] : 0;
-        int incl = c, incl_active = c > 0;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(incl, d, 64), oa = __shfl_up(incl_active, d, 64);
-            if (lane >= d) {
-                incl += o;
-                incl_active += oa;
-            }
-        }
+        const int c = e < n_experts ? expert_pairs(table, e) : 0;
+        int total, total_active;
+        int before = lanes_before(c, n_pairs, lane, total), active_before = lanes_before(c > 0 ? 1 : 0, 1, lane, total_active);
         if (lane == 63) {
-            wave_total[wave] = incl;
-            wave_active[wave] = incl_active;
+            wave_total[wave] = total;
+            wave_active[wave] = total_active;
         }
         __syncthreads();
-        int before = incl - c, active_before = incl_active - (c > 0);
         for (int w = 0; w < wave; ++w) {
             before += wave_total[w];
             active_before += wave_active[w];
@@ -400,22 +440,18 @@ __device__ void align_in_block(const int* pair_expert, int n_pairs, int n_expert
         }
     }
     __syncthreads();
-    if (mine >= 0) {
-        int rank = 0;
-        for (int q = 0; q < tid; ++q) rank += pair_expert[q] == mine;
-        list[offs[mine] + rank] = tid;
-    }
+    if (mine >= 0) list[offs[mine] + rank] = tid;
 }
 
 __global__ void __launch_bounds__(1024) moe_align_small_kernel(const int* __restrict__ ids, int n_pairs, int n_experts, int* __restrict__ counts,
                                                               int* __restrict__ offsets, int* __restrict__ list, int* __restrict__ active,
                                                               int* __restrict__ n_active) {
     __shared__ int pair_expert[ALIGN_SMALL_PAIRS];
-    __shared__ int cnt[1024];
+    __shared__ __attribute__((aligned(16))) PairTable table;
     __shared__ int offs[1024];
     for (int p = threadIdx.x; p < n_pairs; p += 1024) pair_expert[p] = ids[p];
     __syncthreads();
-    align_in_block(pair_expert, n_pairs, n_experts, cnt, offs, counts, offsets, list, active, n_active);
+    align_in_block(pair_expert, n_pairs, n_experts, table, offs, counts, offsets, list, active, n_active);
 }
 
 // Many pairs, with scratch [ceil(n_pairs / 1024)][n_experts] (at most 1024 experts): the pairs are cut into chunks of
@@ -436,38 +472,53 @@ __global__ void __launch_bounds__(1024) moe_chunk_count_kernel(const int* __rest
 
 __global__ void __launch_bounds__(1024) moe_chunk_scan_kernel(int n_chunks, int n_experts, int* __restrict__ chunk_counts, int* __restrict__ counts,
                                                              int* __restrict__ offsets, int* __restrict__ active, int* __restrict__ n_active,
-                                                             int* __restrict__ tiles128) {
-    __shared__ int wave_total[16], wave_active[16], wave_tiles[16];
+                                                             int* __restrict__ tiles128, int* __restrict__ tile_choice) {
+    __shared__ int wave_total[16], wave_active[16], wave_tiles[16], wave_halves[16];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int e = tid;
-    int c = 0;
-    if (e < n_experts)
-        for (int b = 0; b < n_chunks; ++b) c += chunk_counts[(size_t)b * n_experts + e];
-    int incl = c, incl_active = c > 0;
+    // chunks in batches whose counts are asked for together; the first batch stays in registers for the second pass
+    constexpr int BATCH = 16;
+    int first[BATCH], c = 0;
+    const int le = e < n_experts ? e : 0;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(incl, d, 64), oa = __shfl_up(incl_active, d, 64);
-        if (lane >= d) {
-            incl += o;
-            incl_active += oa;
-        }
+    for (int u = 0; u < BATCH; ++u) first[u] = chunk_counts[(size_t)min(u, n_chunks - 1) * n_experts + le];
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u) c += u < n_chunks ? first[u] : 0;
+    for (int b0 = BATCH; b0 < n_chunks; b0 += BATCH) {
+        int v[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) v[u] = chunk_counts[(size_t)min(b0 + u, n_chunks - 1) * n_experts + le];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) c += b0 + u < n_chunks ? v[u] : 0;
     }
-    // how many tiles of 128 rows the experts' runs make: the products choose their tile size by it
-    int t128 = (c + 127) / 128;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) t128 += __shfl_xor(t128, d, 64);
+    if (e >= n_experts) c = 0;
+    int total, total_active, tiles, halves;
+    int before = lanes_before(c, n_chunks * 1024, lane, total), active_before = lanes_before(c > 0 ? 1 : 0, 1, lane, total_active);
+    // how many tiles of 128 and of 64 rows the experts' runs make: the products choose their tile size by them
+    lanes_before((c + 127) / 128, n_chunks * 8, lane, tiles);
+    lanes_before((c + 63) / 64, n_chunks * 16, lane, halves);
     if (lane == 63) {
-        wave_total[wave] = incl;
-        wave_active[wave] = incl_active;
-        wave_tiles[wave] = t128;
+        wave_total[wave] = total;
+        wave_active[wave] = total_active;
+        wave_tiles[wave] = tiles;
+        wave_halves[wave] = halves;
     }
     __syncthreads();
     if (tid == 0 && tiles128) {
-        int sum = 0;
-        for (int w = 0; w < 16; ++w) sum += wave_tiles[w];
-        tiles128[0] = sum;
+        int n128 = 0, n64 = 0, experts = 0;
+        for (int w = 0; w < 16; ++w) {
+            n128 += wave_tiles[w];
+            n64 += wave_halves[w];
+            experts += wave_active[w];
+        }
+        tiles128[0] = n128;
+        // Which tiles the products take.  While an expert's weights stream from memory a first tile costs about 3.6 (64 rows) and 3.8
+        // (128) of what a further one of 64 costs 1.25 and of 128 2.5 (256 experts of 3,072 x 3,072, us x 256): 128-row tiles win
+        // when 3.8 A + 2.5 (n128 - A) < 3.6 A + 1.25 (n64 - A); where few experts share many rows the tiles' own time counts, 2.8
+        // against 1.7.  Measured, gate_up + down, 64- against 128-row tiles: 52 rows an expert 957 + 560 : 916 + 545 us, 65 rows 1,053 +
+        // 600 : 942 + 566, 80 rows 1,153 + 640 : 985 + 600, 160 rows 1,557 + 840 : 1,605 + 845; 55 experts of 300 490 + 297 : 478 + 286.
+        if (tile_choice) *tile_choice = 200L * n128 <= 84L * experts + 100L * n64 || 100L * n128 <= 61L * n64 ? 0 : 1 << 30;
     }
-    int before = incl - c, active_before = incl_active - (c > 0);
     for (int w = 0; w < wave; ++w) {
         before += wave_total[w];
         active_before += wave_active[w];
@@ -482,37 +533,38 @@ __global__ void __launch_bounds__(1024) moe_chunk_scan_kernel(int n_chunks, int 
     }
     // the chunks' first places within the expert's run, in chunk order
     int at = before;
-    for (int b = 0; b < n_chunks; ++b) {
-        const int n = chunk_counts[(size_t)b * n_experts + e];
-        chunk_counts[(size_t)b * n_experts + e] = at;
-        at += n;
+    for (int b0 = 0; b0 < n_chunks; b0 += BATCH) {
+        if (b0 > 0) {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) first[u] = chunk_counts[(size_t)min(b0 + u, n_chunks - 1) * n_experts + e];
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+            if (b0 + u < n_chunks) {
+                chunk_counts[(size_t)(b0 + u) * n_experts + e] = at;
+                at += first[u];
+            }
     }
 }
 
 __global__ void __launch_bounds__(1024) moe_chunk_place_kernel(const int* __restrict__ ids, int n_pairs, int n_experts,
                                                               const int* __restrict__ chunk_first, int* __restrict__ list) {
-    __shared__ __attribute__((aligned(16))) int pair_expert[1024];
+    __shared__ __attribute__((aligned(16))) PairTable table;
     const int tid = threadIdx.x, p = blockIdx.x * 1024 + tid;
     int e = p < n_pairs ? ids[p] : -1;
     if (e >= n_experts) e = -1;
-    pair_expert[tid] = e;
-    __syncthreads();
+    const int first = e >= 0 ? chunk_first[(size_t)blockIdx.x * n_experts + e] : 0;
+    const int rank = rank_in_block(table, e, n_experts);
     if (e < 0) return;
-    int rank = 0;
-    const int whole = tid & ~3;
-    for (int q = 0; q < whole; q += 4) {
-        const int4 v = *reinterpret_cast<const int4*>(&pair_expert[q]);
-        rank += (v.x == e) + (v.y == e) + (v.z == e) + (v.w == e);
-    }
-    for (int q = whole; q < tid; ++q) rank += pair_expert[q] == e;
-    list[chunk_first[(size_t)blockIdx.x * n_experts + e] + rank] = p;
+    list[first + rank] = p;
 }
 
 // counts [X], offsets [X+1], list [n_pairs], active [X], n_active [1]
 // scratch (optional): [ceil(n_pairs / 1024) * n_experts] ints for steps of many pairs
-// tiles128 (optional) [1]: with scratch and many pairs, the sum over experts of ceil(rows / 128)
+// tiles128 (optional) [1]: with scratch and many pairs, the sum over experts of ceil(rows / 128); tile_choice (optional, with
+// tiles128): what the routed products take in its place: 0 for tiles of 128 rows, 2^30 for tiles of 64
 extern "C" int llmx_moe_align(const int* ids, int n_pairs, int n_experts, int* counts, int* offsets, int* list, int* active, int* n_active,
-                              int* scratch, int* tiles128, hipStream_t stream) {
+                              int* scratch, int* tiles128, int* tile_choice, hipStream_t stream) {
     if (n_pairs <= 0 || n_experts <= 0) return 0;
     llmx_note_launch(LK_MOE_ALIGN);
     if (n_pairs <= ALIGN_SMALL_PAIRS && n_experts <= 1024) {
@@ -522,7 +574,8 @@ extern "C" int llmx_moe_align(const int* ids, int n_pairs, int n_experts, int* c
     if (scratch && n_experts <= 1024) {
         const int n_chunks = (n_pairs + 1023) / 1024;
         hipLaunchKernelGGL(moe_chunk_count_kernel, dim3(n_chunks), dim3(1024), 0, stream, ids, n_pairs, n_experts, scratch);
-        hipLaunchKernelGGL(moe_chunk_scan_kernel, dim3(1), dim3(1024), 0, stream, n_chunks, n_experts, scratch, counts, offsets, active, n_active, tiles128);
+        hipLaunchKernelGGL(moe_chunk_scan_kernel, dim3(1), dim3(1024), 0, stream, n_chunks, n_experts, scratch, counts, offsets, active, n_active, tiles128,
+                           tile_choice);
         hipLaunchKernelGGL(moe_chunk_place_kernel, dim3(n_chunks), dim3(1024), 0, stream, ids, n_pairs, n_experts, scratch, list);
         return LLMX_CHECK_LAUNCH();
     }
@@ -542,7 +595,7 @@ __global__ void __launch_bounds__(1024) route_topk_align_kernel(float* __restric
                                                                int* __restrict__ counts, int* __restrict__ offsets, int* __restrict__ list,
                                                                int* __restrict__ active, int* __restrict__ n_active) {
     __shared__ int pair_expert[ALIGN_SMALL_PAIRS];
-    __shared__ int cnt[1024];
+    __shared__ __attribute__((aligned(16))) PairTable table;
     __shared__ int offs[1024];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     for (int r = wave; r < rows; r += 16) {
@@ -563,7 +616,7 @@ __global__ void __launch_bounds__(1024) route_topk_align_kernel(float* __restric
         }
     }
     __syncthreads();
-    align_in_block(pair_expert, rows * ldk, n_experts + (ldk - k), cnt, offs, counts, offsets, list, active, n_active);
+    align_in_block(pair_expert, rows * ldk, n_experts + (ldk - k), table, offs, counts, offsets, list, active, n_active);
 }
 
 // At most 16 rows (a wave each), rows * k <= 1024, at most 256 experts and 64 picks.  Returns -2 otherwise.

@@ -108,7 +108,7 @@ def _declare(h) -> None:
         "llmx_memory_prep": [P, I, I, I, I, I, P, P, F, P, L, I, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
         "llmx_paged_attention_mfma": [P, P, P, P, P, P, P, I, I, I, P, I, P, P, P, F, I, I, I, I, I, I, I, P, I, I, P],
         "llmx_route_topk": [P, P, I, L, P, P, P, I, I, I, I, I, F, P, I, I, I, P],
-        "llmx_moe_align": [P, I, I, P, P, P, P, P, P, P, P],
+        "llmx_moe_align": [P, I, I, P, P, P, P, P, P, P, P, P],
         "llmx_route_topk_align": [P, P, I, L, P, P, P, I, I, I, I, I, F, I, I, I, P, P, P, P, P, P],
         "llmx_gemm_skinny": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, P, P, I, L, I, P, P, F, I, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_skinny_normed_ok": [I, I],
@@ -1243,7 +1243,7 @@ def grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, offsets: tor
         _check(lib().llmx_gemm_tile(_dev(a, "a"), _dev(w, "w"), _dev(c, "c"), _code(c.dtype), n_pairs, N, K, K, N, epilogue,
                                     _split_k(-(-N // 16), K), G, min(G, n_pairs) + n_pairs // 64, _dev(offsets, "offsets", torch.int32, (G + 1,)),
                                     _dev(pairs, "pairs", torch.int32), a_div, NW * K, N if epilogue == EPI_SWIGLU else 0,
-                                    _dev(tile_stats if n_pairs >= TILE_STATS_MIN_PAIRS else None, "tile_stats", torch.int32, (1,)), 0, *act_args, *glu_args, _stream()),
+                                    _dev(tile_stats[-1:] if tile_stats is not None and n_pairs >= TILE_STATS_MIN_PAIRS else None, "tile_stats", torch.int32, (1,)), 0, *act_args, *glu_args, _stream()),
                "grouped_gemm_tile")
         return
     _check(lib().llmx_gemm_generic(_dev(a, "a"), _code(a.dtype), _dev(w, "w"), _code(w.dtype), _dev(c, "c"), _code(c.dtype),
@@ -1661,7 +1661,8 @@ def moe_align(ids: torch.Tensor, n_experts: int, counts: torch.Tensor, offsets: 
     """Groups the pairs p = t*k + j by expert (stable): counts [X], offsets [X+1], pairs [T*k], and the experts that
     have rows in increasing order: active [X] (first n_active[0] entries).  `scratch`: moe_align_scratch(...) int32 for
     steps of many pairs (made here when it is not given).  `tile_stats` int32 [1]: for TILE_STATS_MIN_PAIRS pairs or
-    more it receives the sum over experts of ceil(rows / 128), by which grouped_gemm chooses its tile size."""
+    more it receives the sum over experts of ceil(rows / 128), by which grouped_gemm chooses its tile size; int32 [2]: behind it
+    the choice itself, from the tiles of both sizes and the experts that have rows, which grouped_gemm then follows."""
     n_pairs = ids.numel()
     need = moe_align_scratch(n_pairs, n_experts)
     if need and scratch is None:
@@ -1672,7 +1673,8 @@ def moe_align(ids: torch.Tensor, n_experts: int, counts: torch.Tensor, offsets: 
                                 _dev(offsets, "offsets", torch.int32, (n_experts + 1,)), _dev(pairs, "pairs", torch.int32, (n_pairs,)),
                                 _dev(active, "active", torch.int32, (n_experts,)), _dev(n_active, "n_active", torch.int32, (1,)),
                                 _dev(scratch if need else None, "scratch", torch.int32),
-                                _dev(tile_stats if need and n_pairs >= TILE_STATS_MIN_PAIRS else None, "tile_stats", torch.int32, (1,)),
+                                *((_dev(tile_stats[:1], "tile_stats", torch.int32, (1,)), _dev(tile_stats[1:] if tile_stats.shape[0] > 1 else None, "tile_choice", torch.int32, (1,)))
+                                  if tile_stats is not None and need and n_pairs >= TILE_STATS_MIN_PAIRS else (None, None)),
                                 _stream()), "moe_align")
 
 

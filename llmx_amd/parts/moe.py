@@ -206,7 +206,7 @@ class RoutedExperts(FeedForward):
         need = ops.moe_align_scratch(T * slots, groups)
         scratch = step.buf("experts.align_scratch", (need,), torch.int32) if need else None
         # for steps of many pairs the grouping also counts the experts' tiles of 128 rows, by which the products choose their tiles
-        tile_stats = step.buf("experts.tile_stats", (1,), torch.int32) if T * slots >= ops.TILE_STATS_MIN_PAIRS else None
+        tile_stats = step.buf("experts.tile_stats", (2,), torch.int32) if T * slots >= ops.TILE_STATS_MIN_PAIRS else None
         ops.route_topk_align(z, self.bias, ids, weights, k, self.score, self.normalize, self.scale, counts, offsets, pairs, active, n_active,
                              parts=parts, scratch=scratch, tile_stats=tile_stats, logit_bias=self.logit_bias, groups=self.groups)
         step.observe("routing", logits=z, ids=ids[:, :k], weights=weights[:, :k])
