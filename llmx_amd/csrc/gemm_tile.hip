@@ -28,7 +28,12 @@ enum : int { TL_STORE = 0, TL_ADD = 1, TL_SWIGLU = 2 };
 #define TL_BN 128
 #define TL_BK 64
 #define TL_LD 72  // padded row length in bf16 elements (144 bytes)
-#define TILE_RUNS_APART_BELOW 256   // dense products with fewer 64 x 128 tiles than this multiply K's runs in workgroups of their own (measured: 8,192 features up to 192 rows, 3,072 features of K 6,144 up to 640 rows)
+// Dense products of fewer 64 x 128 tiles than this multiply K's runs in workgroups of their own; with more the deep form below walks
+// all of K in one (3,072 features of 6,144 values, runs apart against deep: 144 tiles 40 and 47 us, 192 tiles 49 and 47.5; 8,192 of 3,072:
+// 128 tiles 23.5 and 27.7, 192 tiles 29.7 and 27.8; 2,048 of 2,048: 64 tiles 14.3 and 15.4, 128 tiles 16.8 and 15.8; of 8,192: 160 tiles 48 and 57)
+#define TILE_RUNS_APART_BELOW(K) (100 + (K) / 96)
+#define TL_DEEP_STAGES 3  // ... where no CU gets more than two workgroups (72 KB each): a tile asked for one ahead then arrives a whole trip to memory later, with nobody else to work meanwhile
+#define TL_DEEP_BELOW 512 // (K 8,192, 2,048 features: 512 rows 89 -> 55 us, 1,024 rows 92 -> 59, 2,048 rows 98 -> 87; four stages, one workgroup a CU: 53, 56, 104; 800 tiles of K 2,048, three a CU with two stages: 47 against 40, the wide form 34)
 #define TL_STAGES 2  // tiles in LDS in the lean loop: one being multiplied, the other on its way (48 KB: three workgroups a CU; measured better than deeper stages with fewer workgroups)
 
 // Lane l of the wave: 16 bytes from base + offset (bytes, per lane) to LDS at lds + 16 l (lds the same for the whole
@@ -100,14 +105,35 @@ __device__ __forceinline__ bool tile_launch_runs(const TileArgs& g) {
     return big == (g.run_if_big != 0);
 }
 
+// Which tile a workgroup takes.  Workgroups go round the 8 XCDs in launch order, each with an L2 of its own.  Strips of weights in a
+// multiple of 8 stay on one XCD each as they are launched; any other number of them moves on from row tile to row tile, so that every
+// XCD fetches every strip.  Then an XCD takes a contiguous run of tiles in the order strip after strip, a strip's row tiles together
+// (2,048 rows of 2,048 values: 10,880 features, 43 strips of the wide form, 130 -> 115 us, 85 of the narrow 206 -> 141; for 8,192
+// features, 32 strips, it would be 104 -> 114).  Routed products keep the launch order: an expert's strips, side by side, stream one
+// stretch of memory (256 experts of 3,072 x 3,072, 52 rows each: 916 us, strip after strip 1,010).
+#define TILE_XCDS 8
+template <bool GROUPED>
+__device__ __forceinline__ void tile_place(int& strip, int& rows) {
+    const int gx = gridDim.x, gy = gridDim.y;
+    if (GROUPED || gx % TILE_XCDS == 0) {
+        strip = blockIdx.x;
+        rows = blockIdx.y;
+        return;
+    }
+    const int total = gx * gy, at = (int)blockIdx.y * gx + (int)blockIdx.x;
+    const int xcd = at % TILE_XCDS, share = total / TILE_XCDS, more = total % TILE_XCDS;
+    const int tile = xcd * share + min(xcd, more) + at / TILE_XCDS;
+    strip = tile / gy;
+    rows = tile - strip * gy;
+}
+
 // FAST: K is a multiple of 64 and the runs end on multiples of 64, so nothing in the loop needs a bound: the tiles are
 // loaded without conditions (a row past the tile's rows reads the first row, a feature past N the last; what they
 // produce is never stored, and a column of the product never touches another), straight into LDS, TL_STAGES deep,
 // one barrier a tile.
-template <int EPI, typename TC, bool GROUPED, bool SPLIT, bool FAST, int BM>
+template <int EPI, typename TC, bool GROUPED, bool SPLIT, bool FAST, int BM, int STAGES = TL_STAGES>
 __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
-    // FAST: TL_STAGES tiles of unpadded 128-byte rows whose 16-byte chunks are swizzled; else one tile of padded rows
-    constexpr int STAGES = TL_STAGES;
+    // FAST: STAGES tiles of unpadded 128-byte rows whose 16-byte chunks are swizzled; else one tile of padded rows
     __shared__ __attribute__((aligned(1024))) bf16_t As[FAST ? STAGES * BM * TL_BK : BM * TL_LD];
     __shared__ __attribute__((aligned(1024))) bf16_t Ws[FAST ? STAGES * TL_BN * TL_BK : TL_BN * TL_LD];
     __shared__ int rows_a[BM];
@@ -118,7 +144,9 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const bool runs = !GROUPED || tile_launch_runs(g);   // looked at below, once the first offsets are asked for too
     constexpr int FEATS = (EPI == TL_SWIGLU) ? 64 : 128;  // output features a workgroup covers
-    const int n0 = blockIdx.x * FEATS;
+    int strip, row_tile;
+    tile_place<GROUPED>(strip, row_tile);
+    const int n0 = strip * FEATS;
     const bf16_t* W = g.W;
     int row_begin, row_end;
     if (GROUPED) {
@@ -144,14 +172,14 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
             for (int w = 0; w < wave; ++w) before += scan_waves[w];
             const int round_total = scan_waves[0] + scan_waves[1] + scan_waves[2] + scan_waves[3];
             const int first = before + incl - tiles;
-            if ((int)blockIdx.y >= first && (int)blockIdx.y < first + tiles) {
+            if (row_tile >= first && row_tile < first + tiles) {
                 tile_info[0] = e;
-                tile_info[1] = begin + ((int)blockIdx.y - first) * BM;
+                tile_info[1] = begin + (row_tile - first) * BM;
                 tile_info[2] = end;
             }
             base += round_total;
             __syncthreads();
-            if ((int)blockIdx.y < base) break;
+            if (row_tile < base) break;
         }
         __syncthreads();
         const int e = tile_info[0];
@@ -160,7 +188,7 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
         row_end = min(tile_info[2], row_begin + BM);
         W += (size_t)e * g.w_group_stride;
     } else {
-        row_begin = blockIdx.y * BM;
+        row_begin = row_tile * BM;
         row_end = min(g.M, row_begin + BM);
     }
     if (tid < BM) {
@@ -494,7 +522,9 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
     const bool runs = !GROUPED || tile_launch_runs(g);   // looked at below, once the first offsets are asked for too
     constexpr int HALF = WD_BN / 2;                               // SwiGLU: gate rows, then the up rows of the same features
     constexpr int FEATS = (EPI == TL_SWIGLU) ? HALF : WD_BN;      // output features a workgroup covers
-    const int n0 = blockIdx.x * FEATS;
+    int strip, row_tile;
+    tile_place<GROUPED>(strip, row_tile);
+    const int n0 = strip * FEATS;
     const bf16_t* W = g.W;
     int row_begin, row_end;
     if (GROUPED) {
@@ -521,14 +551,14 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
                 round_total += scan_waves[w];
             }
             const int first = before + incl - tiles;
-            if ((int)blockIdx.y >= first && (int)blockIdx.y < first + tiles) {
+            if (row_tile >= first && row_tile < first + tiles) {
                 tile_info[0] = e;
-                tile_info[1] = begin + ((int)blockIdx.y - first) * WD_BM;
+                tile_info[1] = begin + (row_tile - first) * WD_BM;
                 tile_info[2] = end;
             }
             base += round_total;
             __syncthreads();
-            if ((int)blockIdx.y < base) break;
+            if (row_tile < base) break;
         }
         __syncthreads();
         const int e = tile_info[0];
@@ -537,7 +567,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
         row_end = min(tile_info[2], row_begin + WD_BM);
         W += (size_t)e * g.w_group_stride;
     } else {
-        row_begin = blockIdx.y * WD_BM;
+        row_begin = row_tile * WD_BM;
         row_end = min(g.M, row_begin + WD_BM);
     }
     if (tid < WD_BM) {
@@ -739,13 +769,14 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
 
 // form: which kernel takes the product.  The lean forms need whole 64-wide tiles of K, runs that end on them, and
 // operands whose byte offsets fit 32 bits (llmx_gemm_tile_offsets_fit).
-enum : int { FORM_64 = 0, FORM_128 = 1, FORM_WIDE = 2, FORM_BOUNDED = 3 };
+enum : int { FORM_64 = 0, FORM_128 = 1, FORM_WIDE = 2, FORM_BOUNDED = 3, FORM_64_DEEP = 4 };
 
 template <int EPI, typename TC, bool GROUPED, bool SPLIT>
 static void tile_launch_form(const TileArgs& g, int form, dim3 grid, hipStream_t stream) {
     if (form == FORM_WIDE) hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT>), grid, dim3(512), 0, stream, g);
     else if (form == FORM_128) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, true, 128>), grid, dim3(256), 0, stream, g);
     else if (form == FORM_64) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, true, 64>), grid, dim3(256), 0, stream, g);
+    else if (form == FORM_64_DEEP && !GROUPED) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, false, SPLIT, true, 64, TL_DEEP_STAGES>), grid, dim3(256), 0, stream, g);
     else hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, false, 64>), grid, dim3(256), 0, stream, g);
 }
 
@@ -822,7 +853,7 @@ __global__ void __launch_bounds__(256) gemm_runs_sum_kernel(const float* __restr
     store_quad<ADD>(C + (size_t)m * ldc, n, N, ldc % 4 == 0 && ((uintptr_t)C & 15) == 0, v);
 }
 
-static int form_rows(int form) { return form == FORM_64 || form == FORM_BOUNDED ? 64 : 128; }
+static int form_rows(int form) { return form == FORM_WIDE || form == FORM_128 ? 128 : 64; }
 static int form_feats(int form, int epi) { return (epi == TL_SWIGLU ? 64 : 128) * (form == FORM_WIDE ? 2 : 1); }
 
 // A and W bfloat16, K a multiple of 8.  n_groups == 0: dense over M rows.  n_groups > 0: grouped over the n_pairs = M
@@ -831,8 +862,10 @@ static int form_feats(int form, int epi) { return (epi == TL_SWIGLU ? 64 : 128) 
 // tile_stats (grouped, optional): device int [1], the sum over groups of ceil(rows / 128), from the grouping.
 //
 // Which form runs (every form gives an output element the same bits):
-//   dense: the wide form (8 waves, 128 x 256, three tiles deep) where it has at least 192 tiles for the 256 CUs
-//     (measured on 2,048 rows: 8,192 features 113 against 165 us, 3,072 features 100 against 108 us), else 64-row
+//   dense: up to 512 tiles of 64 rows the 64-row form three tiles deep (two workgroups a CU at most); else the wide form (8
+//     waves, 128 x 256, three tiles deep) where it has at least 192 tiles for the 256 CUs, of long K 150
+//     (measured on 2,048 rows: 8,192 features 113 against 165 us, 3,072 features 100 against 108 us; 1,600 rows of 3,072
+//     features of 6,144 values, 156 tiles: 86 against 92), else 64-row
 //     tiles (three workgroups a CU; more, smaller tiles fill the chip better when there are few, and up to 64 rows half
 //     of a 128-row tile is padding: 200,064 features of 3,072, 48 rows 265 -> 257 us, 64 rows 276 -> 268).
 //     With `runs_scratch` (llmx_gemm_tile_runs_scratch floats) a product of few tiles and several runs of K gives each
@@ -845,7 +878,7 @@ extern "C" long llmx_gemm_tile_runs_scratch(int M, int N, int K, int epi, int ks
     const int steps = (K + 31) / 32, per = (steps + ks - 1) / ks;
     if (per % 2) return 0;
     const long tiles = (long)((M + 63) / 64) * ((N + TL_BN - 1) / TL_BN);
-    if (tiles >= TILE_RUNS_APART_BELOW) return 0;     // enough workgroups without
+    if (tiles >= TILE_RUNS_APART_BELOW(K)) return 0;     // enough workgroups without
     const int runs = (K / TL_BK + per / 2 - 1) / (per / 2);
     return runs < 2 ? 0 : (long)runs * M * N;
 }
@@ -873,7 +906,7 @@ extern "C" int llmx_gemm_tile(const void* A, const void* W, void* C, int c_dtype
         if (grid.y > 65535) return -2;
         llmx_note_launch(form == FORM_WIDE ? (grouped ? LK_GEMM_TILE_GROUPED_WIDE : LK_GEMM_TILE_WIDE)
                          : form == FORM_128 ? LK_GEMM_TILE_GROUPED_128
-                         : form == FORM_64 ? (grouped ? LK_GEMM_TILE_GROUPED_64 : LK_GEMM_TILE_64)
+                         : form == FORM_64 || form == FORM_64_DEEP ? (grouped ? LK_GEMM_TILE_GROUPED_64 : LK_GEMM_TILE_64)
                                            : (grouped ? LK_GEMM_TILE_GROUPED_BOUNDED : LK_GEMM_TILE_BOUNDED));
         return tile_launch_typed(g, form, grid, grouped, epi, c_dtype, stream);
     };
@@ -907,7 +940,8 @@ extern "C" int llmx_gemm_tile(const void* A, const void* W, void* C, int c_dtype
         rc = 0;
     } else if (!grouped) {
         const long wide_tiles = (long)((M + WD_BM - 1) / WD_BM) * ((N + form_feats(FORM_WIDE, epi) - 1) / form_feats(FORM_WIDE, epi));
-        rc = launch(wide_tiles >= 192 && M > 64 ? FORM_WIDE : FORM_64, 0);
+        const long narrow_tiles = (long)((M + 63) / 64) * ((N + form_feats(FORM_64, epi) - 1) / form_feats(FORM_64, epi));
+        rc = launch(narrow_tiles <= TL_DEEP_BELOW ? FORM_64_DEEP : wide_tiles >= (K >= 4096 ? 150 : 192) && M > 64 ? FORM_WIDE : FORM_64, 0);
     } else if (tile_stats) {
         // 128-row tiles: each group adds at most one partial tile
         const int big_tiles = (n_groups < M ? n_groups : M) + M / 128;
