@@ -198,7 +198,8 @@ class ChannelDeltaRule(Mixer):
         self.w_in = self.conv = self.a_log = self.dt_bias = self.w_low = self.norm = self.w_o = None
 
     def cache_need(self):
-        return StateNeed((self.state_matrix + (self.taps - 1) * self.channels,), "float32")
+        # slots a multiple of four floats apart, so that the step of single tokens reads them 16 bytes at a time
+        return StateNeed((-(-(self.state_matrix + (self.taps - 1) * self.channels) // 4) * 4,), "float32")
 
     def tensor_specs(self, available):
         E, H, D, V = self.hidden, self.heads, self.dim, self.vdim
@@ -238,14 +239,19 @@ class ChannelDeltaRule(Mixer):
         low = step.buf("delta.low", (T, H * D + H * V), f32)
         ops.gemm(inner, self.w_low, low, scratch=step.buf)
         step_pre, gate_pre = low[:, :H * D], low[:, H * D:]
-        q, k = step.buf("delta.q", (T, G * D), f32), step.buf("delta.k", (T, G * D), f32)
-        v, decay, beta = step.buf("delta.v", (T, H * V), f32), step.buf("delta.decay", (T, H * D), f32), step.buf("delta.beta", (T, H), f32)
-        ops.delta_prep(pre, self.conv, step_pre, self.dt_bias, self.a_log, cache.state, self.state_matrix, step.entry_held_slots,
-                       step.row_entry, step.entry_rows, q, k, v, decay, beta, G, H, D, V, self.cols["b"][0])
         o = step.buf("delta.o", (T, H * V), f32)
-        tail = (pre[:, :self.channels], self.taps, self.state_matrix) if self.taps > 1 else None
-        ops.state_scan(q, k, v, decay, beta, cache.state, step.entry_held_slots, step.entry_slots, step.entry_rows, o, float(D) ** -0.5,
-                       H, G, D, V, tail=tail, max_rows=step.max_rows_per_entry)
+        # single tokens: one launch, the scan's bits (a token's preparation and scan at 16 heads of 128 x 128: 15 -> 8 us)
+        if step.max_rows_per_entry == 1 and ops.delta_step_ok(D, cache.state):
+            ops.delta_step(pre, self.conv, step_pre, self.dt_bias, self.a_log, cache.state, self.state_matrix, step.entry_held_slots,
+                           step.entry_slots, step.entry_rows, o, float(D) ** -0.5, G, H, D, V, self.cols["b"][0])
+        else:
+            q, k = step.buf("delta.q", (T, G * D), f32), step.buf("delta.k", (T, G * D), f32)
+            v, decay, beta = step.buf("delta.v", (T, H * V), f32), step.buf("delta.decay", (T, H * D), f32), step.buf("delta.beta", (T, H), f32)
+            ops.delta_prep(pre, self.conv, step_pre, self.dt_bias, self.a_log, cache.state, self.state_matrix, step.entry_held_slots,
+                           step.row_entry, step.entry_rows, q, k, v, decay, beta, G, H, D, V, self.cols["b"][0])
+            tail = (pre[:, :self.channels], self.taps, self.state_matrix) if self.taps > 1 else None
+            ops.state_scan(q, k, v, decay, beta, cache.state, step.entry_held_slots, step.entry_slots, step.entry_rows, o, float(D) ** -0.5,
+                           H, G, D, V, tail=tail, max_rows=step.max_rows_per_entry)
         gated = step.buf("delta.gated", (T, H * V), step.act_dtype)
         ops.head_norm_gate(o, self.norm, gate_pre, gated, self.eps, H, V, ops.GATE_SIGMOID)
         ops.gemm(gated, self.w_o, out, ops.EPI_ADD if accumulate else ops.EPI_STORE, scratch=step.buf)

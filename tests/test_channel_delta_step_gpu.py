@@ -1,0 +1,42 @@
+"""The delta rule's step of single tokens with one decay a key channel, against preparation and scan as launches of their own."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# (heads, key groups, key channels, value channels, taps): key channels at and beside each width of a workgroup (64, 128, 256),
+# value channels short of a tile and over several workgroups, no convolution, slots whose size is no multiple of four floats
+@pytest.mark.parametrize("H,G,D,V,taps", [(4, 2, 16, 24, 3), (3, 3, 5, 7, 1), (2, 1, 64, 64, 4), (6, 2, 65, 33, 2), (2, 1, 128, 128, 4), (1, 1, 129, 1, 8), (1, 1, 256, 100, 4)])
+@pytest.mark.parametrize("entries", [1, 9])
+def test_a_single_token_has_the_bits_of_preparation_and_scan(H, G, D, V, taps, entries):
+    from llmx_amd import ops
+
+    gen = torch.Generator().manual_seed(H * 1000 + D * 10 + taps)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    C, T = 2 * G * D + H * V, entries
+    matrix = ops.state_matrix_size(H, D, V)
+    stride = -(-(matrix + (taps - 1) * C) // 4) * 4
+    pre, conv, low = rand(T, C + H + 3), rand(C, taps) * 0.6, rand(T, H * D + H * V)
+    step_pre, dt_bias, a_log = low[:, :H * D], rand(H * D), rand(H) - 1.0
+    start = rand(2 * T + 1, stride)
+    held, written = i32(range(T)), i32([2 * T - 1 - e for e in range(T)])
+    rows, entry = i32([[e, 1] for e in range(T)]), i32(range(T))
+
+    one, apart = start.clone(), start.clone()
+    got, want = torch.full((T, H * V), 9.0, device="cuda"), torch.full((T, H * V), 7.0, device="cuda")
+    assert ops.delta_step_ok(D, one)
+    ops.delta_step(pre, conv, step_pre, dt_bias, a_log, one, matrix, held, written, rows, got, D ** -0.5, G, H, D, V, C)
+    q, k, v, decay, beta = (torch.empty(T, w, device="cuda") for w in (G * D, G * D, H * V, H * D, H))
+    ops.delta_prep(pre, conv, step_pre, dt_bias, a_log, apart, matrix, held, entry, rows, q, k, v, decay, beta, G, H, D, V, C)
+    tail = (pre[:, :C], taps, matrix) if taps > 1 else None
+    ops.state_scan(q, k, v, decay, beta, apart, held, written, rows, want, D ** -0.5, H, G, D, V, tail=tail, max_rows=1)
+    assert torch.equal(got, want)
+    for s in written.tolist():          # what a request keeps; a tile's columns beyond V and the slot's padding are nobody's
+        assert torch.equal(ops.state_matrix_plain(one[s], H, D, V), ops.state_matrix_plain(apart[s], H, D, V))
+        assert torch.equal(one[s, matrix:matrix + (taps - 1) * C], apart[s, matrix:matrix + (taps - 1) * C])
+    assert torch.equal(one[:T], start[:T]) and torch.equal(one[2 * T], start[2 * T])
+    assert np.isfinite(got.cpu().numpy()).all()
