@@ -168,9 +168,14 @@ __device__ __forceinline__ float strided_squares(const float* __restrict__ row, 
 // block.  store(row, i, y) receives every element.  Rows of at most 4,096 values with at least 4 waves are kept in
 // registers, all asked for (with the weights) before anything is added, so the workgroup waits for memory once a row.
 // scratch32: 32 floats of LDS.  The caller puts a barrier between the stores and their first read.
-template <int NW, typename Store>
+// meanwhile(): called once, when the first row's values are on their way (or before them, for rows that are not kept): what the caller
+// asks memory for beside the norm goes there, behind what the norm waits for.
+struct NothingMeanwhile {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <int NW, typename Store, typename Meanwhile = NothingMeanwhile>
 __device__ __forceinline__ void rms_rows_as_1024(const float* __restrict__ X, size_t ldx, int rows, int n, const float* __restrict__ w,
-                                                 float eps, float* scratch32, Store store) {
+                                                 float eps, float* scratch32, Store store, Meanwhile meanwhile = Meanwhile()) {
     static_assert(NW == 1 || NW == 2 || NW == 4 || NW == 8 || NW == 16, "waves of the workgroup");
     constexpr int VW = 16 / NW;       // waves of the 1,024-thread block that one wave stands for
     constexpr int KEPT = 4;
@@ -195,6 +200,11 @@ __device__ __forceinline__ void rms_rows_as_1024(const float* __restrict__ X, si
                     const int i = (wave + j * NW) * LLMX_WAVE + lane + e * 1024;
                     v[j][e] = i < n ? x[i] : 0.0f;
                 }
+            if (row == 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                meanwhile();
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int j = 0; j < VW; ++j) {
                 float sq = 0.0f;     // an element past the end adds fmaf(0, 0, s) = s
@@ -218,6 +228,7 @@ __device__ __forceinline__ void rms_rows_as_1024(const float* __restrict__ X, si
         }
         return;
     }
+    meanwhile();
     for (int row = 0; row < rows; ++row) {
         const float* x = X + (size_t)row * ldx;
         float* scratch = scratch32 + 16 * (row & 1);
@@ -241,9 +252,11 @@ __device__ __forceinline__ void rms_rows_as_1024(const float* __restrict__ X, si
 // wave_sum, the four waves' sums in wave order; then the squared deviations likewise, each with fmaf.  A workgroup of NW waves does the
 // same: wave w stands for the waves w, w + NW, ... of those four (with 8 waves the last four only wait).  Rows of n values, n a multiple
 // of 4, at most 4,096; 16-byte aligned.  scratch32: 32 floats of LDS.  The caller puts a barrier between the stores and their first read.
-template <int NW, typename Store>
+// meanwhile(): as above.
+template <int NW, typename Store, typename Meanwhile = NothingMeanwhile>
 __device__ __forceinline__ void layer_norm_rows_as_256(const float* __restrict__ X, size_t ldx, int rows, int n, const float* __restrict__ w,
-                                                       const float* __restrict__ bias, float eps, float* scratch32, Store store) {
+                                                       const float* __restrict__ bias, float eps, float* scratch32, Store store,
+                                                       Meanwhile meanwhile = Meanwhile()) {
     typedef float quad_t __attribute__((ext_vector_type(4)));
     constexpr int VW = NW >= 4 ? 1 : 4 / NW;      // waves of the 256-thread block that one wave stands for
     const int wave = threadIdx.x / LLMX_WAVE, lane = threadIdx.x & (LLMX_WAVE - 1);
@@ -261,6 +274,11 @@ __device__ __forceinline__ void layer_norm_rows_as_256(const float* __restrict__
                 wk[u][j] = in ? *reinterpret_cast<const quad_t*>(w + at) : quad_t{0.0f, 0.0f, 0.0f, 0.0f};
                 bk[u][j] = in ? *reinterpret_cast<const quad_t*>(bias + at) : quad_t{0.0f, 0.0f, 0.0f, 0.0f};
             }
+        if (row == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            meanwhile();
+            __builtin_amdgcn_sched_barrier(0);
+        }
         float* scratch = scratch32 + 8 * (row & 1);       // rows take turns in two sets
 #pragma unroll
         for (int u = 0; u < VW; ++u) {

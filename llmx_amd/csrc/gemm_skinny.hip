@@ -7,6 +7,12 @@
 // An output element is sum over waves (in order) of sum over that wave's k-steps (in order) of one MFMA's 32 products:
 // its bits depend on K and KS only, not on M or on the other rows.
 //
+// What bounds it is the weights' way from memory: whole lines asked for as bytes read once (two_steps), and loads that wait for nothing but
+// themselves (the rounds below; with a condition at each load the compiler waited for everything on its way before it multiplied).  MiniMax-M3's
+// layers, us, half lines kept by the caches and before: gate_up 8 rows of 57 experts 188 -> 158 (6.8 TB/s), 1 row of 8 experts 33.3 -> 29.0; down
+// 95.7 -> 85.8 and 18.8 -> 15.4; one row of 200,064 features 215 -> 190.  The kernels between them gain by what the caches still hold: routing 9.5 ->
+// 8.0, q and k norms 6.5 -> 6.0, a batch of 1 752 -> 683 us a step.
+//
 // Grouped form: blockIdx.y walks the experts that have rows; A's rows are gathered through the expert-sorted pair list
 // and C's rows scattered to the pairs.  The SwiGLU form streams a gate strip and the matching up strip together and
 // stores silu(gate) * up.
@@ -15,6 +21,7 @@
 // instead of A; every workgroup forms the normed, rounded rows itself (in LDS) while its first weights travel, and no
 // norm kernel is launched.  The rows' values are the norm kernel's, bit for bit.  With a bias the norm is a layer norm.
 #include "common.h"
+#include <type_traits>
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -54,27 +61,53 @@ __device__ __forceinline__ bf16x8_t load_frag(const bf16_t* p, bool in) {
     return __builtin_bit_cast(bf16x8_t, v);
 }
 
+// Two steps of a strip's weights (16 rows of 32 k, twice).  Memory gives and the caches keep lines of 128 bytes, so the loads are whole
+// lines, eight rows' each, and the halves that belong to another lane are exchanged between lanes 8 apart in a row of 16: lane (r, kg) asks
+// for chunk kg + 4 (r / 8) (of 8 of 16 bytes) of rows r % 8 and 8 + r % 8.  Whole lines can be asked for as bytes that are read once
+// (LINES), which the caches then do not keep: a kernel that only reads gets 7.1 TB/s that way and 6.3 without, and what the step's other
+// kernels read stays near; half lines asked for so arrive twice (5.6 TB/s).
+struct WeightLines {
+    u32x4_t lo, hi;
+};
+// A strip's rows as the loads see them: 32-bit byte offsets from a base the wave shares; what lies past the strip's last row reads as 0.
+typedef __amdgpu_buffer_rsrc_t strip_t;
+__device__ __forceinline__ strip_t strip_of(const bf16_t* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00027000);
+}
+template <bool LINES>
+__device__ __forceinline__ u32x4_t load_line(strip_t strip, uint32_t lane_byte, uint32_t wave_byte) {
+    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(strip, (int)lane_byte, (int)wave_byte, LINES ? 2 : 0));
+}
+__device__ __forceinline__ void two_steps(const WeightLines& l, bf16x8_t (&step)[2]) {
+    u32x4_t a, b;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        a[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)l.lo[i], (int)l.hi[i], 0x128, 0xf, 0xc, false);
+        b[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)l.hi[i], (int)l.lo[i], 0x128, 0xf, 0x3, false);
+    }
+    step[0] = __builtin_bit_cast(bf16x8_t, a);
+    step[1] = __builtin_bit_cast(bf16x8_t, b);
+}
+
 // NORM: what a product that norms its own rows forms (SK_RMS, SK_LAYER), or SK_ROWS: A is read.  BIASED: g.act reads a number a feature.
 enum : int { SK_ROWS = 0, SK_RMS = 1, SK_LAYER = 2 };
-template <int KS, int MT, int EPI, typename TC, bool GROUPED, int SK_UNROLL, int NORM, bool BIASED>
-__global__ void __launch_bounds__(64 * KS) gemm_skinny_kernel(SkinnyArgs g) {
+template <int KS, int MT, int EPI, typename TC, bool GROUPED, int NORM, bool BIASED>
+__global__ void __launch_bounds__(64 * KS, MT == 1 ? (NORM == SK_LAYER ? 1 : 4) : 1) gemm_skinny_kernel(SkinnyArgs g) {
     constexpr int NACC = (EPI == SK_SWIGLU) ? 2 : 1;
     constexpr bool NORMED = NORM != SK_ROWS;
-    __shared__ float red[KS > 1 ? KS : 1][MT * NACC][256];
-    __shared__ int rows_a[MT * 16];
-    __shared__ int rows_c[MT * 16];
+    __shared__ __attribute__((aligned(16))) float red[KS > 1 ? KS : 1][MT * NACC][256];
     __shared__ float norm_scratch[32];
     extern __shared__ __attribute__((aligned(16))) bf16_t normed_rows[];   // NORMED: [x_rows][K]
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, kg = lane >> 4;
     const int n0 = blockIdx.x * 16;
     const ActParams act_params(EPI == SK_STORE && !BIASED ? g.act : LLMX_ACT_NONE, g.act_params);
     const bf16_t* W = g.W;
     int row_begin = 0, row_end = g.M;
     if (GROUPED) {
-        if ((int)blockIdx.y >= *g.n_active) return;
-        const int e = g.active[blockIdx.y];
+        const int e = g.active[blockIdx.y], groups = *g.n_active;     // asked for together; beyond the groups that have rows the first means nothing
+        if ((int)blockIdx.y >= groups) return;
         row_begin = g.group_offsets[e];
         row_end = g.group_offsets[e + 1];
         W += (size_t)e * g.w_group_stride;
@@ -82,64 +115,66 @@ __global__ void __launch_bounds__(64 * KS) gemm_skinny_kernel(SkinnyArgs g) {
     const int K = g.K;
     const int steps_total = (K + 31) >> 5;
     const int per = (steps_total + KS - 1) / KS;
-    const int s_begin = wave * per;
-    const int s_end = min(steps_total, s_begin + per);
-    const int w_row = min(n0 + r, g.N - 1);
-    const bf16_t* wp = W + (size_t)w_row * K + kg * 8;
-    const bf16_t* up = (EPI == SK_SWIGLU) ? wp + (size_t)g.up_offset * K : wp;
+    const int s_begin = min(steps_total, wave * per), s_end = min(steps_total, s_begin + per);
+    const int pairs = max(min(s_end, K >> 5) - s_begin, 0) >> 1;      // the wave's pairs of whole steps
+    const int line_step = r >> 3;
+    const bf16_t* wp = W + (size_t)n0 * K;
+    const uint32_t strip_bytes = 2u * (uint32_t)min(16, g.N - n0) * K, w_at = 2u * ((uint32_t)(r & 7) * K + 8 * kg + 32 * line_step), w_next = 16u * K;
+    const strip_t w_strip = strip_of(wp, strip_bytes), u_strip = strip_of(wp + (EPI == SK_SWIGLU ? (size_t)g.up_offset * K : 0), strip_bytes);
+    const bool lines = K % 64 == 0 && per % 2 == 0;     // a pair of steps is a line of each row
 
-    // A wave's share of K is fetched in rounds of SK_UNROLL steps.  With one tile of rows the rounds take turns in two
-    // sets of registers: the next round is asked for before the present one is multiplied, so the wave waits for memory
-    // once, not once a round; and a round's weights are asked for before anything else the workgroup reads (the rows'
-    // list, the old values an adding epilogue joins), since their addresses depend on nothing but the strip.
-    constexpr bool PIPELINED = MT == 1 && EPI != SK_SWIGLU;   // the SwiGLU form streams two strips: a second set of registers costs it a wave a SIMD (measured slower)
+    // A wave's pairs are fetched in rounds of RP, which take turns in two sets of registers: the next round is asked for before the present
+    // one is multiplied.  No load sits behind a condition (a row the tile does not have is another one whose column is not stored), so that
+    // waiting for one round leaves the next on its way.  Loads arrive in the order they were asked for: what the first multiplication waits
+    // for beside its weights (the rows' list, the rows that a norm reads) goes ahead of them, everything else comes after.
+    constexpr int RP = MT == 1 && EPI != SK_SWIGLU ? 2 : 1;
+    const int rounds = pairs / RP;
+    const bool odd = RP == 2 && pairs % 2 != 0;      // a pair after the last round
     struct Round {
-        bf16x8_t wf[SK_UNROLL], uf[SK_UNROLL], af[SK_UNROLL][MT];
+        WeightLines wl[RP], ul[EPI == SK_SWIGLU ? RP : 1];
+        bf16x8_t af[RP][2][MT];
     };
-    auto fetch_weights = [&](int s, Round& f) {
+    Round r0, r1;
+    auto fetch_weights = [&](auto as_lines, int round, Round& f, int n = 2) {
+        constexpr bool L = decltype(as_lines)::value;
 #pragma unroll
-        for (int u = 0; u < SK_UNROLL; ++u) {
-            const int k = (s + u) * 32 + kg * 8;
-            const bool in = (s + u) < s_end && k < K;
-            f.wf[u] = load_frag(wp + (size_t)(s + u) * 32, in);
-            if (EPI == SK_SWIGLU) f.uf[u] = load_frag(up + (size_t)(s + u) * 32, in);
+        for (int u = 0; u < RP && u < n; ++u) {
+            const uint32_t at = pairs > 0 ? 64u * (s_begin + 2 * (RP * round + u)) : 0u;
+            f.wl[u] = WeightLines{load_line<L>(w_strip, w_at, at), load_line<L>(w_strip, w_at + w_next, at)};
+            if (EPI == SK_SWIGLU) f.ul[u] = WeightLines{load_line<L>(u_strip, w_at, at), load_line<L>(u_strip, w_at + w_next, at)};
         }
     };
-
-    bool rows_normed = false;
-    for (int m0 = row_begin; m0 < row_end; m0 += 16 * MT) {
-        Round r0, r1;
-        if (PIPELINED) fetch_weights(s_begin, r0);
-        if (NORMED && !rows_normed) {
-            // the step's rows, normed and rounded as the norm kernel stores them, while the first weights travel
-            auto keep = [&](int row, int i, float y) { normed_rows[(size_t)row * K + i] = f32_to_bf16(y); };
-            if (NORM == SK_LAYER) layer_norm_rows_as_256<KS>(g.X, (size_t)K, g.x_rows, K, g.norm_w, g.norm_bias, g.norm_eps, norm_scratch, keep);
-            else rms_rows_as_1024<KS>(g.X, (size_t)K, g.x_rows, K, g.norm_w, g.norm_eps, norm_scratch, keep);
-            rows_normed = true;   // the barrier below stands between these stores and the first read
-        }
-        if (tid < MT * 16) {
-            const int m = m0 + tid;
-            int ra = -1, rc = -1;
-            if (m < row_end) {
-                if (GROUPED) {
-                    const int p = g.list[m];
-                    ra = p / g.a_div;
-                    rc = p;
-                } else {
-                    ra = rc = m;
-                }
-            }
-            rows_a[tid] = ra;
-            rows_c[tid] = rc;
-        }
-        __syncthreads();
-        const bf16_t* ap[MT];
-        bool a_in[MT];
+    int pair[MT];        // the row of C (and of A, times a_div) of the lane's column
+    auto ask_pairs = [&](int m0) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            const int ra = rows_a[t * 16 + r];
-            a_in[t] = ra >= 0;
-            ap[t] = (NORMED ? normed_rows : g.A) + (size_t)(ra >= 0 ? ra : 0) * (NORMED ? K : g.lda) + kg * 8;
+            const int m = min(m0 + 16 * t + r, row_end - 1);
+            pair[t] = GROUPED ? g.list[m] : m;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (row_begin >= row_end) return;
+    ask_pairs(row_begin);
+    if (NORMED) {
+        // the step's rows, normed and rounded as the norm kernel stores them, while the first weights travel
+        auto keep = [&](int row, int i, float y) { normed_rows[(size_t)row * K + i] = f32_to_bf16(y); };
+        auto ask = [&]() {
+            if (lines) fetch_weights(std::true_type{}, 0, r0);
+            else fetch_weights(std::false_type{}, 0, r0);
+        };
+        if (NORM == SK_LAYER) layer_norm_rows_as_256<KS>(g.X, (size_t)K, g.x_rows, K, g.norm_w, g.norm_bias, g.norm_eps, norm_scratch, keep, ask);
+        else rms_rows_as_1024<KS>(g.X, (size_t)K, g.x_rows, K, g.norm_w, g.norm_eps, norm_scratch, keep, ask);
+        __syncthreads();
+    }
+    auto all_rows = [&](auto as_lines) {
+    for (int m0 = row_begin; m0 < row_end; m0 += 16 * MT) {
+        if (!NORMED || m0 > row_begin) fetch_weights(as_lines, 0, r0);      // also where the wave has no round: it is not multiplied
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16_t* ap[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const int row = GROUPED ? pair[t] / g.a_div : pair[t];
+            ap[t] = (NORMED ? normed_rows : g.A) + (size_t)row * (NORMED ? K : g.lda) + kg * 8 + s_begin * 32;
         }
         f32x4_t acc[MT][NACC];
 #pragma unroll
@@ -155,56 +190,93 @@ __global__ void __launch_bounds__(64 * KS) gemm_skinny_kernel(SkinnyArgs g) {
         if (EPI == SK_ADD && wave == 0) {
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                const int rc = rows_c[t * 16 + r];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const bool in = rc >= 0 && n0 + 4 * kg + i < g.N;
-                    c_old[t][i] = in ? ld((const TC*)g.C + (size_t)rc * g.ldc + n0 + 4 * kg + i) : 0.0f;
-                }
+                for (int i = 0; i < 4; ++i) c_old[t][i] = ld((const TC*)g.C + (size_t)pair[t] * g.ldc + min(n0 + 4 * kg + i, g.N - 1));
             }
         }
-        auto fetch_rows = [&](int s, Round& f) {
+        auto row_frag = [&](int round, int u, int v, int t) { return load_frag(ap[t] + 64 * (RP * round + u) + 32 * v, true); };
+        auto fetch_rows = [&](int round, Round& f, int n = 2) {
+            if (NORMED) return;      // they are in LDS
 #pragma unroll
-            for (int u = 0; u < SK_UNROLL; ++u) {
-                const int k = (s + u) * 32 + kg * 8;
-                const bool in = (s + u) < s_end && k < K;
+            for (int u = 0; u < RP && u < n; ++u)
 #pragma unroll
-                for (int t = 0; t < MT; ++t) f.af[u][t] = load_frag(ap[t] + (size_t)(s + u) * 32, in && a_in[t]);
+                for (int v = 0; v < 2; ++v)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) f.af[u][v][t] = row_frag(round, u, v, t);
+        };
+        auto multiply_step = [&](const bf16x8_t& w, const bf16x8_t& u, const bf16x8_t (&a)[MT]) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a[t], acc[t][0], 0, 0, 0);
+                if (EPI == SK_SWIGLU) acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u, a[t], acc[t][1], 0, 0, 0);
             }
         };
-        auto multiply = [&](const Round& f) {
+        auto multiply = [&](int round, Round& f, int n = 2) {
 #pragma unroll
-            for (int u = 0; u < SK_UNROLL; ++u) {
+            for (int u = 0; u < RP && u < n; ++u) {
+                if (NORMED) {
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.wf[u], f.af[u][t], acc[t][0], 0, 0, 0);
-                    if (EPI == SK_SWIGLU) acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.uf[u], f.af[u][t], acc[t][1], 0, 0, 0);
+                    for (int v = 0; v < 2; ++v)
+#pragma unroll
+                        for (int t = 0; t < MT; ++t) f.af[u][v][t] = row_frag(round, u, v, t);
                 }
+                bf16x8_t w[2], v[2];
+                two_steps(f.wl[u], w);
+                if (EPI == SK_SWIGLU) two_steps(f.ul[u], v);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) multiply_step(w[i], EPI == SK_SWIGLU ? v[i] : w[i], f.af[u][i]);
             }
         };
-        if (PIPELINED) {
-            fetch_rows(s_begin, r0);
-            for (int s = s_begin; s < s_end; s += 2 * SK_UNROLL) {
-                const bool second = s + SK_UNROLL < s_end;     // the same for the whole wave
-                if (second) {
-                    fetch_weights(s + SK_UNROLL, r1);
-                    fetch_rows(s + SK_UNROLL, r1);
-                }
-                multiply(r0);
-                if (second) {
-                    if (s + 2 * SK_UNROLL < s_end) {
-                        fetch_weights(s + 2 * SK_UNROLL, r0);
-                        fetch_rows(s + 2 * SK_UNROLL, r0);
-                    }
-                    multiply(r1);
-                }
+        if (rounds > 0) {
+            fetch_rows(0, r0);
+            int i = 0;
+            for (; i + 2 < rounds; i += 2) {
+                fetch_weights(as_lines, i + 1, r1);
+                fetch_rows(i + 1, r1);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(i, r0);
+                __builtin_amdgcn_sched_barrier(0);
+                fetch_weights(as_lines, i + 2, r0);
+                fetch_rows(i + 2, r0);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(i + 1, r1);
+                __builtin_amdgcn_sched_barrier(0);
             }
-        } else {
-            for (int s = s_begin; s < s_end; s += SK_UNROLL) {
-                fetch_weights(s, r0);
-                fetch_rows(s, r0);
-                multiply(r0);
+            if (i + 1 < rounds) {
+                fetch_weights(as_lines, i + 1, r1);
+                fetch_rows(i + 1, r1);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(i, r0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (odd) {
+                    fetch_weights(as_lines, rounds, r0, 1);
+                    fetch_rows(rounds, r0, 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(i + 1, r1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (odd) multiply(rounds, r0, 1);
+            } else {
+                if (odd) {
+                    fetch_weights(as_lines, rounds, r1, 1);
+                    fetch_rows(rounds, r1, 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(i, r0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (odd) multiply(rounds, r1, 1);
             }
+        } else if (odd) {
+            fetch_rows(0, r0, 1);
+            multiply(0, r0, 1);
+        }
+        for (int s = s_begin + 2 * pairs; s < s_end; ++s) {      // an odd step, K's last one of fewer than 32 values
+            const bool in = s * 32 + kg * 8 < K;
+            const bf16_t* row = W + (size_t)min(n0 + r, g.N - 1) * K + s * 32 + kg * 8;
+            bf16x8_t a[MT];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) a[t] = load_frag(ap[t] + (s - s_begin) * 32, in);
+            multiply_step(load_frag(row, in), load_frag(EPI == SK_SWIGLU ? row + (size_t)g.up_offset * K : row, in), a);
         }
         // partial sums of the waves, added in wave order
         if (KS > 1) {
@@ -231,10 +303,9 @@ __global__ void __launch_bounds__(64 * KS) gemm_skinny_kernel(SkinnyArgs g) {
                     }
                 }
                 // lane: row (tile t, column r), features n0 + 4*kg + 0..3
-                const int rc = rows_c[t * 16 + r];
-                if (rc < 0) continue;
-                TC* c = (TC*)g.C + (size_t)rc * g.ldc + n0 + 4 * kg;
-                const GluRow glu(g.glu, EPI == SK_SWIGLU ? rc : 0);
+                if (m0 + 16 * t + r >= row_end) continue;
+                TC* c = (TC*)g.C + (size_t)pair[t] * g.ldc + n0 + 4 * kg;
+                const GluRow glu(g.glu, EPI == SK_SWIGLU ? pair[t] : 0);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if (n0 + 4 * kg + i >= g.N) continue;
@@ -248,7 +319,16 @@ __global__ void __launch_bounds__(64 * KS) gemm_skinny_kernel(SkinnyArgs g) {
             }
         }
         __syncthreads();
+        if (m0 + 16 * MT < row_end) ask_pairs(m0 + 16 * MT);
     }
+    };
+    if constexpr (MT == 1) {
+        if (lines) {
+            all_rows(std::true_type{});
+            return;
+        }
+    }
+    all_rows(std::false_type{});
 }
 
 // Dense products of 17 to 64 rows: two strips of 16 features a workgroup.  With several tiles of rows a step fetches
@@ -346,8 +426,6 @@ __global__ void __launch_bounds__(64 * KS) gemm_skinny_two_strips_kernel(SkinnyA
     }
 }
 
-// steps of K in a round of loads: with one tile of rows two rounds are in flight (see the kernel)
-#define SKINNY_ROUND(MT, EPI) 4
 #define SKINNY_TWO_STRIPS_MIN_WORKGROUPS 192
 
 // Returns -2 (and launches nothing) for a combination that has no kernel: normed rows with several tiles of rows or
@@ -360,9 +438,9 @@ static int launch_dense(const SkinnyArgs& g, dim3 grid, hipStream_t stream) {
             const size_t lds = (size_t)g.x_rows * g.K * sizeof(bf16_t);
             llmx_note_launch(LK_GEMM_SKINNY_NORMED);
             if (g.norm_bias)
-                hipLaunchKernelGGL((gemm_skinny_kernel<KS, 1, EPI, TC, false, SKINNY_ROUND(MT, EPI), SK_LAYER, BIASED>), grid, dim3(64 * KS), lds, stream, g);
+                hipLaunchKernelGGL((gemm_skinny_kernel<KS, 1, EPI, TC, false, SK_LAYER, BIASED>), grid, dim3(64 * KS), lds, stream, g);
             else
-                hipLaunchKernelGGL((gemm_skinny_kernel<KS, 1, EPI, TC, false, SKINNY_ROUND(MT, EPI), SK_RMS, BIASED>), grid, dim3(64 * KS), lds, stream, g);
+                hipLaunchKernelGGL((gemm_skinny_kernel<KS, 1, EPI, TC, false, SK_RMS, BIASED>), grid, dim3(64 * KS), lds, stream, g);
             return 0;
         }
         return -2;
@@ -376,7 +454,7 @@ static int launch_dense(const SkinnyArgs& g, dim3 grid, hipStream_t stream) {
         }
     }
     llmx_note_launch(LK_GEMM_SKINNY);
-    hipLaunchKernelGGL((gemm_skinny_kernel<KS, MT, EPI, TC, false, SKINNY_ROUND(MT, EPI), SK_ROWS, BIASED>), grid, dim3(64 * KS), 0, stream, g);
+    hipLaunchKernelGGL((gemm_skinny_kernel<KS, MT, EPI, TC, false, SK_ROWS, BIASED>), grid, dim3(64 * KS), 0, stream, g);
     return 0;
 }
 
@@ -393,13 +471,13 @@ static int launch_grouped(const SkinnyArgs& g, dim3 grid, bool grouped, hipStrea
         if constexpr (MT == 1 && EPI != SK_ADD) {
             const size_t lds = (size_t)g.x_rows * g.K * sizeof(bf16_t);
             llmx_note_launch(LK_GEMM_SKINNY_GROUPED_NORMED);
-            hipLaunchKernelGGL((gemm_skinny_kernel<KS, 1, EPI, TC, true, SKINNY_ROUND(MT, EPI), SK_RMS, false>), grid, dim3(64 * KS), lds, stream, g);
+            hipLaunchKernelGGL((gemm_skinny_kernel<KS, 1, EPI, TC, true, SK_RMS, false>), grid, dim3(64 * KS), lds, stream, g);
             return 0;
         }
         return -2;
     }
     llmx_note_launch(LK_GEMM_SKINNY_GROUPED);
-    hipLaunchKernelGGL((gemm_skinny_kernel<KS, MT, EPI, TC, true, SKINNY_ROUND(MT, EPI), SK_ROWS, false>), grid, dim3(64 * KS), 0, stream, g);
+    hipLaunchKernelGGL((gemm_skinny_kernel<KS, MT, EPI, TC, true, SK_ROWS, false>), grid, dim3(64 * KS), 0, stream, g);
     return 0;
 }
 
