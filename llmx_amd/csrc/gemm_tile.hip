@@ -57,6 +57,11 @@ __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, v
     const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
 }
+// The same for bytes that are read once: the caches are told not to keep them.
+__device__ __forceinline__ void stream_to_lds(const void* base, uint32_t offset, void* lds) {
+    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
+}
 
 // Four neighbouring features of one output row (n a multiple of 4): one 16-byte (float) or 8-byte (bfloat16) access
 // when the row allows it, element by element at a ragged edge.  ADD: the values join what the row holds.
@@ -208,6 +213,7 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
                 tile_info[0] = e;
                 tile_info[1] = begin + (row_tile - first) * BM;
                 tile_info[2] = end;
+                tile_info[3] = tiles;
             }
             base += round_total;
             __syncthreads();
@@ -351,13 +357,23 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
             a_at[j] = (uint32_t)(((size_t)(ra >= 0 ? ra : 0) * g.lda + 8 * ch) * sizeof(bf16_t));
         }
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+        // a tile of few rows, weights that no other row tile reads: see the wide form
+        const bool read_once = __builtin_amdgcn_readfirstlane(GROUPED ? tile_info[3] : g.m_tiles) == 1;
+        const int rows_here = row_end - row_begin;
+        const bool brings_rows = (BM / 4) * wave_u < rows_here, works = BM / 2 * __builtin_amdgcn_readfirstlane(wm) < rows_here;
         auto issue = [&](int t, int stage) {
             const bf16_t* wb = W + (size_t)t * TL_BK;
             const bf16_t* ab = g.A + (size_t)t * TL_BK;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) load_to_lds(wb, w_at[j], &Ws[(stage * TL_BN + 32 * wave_u + 8 * j) * TL_BK]);
+            for (int j = 0; j < 4; ++j) {
+                void* to = &Ws[(stage * TL_BN + 32 * wave_u + 8 * j) * TL_BK];
+                if (read_once) stream_to_lds(wb, w_at[j], to);
+                else load_to_lds(wb, w_at[j], to);
+            }
+            if (STAGES > 2 || brings_rows) {
 #pragma unroll
-            for (int j = 0; j < A_LOADS; ++j) load_to_lds(ab, a_at[j], &As[(stage * BM + (BM / 4) * wave_u + 8 * j) * TL_BK]);
+                for (int j = 0; j < A_LOADS; ++j) load_to_lds(ab, a_at[j], &As[(stage * BM + (BM / 4) * wave_u + 8 * j) * TL_BK]);
+            }
         };
         // operand reads: row `row` of a stage, chunk kk/8 + lane/16
         int w_rd[4], a_rd[TT], w_swz[4], a_swz[TT];
@@ -418,7 +434,7 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
                 else __builtin_amdgcn_s_waitcnt(0x0F70);
                 __syncthreads();
                 if (t + STAGES - 1 < n_tiles) issue(t + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
-                multiply(stage);
+                if (works) multiply(stage);
                 stage = stage == STAGES - 1 ? 0 : stage + 1;
             }
             if (t >= n_tiles) break;
@@ -587,6 +603,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
                 tile_info[0] = e;
                 tile_info[1] = begin + (row_tile - first) * WD_BM;
                 tile_info[2] = end;
+                tile_info[3] = tiles;
             }
             base += round_total;
             __syncthreads();
@@ -664,13 +681,29 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
         a_at[j] = (uint32_t)(((size_t)(ra >= 0 ? ra : 0) * g.lda + 8 * ch) * sizeof(bf16_t));
     }
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    // A tile of few rows (an expert's last, or its only one) is not multiplied out to 128: a wave whose 16 rows of A lie past the tile's
+    // rows leaves them unread, and with at most 64 rows the waves of the upper half only bring weights.  What LDS holds for such rows makes
+    // columns of the product that are never stored.  Weights that no other row tile reads come as bytes read once, which the caches do not
+    // keep; where several do, the later ones find them in the caches (all as read once: down of 2,048 rows 596 -> 719 us).  Both, gate_up (256
+    // experts or some 60, 3,072 features of 3,072 values): 2,048 rows in 64 an expert 1,037 -> 984 us, in 300 602 -> 535; 37 prompts of 45
+    // 1,050 -> 952; 64-row tiles: 64 rows in 221 experts 669 -> 601 (6.9 TB/s), 520 rows 752 -> 700, down of 64 rows 345 -> 318.
+    const int rows_here = row_end - row_begin;
+    const bool read_once = __builtin_amdgcn_readfirstlane(GROUPED ? tile_info[3] : g.m_tiles) == 1;
+    const bool brings_rows = __builtin_amdgcn_readfirstlane(16 * wave) < rows_here;
+    const bool works = __builtin_amdgcn_readfirstlane(64 * wm) < rows_here;
     auto issue = [&](int t, int stage) {
         const bf16_t* wb = W + (size_t)t * TL_BK;
         const bf16_t* ab = g.A + (size_t)t * TL_BK;
 #pragma unroll
-        for (int j = 0; j < W_LOADS; ++j) load_to_lds(wb, w_at[j], &Ws[(stage * WD_BN + 32 * wave_u + 8 * j) * TL_BK]);
+        for (int j = 0; j < W_LOADS; ++j) {
+            void* to = &Ws[(stage * WD_BN + 32 * wave_u + 8 * j) * TL_BK];
+            if (read_once) stream_to_lds(wb, w_at[j], to);
+            else load_to_lds(wb, w_at[j], to);
+        }
+        if (brings_rows) {
 #pragma unroll
-        for (int j = 0; j < A_LOADS; ++j) load_to_lds(ab, a_at[j], &As[(stage * WD_BM + 16 * wave_u + 8 * j) * TL_BK]);
+            for (int j = 0; j < A_LOADS; ++j) load_to_lds(ab, a_at[j], &As[(stage * WD_BM + 16 * wave_u + 8 * j) * TL_BK]);
+        }
     };
     int w_rd[4], a_rd[TT], w_swz[4], a_swz[TT];
 #pragma unroll
@@ -709,17 +742,33 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
     issue(0, 0);
     if (1 < n_tiles) issue(1, 1);
     if (2 < n_tiles) issue(2, 2);
-    {
-        const int out = (n_tiles > 2 ? 2 : n_tiles - 1) * LOADS;   // loads of the tiles after the first that may still be out
-        if (out == 2 * LOADS) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * LOADS));
-        else if (out == LOADS) __builtin_amdgcn_s_waitcnt(0x0F70 | LOADS);
-        else __builtin_amdgcn_s_waitcnt(0x0F70);
-    }
+    // until at most the loads of `out` tiles are on their way (LDS reads awaited too where the wave makes any)
+    auto wait_loads = [&](int out) {
+        if (out == 2) {
+            if (brings_rows) __builtin_amdgcn_s_waitcnt(0x0070 | (2 * LOADS));
+            else __builtin_amdgcn_s_waitcnt(0x0070 | (2 * W_LOADS));
+        } else if (out == 1) {
+            if (brings_rows) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);
+            else __builtin_amdgcn_s_waitcnt(0x0070 | W_LOADS);
+        } else {
+            __builtin_amdgcn_s_waitcnt(0x0070);
+        }
+    };
+    wait_loads(min(2, n_tiles - 1));
     __syncthreads();
+    const int last = n_tiles - 1;   // the last tile has no tile after it: it runs after the loop, so the loop's body has no branch around its reads
+    if (!works) {
+        for (int t = 0, stage = 0; t < last; ++t) {
+            wait_loads(t + 2 < n_tiles ? 1 : 0);
+            __syncthreads();
+            if (t + 3 < n_tiles) issue(t + 3, stage);
+            stage = stage == 2 ? 0 : stage + 1;
+        }
+        return;
+    }
     bf16x8_t wf_a[4], af_a[TT], wf_b[4], af_b[TT];
     read_half(0, 0, wf_a, af_a);
     int t = 0, stage = 0;
-    const int last = n_tiles - 1;   // the last tile has no tile after it: it runs after the loop, so the loop's body has no branch around its reads
     for (int run_end = tiles_per_run;; run_end += tiles_per_run) {
         const int stop = min(run_end, last);
         for (; t < stop; ++t) {
@@ -728,8 +777,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
             WD_INTERLEAVE();
             const int next = stage == 2 ? 0 : stage + 1;
             // this wave's operand reads of tile t are done, and its part of tile t+1 has arrived (tile t+2's may be out)
-            if (t + 2 < n_tiles) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);
-            else __builtin_amdgcn_s_waitcnt(0x0070);
+            wait_loads(t + 2 < n_tiles ? 1 : 0);
             __syncthreads();
             if (t + 3 < n_tiles) issue(t + 3, stage);
             read_half(next, 0, wf_a, af_a);
