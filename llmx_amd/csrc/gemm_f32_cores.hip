@@ -6,13 +6,15 @@
 // row's bits depend on its own values and the weights only, not on the rows beside it or on the form.
 //
 //  * stream: few rows.  The weights' way from memory bounds it: a workgroup's `ks` waves share a strip of 16 features, one run of
-//    K each, and ask for a round of steps while the round before is multiplied.  1 row: 32,768 features of 2,048 values 56 us (4.8
-//    TB/s), 8,192 of 3,072 22 us, 3,072 of 2,048 12.8 us; the universal product takes 0.2-0.5 ms for the smallest of these.
+//    K each, and ask for a round of steps while the round before is multiplied, as whole lines that are read once (weight_lines.h).
+//    4 rows, 8 experts of 2 x 2,688 features of 2,048 values: 44.8 us, 60 with half lines that the caches keep; their 2,048 features of
+//    2,688 values 27.5 (41.8), dense 3,072 of 2,048 9.4 (10.9); the universal product takes 0.2-0.5 ms for the smallest of these.
 //  * tiles: many rows.  The instruction's rate bounds it (140 TFLOP/s measured alone): 64 rows x 128 (64) features a workgroup,
 //    operands staged through LDS 32 values of k at a time, its runs folded in registers.  2,048 rows: 8,192 features
 //    of 3,072 values 0.80 ms (130 TFLOP/s); 333 rows of 2,048 values: 32,768 features 0.44 ms (102 TFLOP/s), where the universal
 //    product reaches 8 TFLOP/s.  Chunks asked for two ahead instead of one: 0.84 -> 0.78 ms and 0.47 -> 0.44 ms.
 #include "gemm_args.h"
+#include "weight_lines.h"
 #include <type_traits>
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -45,9 +47,9 @@ __device__ __forceinline__ void f32_store_quad(const GemmArgs& g, const ActFn& a
 
 // Grid: dense (strips, chunks of 16 MT rows); grouped (strips, groups, row chunks of a group).
 template <int KS, int MT, int EPI>
-__global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
+__global__ void __launch_bounds__(64 * KS, MT == 1 ? 4 : 1) gemm_f32_stream_kernel(GemmArgs g) {
     constexpr int NS = EPI == EPI_SWIGLU ? 2 : 1;                  // weight strips: the features', and the up rows' of the same features
-    constexpr int UN = NS * MT == 1 ? 8 : NS * MT == 2 ? 4 : 2;    // steps of a round: its loads travel together
+    constexpr int UN = NS * MT == 1 ? 4 : 2;    // steps of a round: its loads travel together (a wave has two rounds on their way, a SIMD four waves)
     __shared__ __attribute__((aligned(16))) float red[KS > 1 ? KS : 1][NS * MT][256];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, kg = lane >> 4;
@@ -64,11 +66,17 @@ __global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
     const int steps = (K + 15) >> 4, per = (steps + KS - 1) / KS, ranges = (steps + per - 1) / per;
     const int s_begin = min(steps, wave * per), s_end = min(steps, s_begin + per);
     const int whole_end = min(s_end, K >> 4);                      // steps before this one are whole
-    const float* wp[NS];
+    // the strips' rows in memory, the lane's chunk of a line of two steps
+    const uint32_t pitch = 4u * (uint32_t)g.ldw, w_at = (uint32_t)(r & 7) * pitch + line_chunk(r, kg);
+    strip_t strip[NS];
 #pragma unroll
-    for (int ns = 0; ns < NS; ++ns) wp[ns] = W + (size_t)(min(n0 + r, g.N - 1) + (ns ? g.up_offset : 0)) * g.ldw + kg * 4;
+    for (int ns = 0; ns < NS; ++ns)
+        strip[ns] = strip_of(W + (size_t)(n0 + (ns ? g.up_offset : 0)) * g.ldw, (uint32_t)(min(16, g.N - n0) - 1) * pitch + 4u * (uint32_t)K);
+    const bool lines = g.ldw % 32 == 0 && per % 2 == 0;       // a pair of steps is a line of each row
+    const int n_steps = max(whole_end - s_begin, 0), rounds = (n_steps + UN - 1) / UN;
     const ActFn act(EPI != EPI_SWIGLU ? g.act : LLMX_ACT_NONE, g.act_params);
 
+    auto all_rows = [&](auto as_lines) {
     for (; m0 < row_end; m0 += m_step) {
         // a row past the last reads the last one: what its column of the product gives is never stored
         const float* ap[MT];
@@ -85,17 +93,22 @@ __global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
 #pragma unroll
             for (int t = 0; t < MT; ++t) acc[ns][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         struct Round {
-            f32x4_t w[UN][NS], a[UN][MT];
+            WeightLines w[UN / 2][NS];
+            f32x4_t a[UN][MT];
         };
-        auto fetch = [&](Round& f, int s) {
+        // of a last round that is not full the steps past the end are steps fetched before, and not multiplied
+        auto fetch = [&](Round& f, int round) {
+            const int s = s_begin + UN * round;
 #pragma unroll
-            for (int u = 0; u < UN; ++u) {
-                const size_t at = (size_t)max(min(s + u, whole_end - 1), 0) * 16;      // past the end: a step fetched before, not multiplied
+            for (int u = 0; u < UN; u += 2) {
+                const int pair = min(s + u, whole_end - 1), back = s + u + 1 < whole_end ? 0 : 64 * (r >> 3);
 #pragma unroll
-                for (int ns = 0; ns < NS; ++ns) f.w[u][ns] = *reinterpret_cast<const f32x4_t*>(wp[ns] + at);
-#pragma unroll
-                for (int t = 0; t < MT; ++t) f.a[u][t] = *reinterpret_cast<const f32x4_t*>(ap[t] + at);
+                for (int ns = 0; ns < NS; ++ns) f.w[u / 2][ns] = two_lines<decltype(as_lines)::value>(strip[ns], w_at - back, 8 * pitch, 64u * (uint32_t)pair);
             }
+#pragma unroll
+            for (int u = 0; u < UN; ++u)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) f.a[u][t] = *reinterpret_cast<const f32x4_t*>(ap[t] + (size_t)min(s + u, whole_end - 1) * 16);
         };
         auto multiply = [&](const f32x4_t (&w)[NS], const f32x4_t (&a)[MT]) {
 #pragma unroll
@@ -105,26 +118,50 @@ __global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
 #pragma unroll
                     for (int t = 0; t < MT; ++t) acc[ns][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[ns][i], a[t][i], acc[ns][t], 0, 0, 0);
         };
-        auto round = [&](const Round& f, int s) {
+        auto whole = [&](const Round& f, int n) {      // the round's first n steps
 #pragma unroll
-            for (int u = 0; u < UN; ++u)
-                if (s + u < whole_end) multiply(f.w[u], f.a[u]);
+            for (int u = 0; u < UN; u += 2) {
+                if (u >= n) break;
+                f32x4_t first[NS], second[NS];
+#pragma unroll
+                for (int ns = 0; ns < NS; ++ns) two_steps(f.w[u / 2][ns], first[ns], second[ns]);
+                multiply(first, f.a[u]);
+                if (u + 1 < n) multiply(second, f.a[u + 1]);
+            }
         };
-        if (s_begin < whole_end) {
+        if (rounds > 0) {
+            // rounds take turns in two sets of registers: the next is asked for before the present one is multiplied
             Round first, second;
-            fetch(first, s_begin);
-            for (int s = s_begin; s < whole_end; s += 2 * UN) {
-                fetch(second, s + UN);
-                round(first, s);
-                fetch(first, s + 2 * UN);
-                round(second, s + UN);
+            fetch(first, 0);
+            int i = 0;
+            for (; i + 2 < rounds; i += 2) {
+                fetch(second, i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                whole(first, UN);
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(first, i + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                whole(second, UN);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (i + 1 < rounds) {
+                fetch(second, i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                whole(first, UN);
+                __builtin_amdgcn_sched_barrier(0);
+                whole(second, n_steps - UN * (i + 1));
+            } else {
+                whole(first, n_steps - UN * i);
             }
         }
         if (s_end > whole_end) {       // K's last step holds 4, 8 or 12 values
             const bool in = whole_end * 16 + 4 * kg < K;
             f32x4_t w[NS], a[MT];
 #pragma unroll
-            for (int ns = 0; ns < NS; ++ns) w[ns] = in ? *reinterpret_cast<const f32x4_t*>(wp[ns] + (size_t)whole_end * 16) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int ns = 0; ns < NS; ++ns) {
+                const float* row = W + (size_t)(min(n0 + r, g.N - 1) + (ns ? g.up_offset : 0)) * g.ldw + kg * 4;
+                w[ns] = in ? *reinterpret_cast<const f32x4_t*>(row + (size_t)whole_end * 16) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
 #pragma unroll
             for (int t = 0; t < MT; ++t) a[t] = in ? *reinterpret_cast<const f32x4_t*>(ap[t] + (size_t)whole_end * 16) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
             multiply(w, a);
@@ -156,6 +193,14 @@ __global__ void __launch_bounds__(64 * KS) gemm_f32_stream_kernel(GemmArgs g) {
         }
         if (KS > 1) __syncthreads();
     }
+    };
+    if constexpr (MT == 1) {
+        if (lines) {
+            all_rows(std::true_type{});
+            return;
+        }
+    }
+    all_rows(std::false_type{});
 }
 
 // K a multiple of 16.  A workgroup takes 64 rows and BN weight rows (gated: BN / 2 features' gate and up rows); grid (feature tiles,

@@ -21,6 +21,7 @@
 // instead of A; every workgroup forms the normed, rounded rows itself (in LDS) while its first weights travel, and no
 // norm kernel is launched.  The rows' values are the norm kernel's, bit for bit.  With a bias the norm is a layer norm.
 #include "common.h"
+#include "weight_lines.h"
 #include <type_traits>
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -61,34 +62,6 @@ __device__ __forceinline__ bf16x8_t load_frag(const bf16_t* p, bool in) {
     return __builtin_bit_cast(bf16x8_t, v);
 }
 
-// Two steps of a strip's weights (16 rows of 32 k, twice).  Memory gives and the caches keep lines of 128 bytes, so the loads are whole
-// lines, eight rows' each, and the halves that belong to another lane are exchanged between lanes 8 apart in a row of 16: lane (r, kg) asks
-// for chunk kg + 4 (r / 8) (of 8 of 16 bytes) of rows r % 8 and 8 + r % 8.  Whole lines can be asked for as bytes that are read once
-// (LINES), which the caches then do not keep: a kernel that only reads gets 7.1 TB/s that way and 6.3 without, and what the step's other
-// kernels read stays near; half lines asked for so arrive twice (5.6 TB/s).
-struct WeightLines {
-    u32x4_t lo, hi;
-};
-// A strip's rows as the loads see them: 32-bit byte offsets from a base the wave shares; what lies past the strip's last row reads as 0.
-typedef __amdgpu_buffer_rsrc_t strip_t;
-__device__ __forceinline__ strip_t strip_of(const bf16_t* base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00027000);
-}
-template <bool LINES>
-__device__ __forceinline__ u32x4_t load_line(strip_t strip, uint32_t lane_byte, uint32_t wave_byte) {
-    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(strip, (int)lane_byte, (int)wave_byte, LINES ? 2 : 0));
-}
-__device__ __forceinline__ void two_steps(const WeightLines& l, bf16x8_t (&step)[2]) {
-    u32x4_t a, b;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        a[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)l.lo[i], (int)l.hi[i], 0x128, 0xf, 0xc, false);
-        b[i] = (uint32_t)__builtin_amdgcn_update_dpp((int)l.hi[i], (int)l.lo[i], 0x128, 0xf, 0x3, false);
-    }
-    step[0] = __builtin_bit_cast(bf16x8_t, a);
-    step[1] = __builtin_bit_cast(bf16x8_t, b);
-}
-
 // NORM: what a product that norms its own rows forms (SK_RMS, SK_LAYER), or SK_ROWS: A is read.  BIASED: g.act reads a number a feature.
 enum : int { SK_ROWS = 0, SK_RMS = 1, SK_LAYER = 2 };
 template <int KS, int MT, int EPI, typename TC, bool GROUPED, int NORM, bool BIASED>
@@ -117,9 +90,8 @@ __global__ void __launch_bounds__(64 * KS, MT == 1 ? (NORM == SK_LAYER ? 1 : 4) 
     const int per = (steps_total + KS - 1) / KS;
     const int s_begin = min(steps_total, wave * per), s_end = min(steps_total, s_begin + per);
     const int pairs = max(min(s_end, K >> 5) - s_begin, 0) >> 1;      // the wave's pairs of whole steps
-    const int line_step = r >> 3;
     const bf16_t* wp = W + (size_t)n0 * K;
-    const uint32_t strip_bytes = 2u * (uint32_t)min(16, g.N - n0) * K, w_at = 2u * ((uint32_t)(r & 7) * K + 8 * kg + 32 * line_step), w_next = 16u * K;
+    const uint32_t strip_bytes = 2u * (uint32_t)min(16, g.N - n0) * K, w_at = 2u * (uint32_t)(r & 7) * K + line_chunk(r, kg), w_next = 16u * K;
     const strip_t w_strip = strip_of(wp, strip_bytes), u_strip = strip_of(wp + (EPI == SK_SWIGLU ? (size_t)g.up_offset * K : 0), strip_bytes);
     const bool lines = K % 64 == 0 && per % 2 == 0;     // a pair of steps is a line of each row
 
@@ -140,8 +112,8 @@ __global__ void __launch_bounds__(64 * KS, MT == 1 ? (NORM == SK_LAYER ? 1 : 4) 
 #pragma unroll
         for (int u = 0; u < RP && u < n; ++u) {
             const uint32_t at = pairs > 0 ? 64u * (s_begin + 2 * (RP * round + u)) : 0u;
-            f.wl[u] = WeightLines{load_line<L>(w_strip, w_at, at), load_line<L>(w_strip, w_at + w_next, at)};
-            if (EPI == SK_SWIGLU) f.ul[u] = WeightLines{load_line<L>(u_strip, w_at, at), load_line<L>(u_strip, w_at + w_next, at)};
+            f.wl[u] = two_lines<L>(w_strip, w_at, w_next, at);
+            if (EPI == SK_SWIGLU) f.ul[u] = two_lines<L>(u_strip, w_at, w_next, at);
         }
     };
     int pair[MT];        // the row of C (and of A, times a_div) of the lane's column
@@ -221,8 +193,8 @@ __global__ void __launch_bounds__(64 * KS, MT == 1 ? (NORM == SK_LAYER ? 1 : 4) 
                         for (int t = 0; t < MT; ++t) f.af[u][v][t] = row_frag(round, u, v, t);
                 }
                 bf16x8_t w[2], v[2];
-                two_steps(f.wl[u], w);
-                if (EPI == SK_SWIGLU) two_steps(f.ul[u], v);
+                two_steps(f.wl[u], w[0], w[1]);
+                if (EPI == SK_SWIGLU) two_steps(f.ul[u], v[0], v[1]);
 #pragma unroll
                 for (int i = 0; i < 2; ++i) multiply_step(w[i], EPI == SK_SWIGLU ? v[i] : w[i], f.af[u][i]);
             }

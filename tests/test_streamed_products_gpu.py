@@ -81,3 +81,18 @@ def test_grouped_rows_are_the_dense_ones(N, K):
             ops.gemm(a[rows].contiguous(), w[g].contiguous(), dense)
             close(dense, a[rows].double() @ w[g].double().T, K)
             assert torch.equal(c[rows], dense)
+
+
+# waves with no round, part of one, one and more, lines that are whole and not, strips that end early
+@pytest.mark.parametrize("N,K", [(16, 16), (40, 32), (17, 64), (130, 96), (48, 160), (264, 288), (100, 672), (2050, 1344), (4100, 2688)])
+@pytest.mark.parametrize("M", [1, 4, 16])
+def test_float32_rows_have_the_bits_the_tiles_give(M, N, K):
+    from llmx_amd import ops
+    a, w = rnd(80, K, dtype=torch.float32), rnd(N, K, seed=1, dtype=torch.float32)
+    many, c = torch.empty(80, N, device=DEV), torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm(a, w, many)
+    ops.take_launches()
+    ops.gemm(a[:M].contiguous(), w, c)
+    assert ops.take_launches() == {"gemm_generic": 1, "gemm_generic.stream": 1}
+    close(c, a[:M].double() @ w.double().T, K)
+    assert torch.equal(c, many[:M])
