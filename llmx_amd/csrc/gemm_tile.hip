@@ -114,6 +114,7 @@ struct TileArgs {
     int act;                // TL_STORE, TL_ADD: an activation applied to the product (LLMX_ACT_*; a launch of runs' sums leaves it to the kernel that adds them)
     const float* act_params;
     GluArgs glu;            // TL_SWIGLU: the gated unit and its per-row values
+    int* ticket;            // grouped wide form, optional: 0, and 0 again afterwards; workgroups take tile after tile by it
 };
 
 // Whether this launch is the one that works: the grouping's own choice says which tiles the product takes; for a caller
@@ -133,15 +134,15 @@ __device__ __forceinline__ bool tile_launch_runs(const TileArgs& g) {
 // takes a contiguous run of tiles in the order strip after strip instead, a strip's row tiles together, and reads the rows' whole
 // activations for every strip.
 #define TILE_XCDS 8
+#define TILE_CUS 256
 template <bool GROUPED>
-__device__ __forceinline__ void tile_place(const TileArgs& g, int& strip, int& rows) {
-    const int gx = gridDim.x, gy = gridDim.y;
+__device__ __forceinline__ void tile_place(const TileArgs& g, int at, int gx, int gy, int& strip, int& rows) {
     if (GROUPED || !g.strip_runs) {
-        strip = blockIdx.x;
-        rows = blockIdx.y;
+        rows = at / gx;
+        strip = at - rows * gx;
         return;
     }
-    const int total = gx * gy, at = (int)blockIdx.y * gx + (int)blockIdx.x;
+    const int total = gx * gy;
     const int xcd = at % TILE_XCDS, share = total / TILE_XCDS, more = total % TILE_XCDS;
     const int tile = xcd * share + min(xcd, more) + at / TILE_XCDS;
     strip = tile / gy;
@@ -182,7 +183,12 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
     const bool runs = !GROUPED || tile_launch_runs(g);   // looked at below, once the first offsets are asked for too
     constexpr int FEATS = (EPI == TL_SWIGLU) ? 64 : 128;  // output features a workgroup covers
     int strip, row_tile;
-    tile_place<GROUPED>(g, strip, row_tile);
+    if (GROUPED || !g.strip_runs) {
+        strip = blockIdx.x;
+        row_tile = blockIdx.y;
+    } else {
+        tile_place<GROUPED>(g, (int)(blockIdx.y * gridDim.x + blockIdx.x), gridDim.x, gridDim.y, strip, row_tile);
+    }
     const int n0 = strip * FEATS;
     const bf16_t* W = g.W;
     int row_begin, row_end;
@@ -557,27 +563,34 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
             __builtin_amdgcn_sched_group_barrier(0x008, 2, 0); \
         }                                                    \
     } while (0)
-template <int EPI, typename TC, bool GROUPED, bool SPLIT>
+//
+// With one workgroup a CU nothing else works while a tile's place is looked up, its first weights are on their way and its sums are stored.
+// So, for routed products whose caller brings a ticket counter, a workgroup stays on its CU and takes tile after tile: the next one is
+// looked up while this one is multiplied, and its first K tiles are asked for as stages of LDS fall free; only the stores and one wait stand
+// between two tiles.  The tiles are handed out in order by tickets, not in strides: the row tiles of one expert have to stay close in
+// time for its weights to be found in the caches (strides, 256 experts of 300 rows, 3,072 features of 3,072 values: 2,423 -> 2,664 us).
+// A workgroup a tile and tickets, 256 experts: 64 rows an expert 940 -> 864 us, 100 1,038 -> 954, 130 1,427 -> 1,345, 170 1,701 -> 1,654; 55
+// experts of 300 519 -> 526.
+// BARE: nothing is applied to the sums but, gated, silu(gate) * up.  With the other units and activations in the loop over tiles their
+// constants take the registers the sums need; those products launch a workgroup a tile, and dense ones too (nothing gained).
+#define WD_MAX_GROUPS 1536      // groups whose row tiles and places are kept in LDS beside the stages
+template <int EPI, typename TC, bool GROUPED, bool SPLIT, bool BARE>
 __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
     __shared__ __attribute__((aligned(1024))) bf16_t As[WD_STAGES * WD_BM * TL_BK];
     __shared__ __attribute__((aligned(1024))) bf16_t Ws[WD_STAGES * WD_BN * TL_BK];
-    __shared__ int rows_a[WD_BM];
-    __shared__ int rows_c[WD_BM];
-    __shared__ int tile_info[4];
+    __shared__ int tiles_before[GROUPED ? WD_MAX_GROUPS + 1 : 1], places[GROUPED ? WD_MAX_GROUPS + 1 : 1];
+    __shared__ int pairs[3][GROUPED ? WD_BM : 1];        // of the tile before (its sums may still be stored), this one and the next
     __shared__ int scan_waves[8];
+    __shared__ int drawn[2];                             // the next tile and the one after it, taking turns
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const bool runs = !GROUPED || tile_launch_runs(g);   // looked at below, once the first offsets are asked for too
     constexpr int HALF = WD_BN / 2;                               // SwiGLU: gate rows, then the up rows of the same features
-    constexpr int FEATS = (EPI == TL_SWIGLU) ? HALF : WD_BN;      // output features a workgroup covers
-    int strip, row_tile;
-    tile_place<GROUPED>(g, strip, row_tile);
-    const int n0 = strip * FEATS;
-    const bf16_t* W = g.W;
-    int row_begin, row_end;
+    constexpr int FEATS = (EPI == TL_SWIGLU) ? HALF : WD_BN;      // output features a tile covers
+    const int strips = (g.N + FEATS - 1) / FEATS;
+    int row_tiles = g.m_tiles;
     if (GROUPED) {
-        // which (expert, row tile) this workgroup has: experts in order, each with ceil(rows / 128) tiles
-        if (tid == 0) tile_info[0] = -1;
+        // experts in order, each with ceil(rows / 128) row tiles: how many lie before each expert's, and where its rows begin
         int base = 0;
         for (int e0 = 0; e0 < g.n_groups; e0 += 512) {
             const int e = e0 + tid;
@@ -598,136 +611,130 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
                 if (w < wave) before += scan_waves[w];
                 round_total += scan_waves[w];
             }
-            const int first = before + incl - tiles;
-            if (row_tile >= first && row_tile < first + tiles) {
-                tile_info[0] = e;
-                tile_info[1] = begin + (row_tile - first) * WD_BM;
-                tile_info[2] = end;
-                tile_info[3] = tiles;
+            if (e < g.n_groups) {
+                tiles_before[e] = before + incl - tiles;
+                places[e] = begin;
+                if (e == g.n_groups - 1) {
+                    tiles_before[e + 1] = before + incl;
+                    places[e + 1] = end;
+                }
             }
             base += round_total;
             __syncthreads();
-            if (row_tile < base) break;
         }
-        __syncthreads();
-        const int e = tile_info[0];
-        if (e < 0) return;
-        row_begin = tile_info[1];
-        row_end = min(tile_info[2], row_begin + WD_BM);
-        W += (size_t)e * g.w_group_stride;
-    } else {
-        row_begin = row_tile * WD_BM;
-        row_end = min(g.M, row_begin + WD_BM);
+        row_tiles = __builtin_amdgcn_readfirstlane(base);
     }
-    if (tid < WD_BM) {
-        const int m = row_begin + tid;
-        int ra = -1, rc = -1;
-        if (m < row_end) {
-            if (GROUPED) {
-                const int p = g.list[m];
-                ra = p / g.a_div;
-                rc = p;
-            } else {
-                ra = rc = m;
-            }
+    const int total = strips * row_tiles;
+
+    // a tile of the product: which weights, which rows (places in the list, if grouped)
+    struct Tile {
+        const bf16_t* W;
+        int n0, row_begin, row_end, tiles;      // tiles: row tiles that read these weights
+    };
+    auto tile_at = [&](int at) {
+        Tile t;
+        int strip, row_tile;
+        tile_place<GROUPED>(g, at, strips, row_tiles, strip, row_tile);
+        t.n0 = strip * FEATS;
+        t.W = g.W;
+        if (GROUPED) {
+            // the last expert with at most this many row tiles before its own (one without rows has as many as the next)
+            int found = 0;
+            for (int e0 = 0; e0 < g.n_groups; e0 += 64) found += __popcll(__ballot(e0 + lane < g.n_groups && tiles_before[min(e0 + lane, g.n_groups)] <= row_tile));
+            const int e = __builtin_amdgcn_readfirstlane(found) - 1;
+            const int first = __builtin_amdgcn_readfirstlane(tiles_before[e]), end = __builtin_amdgcn_readfirstlane(places[e + 1]);
+            t.tiles = __builtin_amdgcn_readfirstlane(tiles_before[e + 1]) - first;
+            t.row_begin = __builtin_amdgcn_readfirstlane(places[e]) + (row_tile - first) * WD_BM;
+            t.row_end = min(end, t.row_begin + WD_BM);
+            t.W += (size_t)e * g.w_group_stride;
+        } else {
+            t.tiles = g.m_tiles;
+            t.row_begin = row_tile * WD_BM;
+            t.row_end = min(g.M, t.row_begin + WD_BM);
         }
-        rows_a[tid] = ra;
-        rows_c[tid] = rc;
-    }
-    __syncthreads();
+        return t;
+    };
 
     const int K = g.K;
     // wave (wm, wn): rows 64 * wm .. (4 tiles of 16), 4 tiles of 16 weight rows
     const int wm = wave >> 2, wn = wave & 3;
     const int lr = lane & 15;
-    int w_row[4];  // LDS rows of the wave's 4 feature tiles
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        if (EPI == TL_SWIGLU)
-            w_row[f] = (f < 2 ? 0 : HALF) + 32 * wn + 16 * (f & 1) + lr;   // tiles 0,1: gate rows; tiles 2,3: the up rows of the same features
-        else
-            w_row[f] = 64 * wn + 16 * f + lr;
-    }
     constexpr int TT = 4;
-    f32x4_t acc[4][TT], total[SPLIT ? 4 : 1][SPLIT ? TT : 1];
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int t = 0; t < TT; ++t) acc[f][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const int steps_total = (K + 31) >> 5;
     const int per = (steps_total + g.ks - 1) / g.ks;   // 32-wide steps in a run
-    bool first_run = true;
 
     // the same unpadded, swizzled rows as the 4-wave form: chunk c (16 bytes) of row r sits at place c ^ ((r >> 1) & 7)
     constexpr int W_LOADS = 4, A_LOADS = 2, LOADS = W_LOADS + A_LOADS;   // load instructions a wave issues per tile
-    const int n_tiles = K / TL_BK;
+    const int n_tiles = K / TL_BK, last = n_tiles - 1;
     const int tiles_per_run = SPLIT ? per / 2 : n_tiles;
-    uint32_t w_at[W_LOADS], a_at[A_LOADS];
     const int place = lane & 7;
-#pragma unroll
-    for (int j = 0; j < W_LOADS; ++j) {
-        const int r = 32 * wave + 8 * j + (lane >> 3);           // row of the W tile
-        const int ch = place ^ ((r >> 1) & 7);
-        int wr;
-        if (EPI == TL_SWIGLU) wr = (r < HALF ? 0 : g.up_offset) + min(n0 + (r & (HALF - 1)), g.N - 1);
-        else wr = min(n0 + r, g.N - 1);
-        w_at[j] = (uint32_t)(((size_t)wr * K + 8 * ch) * sizeof(bf16_t));
-    }
-#pragma unroll
-    for (int j = 0; j < A_LOADS; ++j) {
-        const int r = 16 * wave + 8 * j + (lane >> 3);           // row of the A tile
-        const int ch = place ^ ((r >> 1) & 7);
-        const int ra = rows_a[r];
-        a_at[j] = (uint32_t)(((size_t)(ra >= 0 ? ra : 0) * g.lda + 8 * ch) * sizeof(bf16_t));
-    }
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    // What the loads are of: weights from a base the workgroup shares, A's rows (those of the wave, where the tile has them).
     // A tile of few rows (an expert's last, or its only one) is not multiplied out to 128: a wave whose 16 rows of A lie past the tile's
     // rows leaves them unread, and with at most 64 rows the waves of the upper half only bring weights.  What LDS holds for such rows makes
     // columns of the product that are never stored.  Weights that no other row tile reads come as bytes read once, which the caches do not
     // keep; where several do, the later ones find them in the caches (all as read once: down of 2,048 rows 596 -> 719 us).  Both, gate_up (256
     // experts or some 60, 3,072 features of 3,072 values): 2,048 rows in 64 an expert 1,037 -> 984 us, in 300 602 -> 535; 37 prompts of 45
     // 1,050 -> 952; 64-row tiles: 64 rows in 221 experts 669 -> 601 (6.9 TB/s), 520 rows 752 -> 700, down of 64 rows 345 -> 318.
-    const int rows_here = row_end - row_begin;
-    const bool read_once = __builtin_amdgcn_readfirstlane(GROUPED ? tile_info[3] : g.m_tiles) == 1;
-    const bool brings_rows = __builtin_amdgcn_readfirstlane(16 * wave) < rows_here;
-    const bool works = __builtin_amdgcn_readfirstlane(64 * wm) < rows_here;
-    auto issue = [&](int t, int stage) {
-        const bf16_t* wb = W + (size_t)t * TL_BK;
-        const bf16_t* ab = g.A + (size_t)t * TL_BK;
+    const bf16_t* w_base;
+    uint32_t w_at[W_LOADS], a_at[A_LOADS];
+    bool brings_rows, read_once;
+    auto rows_in = [&](const Tile& t) { return 16 * wave < t.row_end - t.row_begin; };
+    auto ask_pairs = [&](const Tile& t, int slot) {
+        if (GROUPED && tid < WD_BM) pairs[slot][tid] = g.list[min(t.row_begin + tid, t.row_end - 1)];
+    };
+    auto row_of = [&](const Tile& t, int slot, int r) { return GROUPED ? pairs[slot][r] : min(t.row_begin + r, t.row_end - 1); };
+    auto adopt = [&](const Tile& t, int slot) {
+        w_base = t.W;
+        read_once = t.tiles == 1;
+        brings_rows = rows_in(t);
 #pragma unroll
         for (int j = 0; j < W_LOADS; ++j) {
-            void* to = &Ws[(stage * WD_BN + 32 * wave_u + 8 * j) * TL_BK];
-            if (read_once) stream_to_lds(wb, w_at[j], to);
-            else load_to_lds(wb, w_at[j], to);
+            const int r = 32 * wave + 8 * j + (lane >> 3);           // row of the W tile
+            int wr;
+            if (EPI == TL_SWIGLU) wr = (r < HALF ? 0 : g.up_offset) + min(t.n0 + (r & (HALF - 1)), g.N - 1);
+            else wr = min(t.n0 + r, g.N - 1);
+            w_at[j] = (uint32_t)(((size_t)wr * K + 8 * (place ^ ((r >> 1) & 7))) * sizeof(bf16_t));
+        }
+#pragma unroll
+        for (int j = 0; j < A_LOADS; ++j) {
+            const int r = 16 * wave + 8 * j + (lane >> 3);           // row of the A tile
+            const int ra = GROUPED ? row_of(t, slot, r) / g.a_div : row_of(t, slot, r);
+            a_at[j] = (uint32_t)(((size_t)ra * g.lda + 8 * (place ^ ((r >> 1) & 7))) * sizeof(bf16_t));
+        }
+    };
+    auto issue = [&](int t, int stage) {
+        const bf16_t* wb = w_base + (size_t)t * TL_BK;
+        const bf16_t* ab = g.A + (size_t)t * TL_BK;
+        bf16_t* to = &Ws[(stage * WD_BN + 32 * wave) * TL_BK];
+        if (read_once) {
+#pragma unroll
+            for (int j = 0; j < W_LOADS; ++j) stream_to_lds(wb, w_at[j], to + 8 * j * TL_BK);
+        } else {
+#pragma unroll
+            for (int j = 0; j < W_LOADS; ++j) load_to_lds(wb, w_at[j], to + 8 * j * TL_BK);
         }
         if (brings_rows) {
 #pragma unroll
-            for (int j = 0; j < A_LOADS; ++j) load_to_lds(ab, a_at[j], &As[(stage * WD_BM + 16 * wave_u + 8 * j) * TL_BK]);
+            for (int j = 0; j < A_LOADS; ++j) load_to_lds(ab, a_at[j], &As[(stage * WD_BM + 16 * wave + 8 * j) * TL_BK]);
         }
     };
-    int w_rd[4], a_rd[TT], w_swz[4], a_swz[TT];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        w_rd[f] = w_row[f] * TL_BK;
-        w_swz[f] = (w_row[f] >> 1) & 7;
-    }
-#pragma unroll
-    for (int q = 0; q < TT; ++q) {
-        const int r = 64 * wm + 16 * q + lr;
-        a_rd[q] = r * TL_BK;
-        a_swz[q] = (r >> 1) & 7;
-    }
-    const int kg = lane >> 4;
+    // operand reads: rows 16 apart are swizzled alike, so a lane's places differ by constants.  SwiGLU: feature tiles 0,1: gate rows; 2,3:
+    // the up rows of the same features
+    const int kg = lane >> 4, swizzle = (lr >> 1) & 7;
+    const int w_lane = ((EPI == TL_SWIGLU ? 32 : 64) * wn + lr) * TL_BK, a_lane = (64 * wm + lr) * TL_BK;
+    f32x4_t acc[4][TT], sum[SPLIT ? 4 : 1][SPLIT ? TT : 1];
     // the operands of one half (32 of k) of a stage's tile
     auto read_half = [&](int stage, int kk, bf16x8_t (&wf)[4], bf16x8_t (&af)[TT]) {
-        const bf16_t* ws = &Ws[stage * WD_BN * TL_BK];
-        const bf16_t* as = &As[stage * WD_BM * TL_BK];
+        const int chunk = 8 * ((kk / 8 + kg) ^ swizzle);
+        const bf16_t* ws = &Ws[stage * WD_BN * TL_BK + w_lane + chunk];
+        const bf16_t* as = &As[stage * WD_BM * TL_BK + a_lane + chunk];
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
-            wf[f] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&ws[w_rd[f] + 8 * ((kk / 8 + kg) ^ w_swz[f])]));
+        for (int f = 0; f < 4; ++f) {
+            const int row = EPI == TL_SWIGLU ? (f < 2 ? 0 : HALF) + 16 * (f & 1) : 16 * f;
+            wf[f] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&ws[row * TL_BK]));
+        }
 #pragma unroll
-        for (int q = 0; q < TT; ++q)
-            af[q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&as[a_rd[q] + 8 * ((kk / 8 + kg) ^ a_swz[q])]));
+        for (int q = 0; q < TT; ++q) af[q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(&as[16 * q * TL_BK]));
     };
     auto multiply_half = [&](const bf16x8_t (&wf)[4], const bf16x8_t (&af)[TT]) {
 #pragma unroll
@@ -735,128 +742,206 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
 #pragma unroll
             for (int q = 0; q < TT; ++q) acc[f][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[f], af[q], acc[f][q], 0, 0, 0);
     };
-    // Three tiles in LDS; while a tile's first half is multiplied its second half's operands are read, and while the
-    // second half is multiplied the next tile's first: the matrix cores and LDS work at the same time, also within a
-    // wave.  One barrier a tile, in its middle: by then a wave has all operands of tile t in registers, so after the
-    // barrier tile t's stage takes tile t+3, and tile t+1 (awaited before the barrier) can be read by everybody.
-    issue(0, 0);
-    if (1 < n_tiles) issue(1, 1);
-    if (2 < n_tiles) issue(2, 2);
-    // until at most the loads of `out` tiles are on their way (LDS reads awaited too where the wave makes any)
-    auto wait_loads = [&](int out) {
-        if (out == 2) {
-            if (brings_rows) __builtin_amdgcn_s_waitcnt(0x0070 | (2 * LOADS));
-            else __builtin_amdgcn_s_waitcnt(0x0070 | (2 * W_LOADS));
-        } else if (out == 1) {
-            if (brings_rows) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);
-            else __builtin_amdgcn_s_waitcnt(0x0070 | W_LOADS);
-        } else {
-            __builtin_amdgcn_s_waitcnt(0x0070);
-        }
-    };
-    wait_loads(min(2, n_tiles - 1));
-    __syncthreads();
-    const int last = n_tiles - 1;   // the last tile has no tile after it: it runs after the loop, so the loop's body has no branch around its reads
-    if (!works) {
-        for (int t = 0, stage = 0; t < last; ++t) {
-            wait_loads(t + 2 < n_tiles ? 1 : 0);
-            __syncthreads();
-            if (t + 3 < n_tiles) issue(t + 3, stage);
-            stage = stage == 2 ? 0 : stage + 1;
-        }
-        return;
-    }
-    bf16x8_t wf_a[4], af_a[TT], wf_b[4], af_b[TT];
-    read_half(0, 0, wf_a, af_a);
-    int t = 0, stage = 0;
-    for (int run_end = tiles_per_run;; run_end += tiles_per_run) {
-        const int stop = min(run_end, last);
-        for (; t < stop; ++t) {
-            read_half(stage, 32, wf_b, af_b);
-            multiply_half(wf_a, af_a);
-            WD_INTERLEAVE();
-            const int next = stage == 2 ? 0 : stage + 1;
-            // this wave's operand reads of tile t are done, and its part of tile t+1 has arrived (tile t+2's may be out)
-            wait_loads(t + 2 < n_tiles ? 1 : 0);
-            __syncthreads();
-            if (t + 3 < n_tiles) issue(t + 3, stage);
-            read_half(next, 0, wf_a, af_a);
-            multiply_half(wf_b, af_b);
-            WD_INTERLEAVE();
-            stage = next;
-        }
-        if (SPLIT && t == run_end && t < n_tiles) {
-            // a run of K ends: its sum joins the runs before it, in run order
-#pragma unroll
-            for (int f = 0; f < 4; ++f)
-#pragma unroll
-                for (int q = 0; q < TT; ++q) {
-                    if (first_run) total[f][q] = acc[f][q];
-                    else total[f][q] = f32x4_t{total[f][q][0] + acc[f][q][0], total[f][q][1] + acc[f][q][1],
-                                               total[f][q][2] + acc[f][q][2], total[f][q][3] + acc[f][q][3]};
-                    acc[f][q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                }
-            first_run = false;
-        }
-        if (t >= last) break;
-    }
-    read_half(stage, 32, wf_b, af_b);
-    multiply_half(wf_a, af_a);
-    multiply_half(wf_b, af_b);
-    if (SPLIT && !first_run) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int q = 0; q < TT; ++q)
-                acc[f][q] = f32x4_t{total[f][q][0] + acc[f][q][0], total[f][q][1] + acc[f][q][1], total[f][q][2] + acc[f][q][2],
-                                    total[f][q][3] + acc[f][q][3]};
-    }
-
-    // acc[f][q][i]: feature (tile f) 4*(lane/16) + i, row 64*wm + 16*q + lane%16
     const int fq = 4 * (lane >> 4);
     const bool rows_aligned = g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;   // a lane's four features make one access
     // The activation's numbers formed once: behind the stores, which may write what it reads, they were formed for every tile
     // (a softplus pair 16 times a thread: 2,048 rows, 2,048 -> 8,192 features with xIELU 126 -> 101 us).
-    const ActFn act(EPI == TL_STORE ? g.act : LLMX_ACT_NONE, g.act_params);
-#pragma unroll
-    for (int q = 0; q < TT; ++q) {
-        const int rc = rows_c[64 * wm + 16 * q + lr];
-        if (rc < 0) continue;
-        TC* crow = (TC*)g.C + (size_t)rc * g.ldc;
-        if (EPI == TL_SWIGLU) {
-            const GluRow glu(g.glu, rc);
-#pragma unroll
-            for (int f = 0; f < 2; ++f) {
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = glu(acc[f][q][i], acc[f + 2][q][i]);
-                store_quad<false>(crow, n0 + 32 * wn + 16 * f + fq, g.N, rows_aligned, v);
+    const ActFn act(!BARE && EPI == TL_STORE ? g.act : LLMX_ACT_NONE, g.act_params);
+
+    // Three K tiles in LDS; while a tile's first half is multiplied its second half's operands are read, and while the
+    // second half is multiplied the next tile's first: the matrix cores and LDS work at the same time, also within a
+    // wave.  One barrier a tile, in its middle: by then a wave has all operands of tile t in registers, so after the
+    // barrier tile t's stage takes tile t+3 (past K's end: the next tile of the product's first ones), and tile t+1
+    // (awaited before the barrier) can be read by everybody.
+    if ((int)blockIdx.x >= total) return;
+    // A workgroup's first tile is its number's; the others it draws, two ahead, until the next one is none.  So every workgroup with a first
+    // tile draws two that are none, and who draws the last of all puts the counter back.
+    const bool tickets = BARE && GROUPED && g.ticket != nullptr;       // (K of at least four K tiles: TILE_TICKETS_MIN_K)
+    const int firsts = min((int)gridDim.x, total);
+    auto tile_of = [&](int n) {
+        if (n == total + firsts - 1) atomicExch(g.ticket, 0);
+        return firsts + n;
+    };
+    if (tid == 0) {
+        for (int i = 0; i < 2; ++i) drawn[i] = tickets ? tile_of(atomicAdd(g.ticket, 1)) : total;
+    }
+    __syncthreads();
+    int turn = 0, ticket = 0;
+    bool drew = false;
+    Tile tile = tile_at(blockIdx.x), next = tile;
+    int stage = 0, slot = 0;
+    ask_pairs(tile, 0);
+    if (GROUPED) __syncthreads();
+    adopt(tile, 0);
+    for (int t = 0; t < min(3, n_tiles); ++t) issue(t, t);
+    for (;;) {
+        const int rows_here = tile.row_end - tile.row_begin;
+        const bool works = 64 * wm < rows_here;
+        const int following = __builtin_amdgcn_readfirstlane(drawn[turn]);
+        const bool more = BARE && GROUPED && following < total;
+        const bool brings_now = brings_rows;
+        const int slot_next = slot == 2 ? 0 : slot + 1;
+        if (more) {
+            next = tile_at(following);
+            ask_pairs(next, slot_next);
+        }
+        const bool brings_next = rows_in(next);
+        auto ask = [&](int t, int into) {
+            if (t < n_tiles) {
+                issue(t, into);
+            } else if (more) {
+                if (t == n_tiles) adopt(next, slot_next);
+                issue(t - n_tiles, into);
             }
+        };
+        // until at most the loads of tile t are on their way (LDS reads awaited too where the wave makes any)
+        auto wait_but = [&](int t) {
+            if (t >= n_tiles && !more) __builtin_amdgcn_s_waitcnt(0x0070);
+            else if (t < n_tiles ? brings_now : brings_next) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);
+            else __builtin_amdgcn_s_waitcnt(0x0070 | W_LOADS);
+        };
+        auto last_stage_read = [&]() {          // by this wave, then by all: the stage takes one more K tile of the next tile
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            __syncthreads();
+            ask(n_tiles + 2, stage);
+            stage = stage == 2 ? 0 : stage + 1;
+        };
+        __builtin_amdgcn_s_waitcnt(0x0070);     // the first three K tiles, and the stores of the tile before
+        if (tid == 0 && drew) drawn[1 - turn] = tile_of(ticket);
+        turn = 1 - turn;
+        __syncthreads();
+        drew = more;
+        if (tid == 0 && more) ticket = atomicAdd(g.ticket, 1);      // travels while the tile is multiplied, and is looked at behind the next wait for everything
+        if (!works) {
+            for (int t = 0; t < last; ++t) {
+                wait_but(t + 2);
+                __syncthreads();
+                ask(t + 3, stage);
+                stage = stage == 2 ? 0 : stage + 1;
+            }
+            last_stage_read();
         } else {
 #pragma unroll
-            for (int f = 0; f < 4; ++f) {
-                float v[4] = {acc[f][q][0], acc[f][q][1], acc[f][q][2], acc[f][q][3]};
-                if (llmx_act_reads_vector(g.act)) {
+            for (int f = 0; f < 4; ++f)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = biased_act(g.act, v[i], act_feature(g.act, g.act_params, n0 + 64 * wn + 16 * f + fq + i, g.N));
-                } else if (EPI == TL_STORE && g.act != LLMX_ACT_NONE) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = act(v[i]);
+                for (int q = 0; q < TT; ++q) {
+                    acc[f][q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    if (SPLIT) sum[f][q] = acc[f][q];        // (written before it is read anyway: said here, it need not live from tile to tile)
                 }
-                store_quad<EPI == TL_ADD>(crow, n0 + 64 * wn + 16 * f + fq, g.N, rows_aligned, v);
+            bool first_run = true;
+            bf16x8_t wf_a[4], af_a[TT], wf_b[4], af_b[TT];
+            read_half(stage, 0, wf_a, af_a);
+            auto step = [&](int t, auto inside) {       // inside: K tile t + 3 is one of this tile's
+                read_half(stage, 32, wf_b, af_b);
+                multiply_half(wf_a, af_a);
+                WD_INTERLEAVE();
+                const int after = stage == 2 ? 0 : stage + 1;
+                // this wave's operand reads of tile t are done, and its part of tile t+1 has arrived (tile t+2's may be out)
+                if (!decltype(inside)::value) wait_but(t + 2);
+                else if (brings_now) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);
+                else __builtin_amdgcn_s_waitcnt(0x0070 | W_LOADS);
+                __syncthreads();
+                if (decltype(inside)::value) issue(t + 3, stage);
+                else ask(t + 3, stage);
+                read_half(after, 0, wf_a, af_a);
+                multiply_half(wf_b, af_b);
+                WD_INTERLEAVE();
+                stage = after;
+            };
+            int t = 0;      // the last tile has no tile after it: it runs after the loop, so the loop's body has no branch around its reads
+            for (int run_end = tiles_per_run;; run_end += tiles_per_run) {
+                const int stop = min(run_end, last);
+                for (; t < min(stop, n_tiles - 3); ++t) step(t, std::true_type{});
+                for (; t < stop; ++t) step(t, std::false_type{});
+                if (SPLIT && t == run_end && t < n_tiles) {
+                    // a run of K ends: its sum joins the runs before it, in run order
+#pragma unroll
+                    for (int f = 0; f < 4; ++f)
+#pragma unroll
+                        for (int q = 0; q < TT; ++q) {
+                            if (first_run) sum[f][q] = acc[f][q];
+                            else sum[f][q] = f32x4_t{sum[f][q][0] + acc[f][q][0], sum[f][q][1] + acc[f][q][1], sum[f][q][2] + acc[f][q][2],
+                                                     sum[f][q][3] + acc[f][q][3]};
+                            acc[f][q] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                        }
+                    first_run = false;
+                }
+                if (t >= last) break;
+            }
+            read_half(stage, 32, wf_b, af_b);
+            multiply_half(wf_a, af_a);
+            multiply_half(wf_b, af_b);
+            if (SPLIT && !first_run) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f)
+#pragma unroll
+                    for (int q = 0; q < TT; ++q)
+                        acc[f][q] = f32x4_t{sum[f][q][0] + acc[f][q][0], sum[f][q][1] + acc[f][q][1], sum[f][q][2] + acc[f][q][2],
+                                            sum[f][q][3] + acc[f][q][3]};
+            }
+            last_stage_read();
+
+            // acc[f][q][i]: feature (tile f) 4*(lane/16) + i, row 64*wm + 16*q + lane%16
+#pragma unroll
+            for (int q = 0; q < TT; ++q) {
+                if (64 * wm + 16 * q + lr >= rows_here) continue;
+                const int rc = row_of(tile, slot, 64 * wm + 16 * q + lr);
+                TC* crow = (TC*)g.C + (size_t)rc * g.ldc;
+                if (EPI == TL_SWIGLU) {
+                    const GluRow glu(BARE ? GluArgs{LLMX_GLU_SILU, 0.0f, nullptr, nullptr, 0} : g.glu, rc);
+#pragma unroll
+                    for (int f = 0; f < 2; ++f) {
+                        float v[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = glu(acc[f][q][i], acc[f + 2][q][i]);
+                        store_quad<false>(crow, tile.n0 + 32 * wn + 16 * f + fq, g.N, rows_aligned, v);
+                    }
+                } else {
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) {
+                        const int n = tile.n0 + 64 * wn + 16 * f + fq;
+                        float v[4] = {acc[f][q][0], acc[f][q][1], acc[f][q][2], acc[f][q][3]};
+                        // a copy of the sums: stored as they are, the compiler lays them out for the stores from the first product on
+                        // (and spills a hundred registers in the loop)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(v[i]));
+                        if (!BARE && llmx_act_reads_vector(g.act)) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) v[i] = biased_act(g.act, v[i], act_feature(g.act, g.act_params, n + i, g.N));
+                        } else if (!BARE && EPI == TL_STORE && g.act != LLMX_ACT_NONE) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) v[i] = act(v[i]);
+                        }
+                        store_quad<EPI == TL_ADD>(crow, n, g.N, rows_aligned, v);
+                    }
+                }
             }
         }
+        if (!BARE || !more) return;
+        tile = next;
+        slot = slot_next;
     }
 }
 
 // form: which kernel takes the product.  The lean forms need whole 64-wide tiles of K, runs that end on them, and
 // operands whose byte offsets fit 32 bits (llmx_gemm_tile_offsets_fit).
 enum : int { FORM_64 = 0, FORM_128 = 1, FORM_WIDE = 2, FORM_BOUNDED = 3, FORM_64_DEEP = 4 };
+// Routed products' tiles of 128 rows: the wide form for long K, and with tickets for shorter K too while a group has some 200 rows at most
+// (256 experts, 3,072 features of 1,536 values, four waves a tile and the wide form, us: 64 rows an expert 563 and 525, 100 647 and 605, 130 770
+// and 761, 300 1,357 and 1,411; 2,048 features, 100 rows, of 1,024 315 and 270, of 512 194 and 170, but 64 experts of 150 rows, 512 76 and 79).
+#define TILE_TICKETS_MIN_K 1024
+static bool wide_routed(int K, long pairs, int groups, const int* ticket) { return K >= 2048 || (ticket && K >= TILE_TICKETS_MIN_K && pairs <= 200L * groups); }
 
 template <int EPI, typename TC, bool GROUPED, bool SPLIT>
 static void tile_launch_form(const TileArgs& g, int form, dim3 grid, hipStream_t stream) {
-    if (form == FORM_WIDE) hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT>), grid, dim3(512), 0, stream, g);
-    else if (form == FORM_128) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, true, 128>), grid, dim3(256), 0, stream, g);
+    if (form == FORM_WIDE) {
+        const unsigned tiles = grid.x * grid.y;
+        const bool bare = EPI == TL_SWIGLU ? g.glu.kind == LLMX_GLU_SILU && !g.glu.row_scale && !g.glu.row_gate : g.act == LLMX_ACT_NONE;
+        if (bare) hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT, true>), dim3(g.ticket && tiles > TILE_CUS ? TILE_CUS : tiles), dim3(512), 0, stream, g);
+        else hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT, false>), dim3(tiles), dim3(512), 0, stream, g);
+        return;
+    }
+    if (form == FORM_128) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, true, 128>), grid, dim3(256), 0, stream, g);
     else if (form == FORM_64) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, true, 64>), grid, dim3(256), 0, stream, g);
     else if (form == FORM_64_DEEP && !GROUPED) hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, false, SPLIT, true, 64, TL_DEEP_STAGES>), grid, dim3(256), 0, stream, g);
     else hipLaunchKernelGGL((gemm_tile_kernel<EPI, TC, GROUPED, SPLIT, false, 64>), grid, dim3(256), 0, stream, g);
@@ -954,7 +1039,7 @@ static int form_feats(int form, int epi) { return (epi == TL_SWIGLU ? 64 : 128) 
 //     of a 128-row tile is padding: 200,064 features of 3,072, 48 rows 265 -> 257 us, 64 rows 276 -> 268).
 //     With `runs_scratch` (llmx_gemm_tile_runs_scratch floats) a product of few tiles and several runs of K gives each
 //     run a workgroup of its own and adds the runs' sums in a second kernel, in the order the one kernel adds them.
-//   grouped with tile_stats: both a 128-row form (wide for long K, 4 waves for short K) and the 64-row form are
+//   grouped with tile_stats: both a 128-row form (wide_routed: the wide one, or 4 waves for short K) and the 64-row form are
 //     launched; on the device the one that fits the groups' rows works and the other leaves at once.
 // Floats of scratch with which llmx_gemm_tile multiplies the runs of a dense product apart (0: it would not).
 extern "C" long llmx_gemm_tile_runs_scratch(int M, int N, int K, int epi, int ks, int n_groups) {
@@ -967,10 +1052,10 @@ extern "C" long llmx_gemm_tile_runs_scratch(int M, int N, int K, int epi, int ks
     return runs < 2 ? 0 : (long)runs * M * N;
 }
 
-extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldc, int epi, int ks,
+static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldc, int epi, int ks,
                                      int n_groups, int max_tiles, const int* group_offsets, const int* list, int a_div, long w_group_stride,
                                      int up_offset, const int* tile_stats, int stats_choose, float* runs_scratch, int act, const float* act_params, int glu_kind,
-                                     float glu_limit, const float* glu_row_scale, const float* glu_row_gate, int glu_row_gate_ld, hipStream_t stream) {
+                                     float glu_limit, const float* glu_row_scale, const float* glu_row_gate, int glu_row_gate_ld, int* ticket, hipStream_t stream) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (K % 8) return -2;
     const bool grouped = n_groups > 0;
@@ -980,9 +1065,10 @@ extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int 
     TileArgs g{(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldc, group_offsets, list, n_groups, a_div > 0 ? a_div : 1,
                w_group_stride, up_offset, 0, ks, 64, nullptr, -1, 0, 0, 0, epi != TL_SWIGLU ? act : LLMX_ACT_NONE, act_params,
                GluArgs{epi == TL_SWIGLU ? glu_kind : LLMX_GLU_SILU, glu_limit, epi == TL_SWIGLU ? glu_row_scale : nullptr,
-                       epi == TL_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld}};
+                       epi == TL_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld},
+               ticket};
     if (!llmx_act_fits(act, act_params, epi == TL_STORE, epi == TL_ADD)) return -2;
-    auto launch = [&](int form, int tiles_y) -> int {
+    auto launch = [&](int form, int tiles_y, bool short_k = false) -> int {      // short_k: 128-row tiles of short K, whichever kernel has them
         g.bm = form_rows(form);
         g.m_tiles = (M + g.bm - 1) / g.bm;
         const int feats = form_feats(form, epi);
@@ -990,7 +1076,8 @@ extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int 
         if (grid.y > 65535) return -2;
         g.strip_runs = grouped ? 0 : llmx_gemm_tile_strip_runs((int)grid.x, (int)grid.y, form == FORM_WIDE);
         if (form == FORM_64_DEEP) llmx_note_launch(LK_GEMM_TILE_64_DEEP);
-        llmx_note_launch(form == FORM_WIDE ? (grouped ? LK_GEMM_TILE_GROUPED_WIDE : LK_GEMM_TILE_WIDE)
+        llmx_note_launch(short_k ? LK_GEMM_TILE_GROUPED_128
+                         : form == FORM_WIDE ? (grouped ? LK_GEMM_TILE_GROUPED_WIDE : LK_GEMM_TILE_WIDE)
                          : form == FORM_128 ? LK_GEMM_TILE_GROUPED_128
                          : form == FORM_64 || form == FORM_64_DEEP ? (grouped ? LK_GEMM_TILE_GROUPED_64 : LK_GEMM_TILE_64)
                                            : (grouped ? LK_GEMM_TILE_GROUPED_BOUNDED : LK_GEMM_TILE_BOUNDED));
@@ -1029,13 +1116,13 @@ extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int 
         const long wide_tiles = (long)((M + WD_BM - 1) / WD_BM) * ((N + form_feats(FORM_WIDE, epi) - 1) / form_feats(FORM_WIDE, epi));
         const long narrow_tiles = (long)((M + 63) / 64) * ((N + form_feats(FORM_64, epi) - 1) / form_feats(FORM_64, epi));
         rc = launch(narrow_tiles <= deep_most(M) ? FORM_64_DEEP : wide_tiles >= (K >= 4096 && M >= 512 ? 150 : 192) && M > 64 ? FORM_WIDE : FORM_64, 0);
-    } else if (tile_stats) {
+    } else if (tile_stats && n_groups <= WD_MAX_GROUPS) {     // (more groups: 64-row tiles)
         // 128-row tiles: each group adds at most one partial tile
         const int big_tiles = (n_groups < M ? n_groups : M) + M / 128;
         g.tile_stats = tile_stats;
         g.choice_bit = stats_choose ? tile_k_class(K) : -1;
         g.run_if_big = 1;
-        rc = launch(K >= 2048 ? FORM_WIDE : FORM_128, big_tiles < max_tiles ? big_tiles : max_tiles);
+        rc = launch(wide_routed(K, M, n_groups, g.ticket) ? FORM_WIDE : FORM_128, big_tiles < max_tiles ? big_tiles : max_tiles, K < 2048);
         if (rc == 0) {
             g.run_if_big = 0;
             rc = launch(FORM_64, max_tiles);
@@ -1045,6 +1132,25 @@ extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int 
     }
     if (rc) return rc;
     return LLMX_CHECK_LAUNCH();
+}
+
+// ticket (grouped, optional): device int that holds 0 and does again afterwards; with it the wide form's workgroups stay and take tiles by it.
+extern "C" int llmx_gemm_tile_tickets(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldc, int epi, int ks,
+                                      int n_groups, int max_tiles, const int* group_offsets, const int* list, int a_div, long w_group_stride,
+                                      int up_offset, const int* tile_stats, int stats_choose, int* ticket, float* runs_scratch, int act, const float* act_params,
+                                      int glu_kind, float glu_limit, const float* glu_row_scale, const float* glu_row_gate, int glu_row_gate_ld,
+                                      hipStream_t stream) {
+    return gemm_tile(A, W, C, c_dtype, M, N, K, lda, ldc, epi, ks, n_groups, max_tiles, group_offsets, list, a_div, w_group_stride, up_offset, tile_stats,
+                     stats_choose, runs_scratch, act, act_params, glu_kind, glu_limit, glu_row_scale, glu_row_gate, glu_row_gate_ld, ticket, stream);
+}
+
+// ... without one.
+extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldc, int epi, int ks,
+                                     int n_groups, int max_tiles, const int* group_offsets, const int* list, int a_div, long w_group_stride,
+                                     int up_offset, const int* tile_stats, int stats_choose, float* runs_scratch, int act, const float* act_params, int glu_kind,
+                                     float glu_limit, const float* glu_row_scale, const float* glu_row_gate, int glu_row_gate_ld, hipStream_t stream) {
+    return gemm_tile(A, W, C, c_dtype, M, N, K, lda, ldc, epi, ks, n_groups, max_tiles, group_offsets, list, a_div, w_group_stride, up_offset, tile_stats,
+                     stats_choose, runs_scratch, act, act_params, glu_kind, glu_limit, glu_row_scale, glu_row_gate, glu_row_gate_ld, nullptr, stream);
 }
 
 // ... with the bare count in tile_stats, or none.

@@ -473,7 +473,7 @@ __global__ void __launch_bounds__(1024) moe_chunk_count_kernel(const int* __rest
 
 __global__ void __launch_bounds__(1024) moe_chunk_scan_kernel(int n_chunks, int n_pairs, int n_experts, int* __restrict__ chunk_counts, int* __restrict__ counts,
                                                              int* __restrict__ offsets, int* __restrict__ active, int* __restrict__ n_active,
-                                                             int* __restrict__ tiles128, int* __restrict__ choice) {
+                                                             int* __restrict__ tiles128, int* __restrict__ choice, int* __restrict__ ticket) {
     __shared__ int wave_total[16], wave_active[16], wave_tiles[16], wave_halves[16];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int e = tid;
@@ -505,6 +505,7 @@ __global__ void __launch_bounds__(1024) moe_chunk_scan_kernel(int n_chunks, int 
         wave_halves[wave] = halves;
     }
     __syncthreads();
+    if (tid == 0 && ticket) *ticket = 0;
     if (tid == 0 && tiles128) {
         int n128 = 0, n64 = 0, experts = 0;
         for (int w = 0; w < 16; ++w) {
@@ -560,9 +561,9 @@ extern "C" int llmx_tile_choice(int n_pairs, int n128, int n64, int experts) { r
 // counts [X], offsets [X+1], list [n_pairs], active [X], n_active [1]
 // scratch (optional): [ceil(n_pairs / 1024) * n_experts] ints for steps of many pairs
 // tiles128 (optional) [1]: with scratch and many pairs, the sum over experts of ceil(rows / 128); choice (optional, with tiles128):
-// which routed products take tiles of 128 rows, a bit a class of K (tile_choice.h)
-extern "C" int llmx_moe_align(const int* ids, int n_pairs, int n_experts, int* counts, int* offsets, int* list, int* active, int* n_active,
-                              int* scratch, int* tiles128, int* choice, hipStream_t stream) {
+// which routed products take tiles of 128 rows, a bit a class of K (tile_choice.h); ticket (optional) [1], with scratch and many pairs: set to 0
+extern "C" int llmx_moe_align_ticket(const int* ids, int n_pairs, int n_experts, int* counts, int* offsets, int* list, int* active, int* n_active,
+                                     int* scratch, int* tiles128, int* choice, int* ticket, hipStream_t stream) {
     if (n_pairs <= 0 || n_experts <= 0) return 0;
     llmx_note_launch(LK_MOE_ALIGN);
     if (n_pairs <= ALIGN_SMALL_PAIRS && n_experts <= 1024) {
@@ -573,13 +574,17 @@ extern "C" int llmx_moe_align(const int* ids, int n_pairs, int n_experts, int* c
         const int n_chunks = (n_pairs + 1023) / 1024;
         hipLaunchKernelGGL(moe_chunk_count_kernel, dim3(n_chunks), dim3(1024), 0, stream, ids, n_pairs, n_experts, scratch);
         hipLaunchKernelGGL(moe_chunk_scan_kernel, dim3(1), dim3(1024), 0, stream, n_chunks, n_pairs, n_experts, scratch, counts, offsets, active, n_active, tiles128,
-                           choice);
+                           choice, ticket);
         hipLaunchKernelGGL(moe_chunk_place_kernel, dim3(n_chunks), dim3(1024), 0, stream, ids, n_pairs, n_experts, scratch, list);
         return LLMX_CHECK_LAUNCH();
     }
     hipLaunchKernelGGL(moe_count_kernel, dim3(n_experts), dim3(256), 0, stream, ids, n_pairs, counts);
     hipLaunchKernelGGL(moe_place_kernel, dim3(n_experts), dim3(64), 0, stream, ids, n_pairs, n_experts, counts, offsets, list, active, n_active);
     return LLMX_CHECK_LAUNCH();
+}
+extern "C" int llmx_moe_align(const int* ids, int n_pairs, int n_experts, int* counts, int* offsets, int* list, int* active, int* n_active,
+                              int* scratch, int* tiles128, int* choice, hipStream_t stream) {
+    return llmx_moe_align_ticket(ids, n_pairs, n_experts, counts, offsets, list, active, n_active, scratch, tiles128, choice, nullptr, stream);
 }
 
 // ---------------------------------------------------------------------------

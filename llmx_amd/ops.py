@@ -110,6 +110,7 @@ def _declare(h) -> None:
         "llmx_paged_attention_mfma": [P, P, P, P, P, P, P, I, I, I, P, I, P, P, P, F, I, I, I, I, I, I, I, P, I, I, P],
         "llmx_route_topk": [P, P, I, L, P, P, P, I, I, I, I, I, F, P, I, I, I, P],
         "llmx_moe_align": [P, I, I, P, P, P, P, P, P, P, P, P],
+        "llmx_moe_align_ticket": [P, I, I, P, P, P, P, P, P, P, P, P, P],
         "llmx_route_topk_align": [P, P, I, L, P, P, P, I, I, I, I, I, F, I, I, I, P, P, P, P, P, P],
         "llmx_gemm_skinny": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, P, P, I, L, I, P, P, F, I, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_skinny_normed_ok": [I, I],
@@ -119,6 +120,7 @@ def _declare(h) -> None:
         "llmx_tile_choice": [I, I, I, I],
         "llmx_gemm_tile": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_chosen": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, I, P, I, F, P, P, I, P],
+        "llmx_gemm_tile_tickets": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_offsets_fit": [I, I, I, I, I, I, I, I],
         "llmx_sample_all": [P, P, P, P, P, P, I, I, P, P],
         "llmx_sample_topk": [P, P, P, P, P, P, P, P, I, I, P, I, P],
@@ -1201,13 +1203,14 @@ def gemm(a, w: torch.Tensor, c: torch.Tensor, epilogue: int = EPI_STORE, force_g
 def grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, offsets: torch.Tensor, pairs: torch.Tensor, a_div: int,
                  epilogue: int = EPI_STORE, active: Optional[torch.Tensor] = None, n_active: Optional[torch.Tensor] = None,
                  token_rows: Optional[int] = None, force_generic: bool = False, tile_stats: Optional[torch.Tensor] = None,
-                 glu: Optional["Glu"] = None, scratch=None, act=None) -> None:
+                 glu: Optional["Glu"] = None, scratch=None, act=None, ticket: Optional[torch.Tensor] = None) -> None:
     """For each group g: rows p in pairs[offsets[g]:offsets[g+1]] get c[p] = a[p // a_div] @ w[g]^T.
     `act`: as gemm's, for the store epilogue.
 
     With EPI_SWIGLU w[g] holds gate rows then up rows and c[p] = silu(gate) * up.  `active` / `n_active` (from
     moe_align) list the groups that have rows; with them, steps of few token rows (`token_rows`, default the pair
-    count) take the weight-streaming kernel.
+    count) take the weight-streaming kernel.  `ticket` int32 [1], as moe_align leaves it (0; it is 0 again afterwards, for the next product on
+    the stream): with `tile_stats` of two numbers, a product of many pairs may have its workgroups take tile after tile by it.
     """
     G, NW, K = w.shape
     if _glu_apart(glu, epilogue):
@@ -1246,10 +1249,12 @@ def grouped_gemm(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, offsets: tor
         return
     if not force_generic and _skinny_ok(a, w, c, epilogue):
         stats = _tile_stats(tile_stats)
-        _check(lib().llmx_gemm_tile_chosen(_dev(a, "a"), _dev(w, "w"), _dev(c, "c"), _code(c.dtype), n_pairs, N, K, K, N, epilogue,
-                                           _split_k(-(-N // 16), K), G, min(G, n_pairs) + n_pairs // 64, _dev(offsets, "offsets", torch.int32, (G + 1,)),
-                                           _dev(pairs, "pairs", torch.int32), a_div, NW * K, N if epilogue == EPI_SWIGLU else 0,
-                                           *((stats[-1], len(stats) - 1) if n_pairs >= TILE_STATS_MIN_PAIRS else (0, 0)), 0, *act_args, *glu_args, _stream()),
+        many = n_pairs >= TILE_STATS_MIN_PAIRS
+        _check(lib().llmx_gemm_tile_tickets(_dev(a, "a"), _dev(w, "w"), _dev(c, "c"), _code(c.dtype), n_pairs, N, K, K, N, epilogue,
+                                            _split_k(-(-N // 16), K), G, min(G, n_pairs) + n_pairs // 64, _dev(offsets, "offsets", torch.int32, (G + 1,)),
+                                            _dev(pairs, "pairs", torch.int32), a_div, NW * K, N if epilogue == EPI_SWIGLU else 0,
+                                            *((stats[-1], len(stats) - 1) if many else (0, 0)),
+                                            _dev(ticket, "ticket", torch.int32, (1,)) if many and len(stats) == 2 else 0, 0, *act_args, *glu_args, _stream()),
                "grouped_gemm_tile")
         return
     _check(lib().llmx_gemm_generic(_dev(a, "a"), _code(a.dtype), _dev(w, "w"), _code(w.dtype), _dev(c, "c"), _code(c.dtype),
@@ -1673,30 +1678,32 @@ def _tile_stats(tile_stats: Optional[torch.Tensor]) -> list:
 
 def moe_align(ids: torch.Tensor, n_experts: int, counts: torch.Tensor, offsets: torch.Tensor, pairs: torch.Tensor,
               active: torch.Tensor, n_active: torch.Tensor, scratch: Optional[torch.Tensor] = None,
-              tile_stats: Optional[torch.Tensor] = None) -> None:
+              tile_stats: Optional[torch.Tensor] = None, ticket: Optional[torch.Tensor] = None) -> None:
     """Groups the pairs p = t*k + j by expert (stable): counts [X], offsets [X+1], pairs [T*k], and the experts that
     have rows in increasing order: active [X] (first n_active[0] entries).  `scratch`: moe_align_scratch(...) int32 for
     steps of many pairs (made here when it is not given).  `tile_stats` int32 [1]: for TILE_STATS_MIN_PAIRS pairs or
     more it receives the sum over experts of ceil(rows / 128), by which grouped_gemm chooses its tile size; int32 [2]: behind it
-    the choice itself, from the tiles of both sizes and the experts that have rows, a bit a class of K, which grouped_gemm then follows."""
+    the choice itself, from the tiles of both sizes and the experts that have rows, a bit a class of K, which grouped_gemm then follows.
+    `ticket` int32 [1]: set to 0 for grouped_gemm where moe_align_scratch(...) is not 0."""
     n_pairs = ids.numel()
     need = moe_align_scratch(n_pairs, n_experts)
     if need and scratch is None:
         scratch = torch.empty(need, dtype=torch.int32, device=ids.device)
     if scratch is not None and scratch.numel() < need:
         raise KernelError(f"moe_align: scratch of {scratch.numel()} ints, {need} needed")
-    _check(lib().llmx_moe_align(_dev(ids, "ids", torch.int32), n_pairs, n_experts, _dev(counts, "counts", torch.int32, (n_experts,)),
+    _check(lib().llmx_moe_align_ticket(_dev(ids, "ids", torch.int32), n_pairs, n_experts, _dev(counts, "counts", torch.int32, (n_experts,)),
                                 _dev(offsets, "offsets", torch.int32, (n_experts + 1,)), _dev(pairs, "pairs", torch.int32, (n_pairs,)),
                                 _dev(active, "active", torch.int32, (n_experts,)), _dev(n_active, "n_active", torch.int32, (1,)),
                                 _dev(scratch if need else None, "scratch", torch.int32),
-                                *(_tile_stats(tile_stats) + [0])[:2] if need and n_pairs >= TILE_STATS_MIN_PAIRS else (0, 0), _stream()), "moe_align")
+                                *(_tile_stats(tile_stats) + [0])[:2] if need and n_pairs >= TILE_STATS_MIN_PAIRS else (0, 0),
+                                _dev(ticket if need else None, "ticket", torch.int32, (1,)), _stream()), "moe_align")
 
 
 def route_topk_align(z: torch.Tensor, bias: Optional[torch.Tensor], ids: torch.Tensor, weights: torch.Tensor, k: int, score: int,
                      normalize: bool, scale: float, counts: torch.Tensor, offsets: torch.Tensor, pairs: torch.Tensor,
                      active: torch.Tensor, n_active: torch.Tensor, parts: Optional[torch.Tensor] = None,
                      scratch: Optional[torch.Tensor] = None, tile_stats: Optional[torch.Tensor] = None,
-                     logit_bias: Optional[torch.Tensor] = None, groups=None) -> None:
+                     logit_bias: Optional[torch.Tensor] = None, groups=None, ticket: Optional[torch.Tensor] = None) -> None:
     """route_topk followed by moe_align; a step of at most 16 rows (at most 256 experts and 64 picks, no logit bias) does
     both in one launch, with the same bits.  With k + 1 slots a row in ids and weights (see route_topk) the pairs of the expert that
     every row runs are grouped with the others': counts [experts + 1] and so on."""
@@ -1714,7 +1721,7 @@ def route_topk_align(z: torch.Tensor, bias: Optional[torch.Tensor], ids: torch.T
             _dev(n_active, "n_active", torch.int32, (1,)), _stream()), "route_topk_align")
         return
     route_topk(z, bias, ids, weights, k, score, normalize, scale, parts, logit_bias, groups)
-    moe_align(ids, groups_out, counts, offsets, pairs, active, n_active, scratch, tile_stats)
+    moe_align(ids, groups_out, counts, offsets, pairs, active, n_active, scratch, tile_stats, ticket)
 
 
 def moe_combine(x: torch.Tensor, y: torch.Tensor, ids: torch.Tensor, weights: Optional[torch.Tensor], accumulate: bool = True) -> None:

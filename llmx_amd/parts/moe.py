@@ -207,20 +207,22 @@ class RoutedExperts(FeedForward):
         scratch = step.buf("experts.align_scratch", (need,), torch.int32) if need else None
         # for steps of many pairs the grouping also counts the experts' tiles of 128 rows, by which the products choose their tiles
         tile_stats = step.buf("experts.tile_stats", (2,), torch.int32) if T * slots >= ops.TILE_STATS_MIN_PAIRS else None
+        # ... and readies the counter by which the products' workgroups take tile after tile
+        ticket = step.buf("experts.ticket", (1,), torch.int32) if tile_stats is not None and need else None
         ops.route_topk_align(z, self.bias, ids, weights, k, self.score, self.normalize, self.scale, counts, offsets, pairs, active, n_active,
-                             parts=parts, scratch=scratch, tile_stats=tile_stats, logit_bias=self.logit_bias, groups=self.groups)
+                             parts=parts, scratch=scratch, tile_stats=tile_stats, logit_bias=self.logit_bias, groups=self.groups, ticket=ticket)
         step.observe("routing", logits=z, ids=ids[:, :k], weights=weights[:, :k])
         act = step.buf("experts.act", (T * slots, self.intermediate), step.act_dtype)
         on_input = self.weight_on == "input"
         if self.plain_unit is not None:
             ops.grouped_gemm(h, self.w_gate_up, act, offsets, pairs, slots, ops.EPI_STORE, active, n_active, token_rows=T, tile_stats=tile_stats,
-                             act=(self.plain_unit, None))
+                             act=(self.plain_unit, None), ticket=ticket)
         else:
             glu = ops.Glu(self.unit, self.limit, weights.view(T * slots) if on_input else None)
             ops.grouped_gemm(h, self.w_gate_up, act, offsets, pairs, slots, ops.EPI_SWIGLU, active, n_active, token_rows=T, tile_stats=tile_stats,
-                             glu=glu, scratch=step.buf)
+                             glu=glu, scratch=step.buf, ticket=ticket)
         y = step.buf("experts.y", (T * slots, self.hidden), torch.float32)
-        ops.grouped_gemm(act, self.w_down, y, offsets, pairs, 1, ops.EPI_STORE, active, n_active, token_rows=T, tile_stats=tile_stats)
+        ops.grouped_gemm(act, self.w_down, y, offsets, pairs, 1, ops.EPI_STORE, active, n_active, token_rows=T, tile_stats=tile_stats, ticket=ticket)
         ops.moe_combine(out, y, ids, None if on_input else weights, accumulate)
         if self.shared_width and not self.shared_joins:
             # the shared expert: its switch is a factor on the rows its second product reads (that product is linear), so the

@@ -1,0 +1,47 @@
+"""Routed tiled products whose workgroups take tile after tile by tickets, against a workgroup a tile: the same bits, and the counter 0 again."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# fewer tiles than CUs and many rounds of them; experts without rows, of one row, of whole tiles and one more, of few and many rows; a last strip that
+# is partial; K about the forms' bounds
+@pytest.mark.parametrize("N,K", [(256, 1024), (520, 1088), (1024, 2048), (2056, 2560)])
+@pytest.mark.parametrize("counts", ["even", "uneven", "few"])
+def test_tickets_change_no_bit(counts, N, K):
+    from llmx_amd import ops
+    X = 40
+    gen = torch.Generator().manual_seed(N + K)
+    if counts == "even":
+        n = [120 + i % 17 for i in range(X)]
+    elif counts == "uneven":
+        n = [(0, 1, 64, 65, 128, 129, 300, 777)[i % 8] for i in range(X)]
+    else:
+        n = [0] * X
+        n[3], n[39] = 4095, 1
+    P = sum(n)
+    ids = torch.repeat_interleave(torch.arange(X), torch.tensor(n))[torch.randperm(P, generator=gen)].to(torch.int32).view(P, 1).to(DEV)
+    held, offsets, active = (torch.zeros(m, dtype=torch.int32, device=DEV) for m in (X, X + 1, X))
+    pairs, n_active, ticket, stats = (torch.full((m,), -7, dtype=torch.int32, device=DEV) for m in (P, 1, 1, 2))
+    ops.moe_align(ids, X, held, offsets, pairs, active, n_active, tile_stats=stats, ticket=ticket)
+    assert int(ticket) == 0
+    a = torch.randn(P, K, generator=gen).to(DEV, torch.bfloat16)
+    w = (torch.randn(X, N, K, generator=gen) * 0.05).to(DEV, torch.bfloat16)
+    for choice in (15, int(stats[1])):
+        stats[1] = choice
+        for epi, shape, dtype in ((ops.EPI_STORE, N, torch.float32), (ops.EPI_SWIGLU, N // 2, torch.bfloat16)):
+            want, got = (torch.full((P, shape), float("nan"), dtype=dtype, device=DEV) for _ in range(2))
+            ops.grouped_gemm(a, w, want, offsets, pairs, 1, epi, tile_stats=stats)
+            for _ in range(2):
+                got.fill_(float("nan"))
+                ops.grouped_gemm(a, w, got, offsets, pairs, 1, epi, tile_stats=stats, ticket=ticket)
+                assert int(ticket) == 0
+                assert torch.equal(got, want)
+            if epi == ops.EPI_STORE:
+                rows = pairs[int(offsets[3]):int(offsets[3]) + 64].long()
+                exact = a[rows].double() @ w[3].double().T
+                # float32 sums of K exact products of random sign
+                assert (got[rows].double() - exact).abs().max() <= 4 * 2.0 ** -24 * K ** 0.5 * exact.abs().max() * 4
