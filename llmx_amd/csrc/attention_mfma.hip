@@ -257,13 +257,20 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     for (int dt = 0; dt < (PARTIAL ? 1 : DT); ++dt) o_tot[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     float m_tot = -INFINITY, l_tot = 0.0f;   // the segments folded so far (slot < 0)
 
-    // the pages of a segment's 8 tiles of 16 keys (-1: the tile holds no key of the item) and the tiles' places in them;
-    // a cursor steps from tile to tile, so that nothing is divided
+    // the pages of a segment's 8 tiles of 16 keys and the tiles' places in them; a cursor steps from tile to tile, so that nothing is divided.
+    // A tile that holds no key of the item (`missing`, a bit a tile) stands at the page of the request's last token instead: its keys
+    // do not count, and no load sits behind a condition (with one at each load a wave waited for all it had asked for before it went on: 64
+    // requests of 1,280 tokens, 512 waves, 84 us and now 74.5; many waves of a segment each hide that among themselves, 35.8 and 35.8)
+    const int own_page = table[p_last / bt];
     int cur_blk = key_begin / bt, cur_sub = key_begin % bt, cur_key = key_begin;
-    auto locate = [&](int (&pages)[8], int (&subs)[8]) {
+    auto locate = [&](int (&pages)[8], int (&subs)[8], int& missing) {
+        missing = 0;
 #pragma unroll
         for (int tl = 0; tl < 8; ++tl) {
-            pages[tl] = cur_key < key_end ? table[cur_blk] : -1;
+            const int page = table[cur_key < key_end ? cur_blk : 0];
+            const bool none = cur_key >= key_end || page < 0;
+            pages[tl] = none ? own_page : page;
+            missing |= none ? 1 << tl : 0;
             subs[tl] = cur_sub;
             cur_key += 16;
             cur_sub += 16;
@@ -276,15 +283,16 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     // K fragments of chunk v of the segment: lane (row c of each score tile: key chunk_key(u, c) of the chunk, which
     // lies in the chunk's second 16 keys (their own page) from row 8 on; dims 32s + 8g ..)
     auto load_keys = [&](const int (&pages)[8], const int (&subs)[8], int v, bf16x8_t (&kf)[2][QS]) {
+        const int page = c >= 8 ? pages[2 * v + 1] : pages[2 * v];
+        const int sub = c >= 8 ? subs[2 * v + 1] : subs[2 * v];
+        const bf16_t* base = a.k_cache + (((size_t)page * Hkv + kvh) * bt + sub) * D + 8 * g;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            const int page = c >= 8 ? pages[2 * v + 1] : pages[2 * v];
-            const int sub = c >= 8 ? subs[2 * v + 1] : subs[2 * v];
-            const bf16_t* src = a.k_cache + (((size_t)(page < 0 ? 0 : page) * Hkv + kvh) * bt + sub + (chunk_key(u, c) & 15)) * D + 8 * g;
+            const bf16_t* src = base + (chunk_key(u, c) & 15) * D;
 #pragma unroll
             for (int s = 0; s < QS; ++s) {
                 u32x4_t x = {0u, 0u, 0u, 0u};
-                if (page >= 0 && frag_in<DT>(s, g)) x = *reinterpret_cast<const u32x4_t*>(src + 32 * s);
+                if (frag_in<DT>(s, g)) x = *reinterpret_cast<const u32x4_t*>(src + 32 * s);
                 kf[u][s] = __builtin_bit_cast(bf16x8_t, x);
             }
         }
@@ -294,56 +302,64 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     auto load_values = [&](const int (&pages)[8], const int (&subs)[8], int v, bf16x8_t (&vf)[DT]) {
         const int page = g >= 2 ? pages[2 * v + 1] : pages[2 * v];
         const int sub = g >= 2 ? subs[2 * v + 1] : subs[2 * v];
-        const bf16_t* src = a.v_cache + (((size_t)(page < 0 ? 0 : page) * Hkv + kvh) * D + c) * bt + sub + 8 * (g & 1);
+        const bf16_t* src = a.v_cache + (((size_t)page * Hkv + kvh) * D + c) * bt + sub + 8 * (g & 1);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            u32x4_t x = {0u, 0u, 0u, 0u};
-            if (page >= 0) x = *reinterpret_cast<const u32x4_t*>(src + (size_t)16 * dt * bt);
-            vf[dt] = __builtin_bit_cast(bf16x8_t, x);
-        }
+        for (int dt = 0; dt < DT; ++dt) vf[dt] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(src + (size_t)16 * dt * bt));
     };
 
     if (key_begin >= key_end) return;
-    int pages[8], subs[8], pages_next[8], subs_next[8];
-    locate(pages, subs);
+    int pages[8], subs[8], pages_next[8], subs_next[8], missing, missing_next;
+    locate(pages, subs, missing);
     // Two chunks' loads are always on their way: keys in two register sets that take turns, values in two more.  The
     // first two value chunks of a segment are asked for before its scores are formed, the first two key chunks of the
     // next segment while its last values are multiplied.
     bf16x8_t kf_a[2][QS], kf_b[2][QS];
     load_keys(pages, subs, 0, kf_a);
     load_keys(pages, subs, 1, kf_b);
-    for (int seg0 = key_begin; seg0 < key_end; seg0 += AM_SEG) {
-        locate(pages_next, subs_next);   // the next segment's pages are looked up while this one is worked on
+    auto segment = [&](int seg0, auto is_last) {      // the last segment asks for no keys of a next one
+        constexpr bool LAST = decltype(is_last)::value;
+        if (!LAST) locate(pages_next, subs_next, missing_next);   // the next segment's pages are looked up while this one is worked on
         bf16x8_t vf_a[DT], vf_b[DT];
         load_values(pages, subs, 0, vf_a);
         load_values(pages, subs, 1, vf_b);
         f32x4_t s[8];
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_a, qf, s[0], s[1]);
+        __builtin_amdgcn_sched_barrier(0);
         load_keys(pages, subs, 2, kf_a);
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_b, qf, s[2], s[3]);
+        __builtin_amdgcn_sched_barrier(0);
         load_keys(pages, subs, 3, kf_b);
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_a, qf, s[4], s[5]);
-        load_keys(pages_next, subs_next, 0, kf_a);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!LAST) load_keys(pages_next, subs_next, 0, kf_a);
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_b, qf, s[6], s[7]);
-        load_keys(pages_next, subs_next, 1, kf_b);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!LAST) load_keys(pages_next, subs_next, 1, kf_b);
+        __builtin_amdgcn_sched_barrier(0);
         float m, l;
         bf16x8_t pf[4];
-        bool all_in = true;
-#pragma unroll
-        for (int tl = 0; tl < 8; ++tl) all_in = all_in && pages[tl] >= 0;
-        if (seg0 + AM_SEG - 1 <= p_first && seg0 >= lo_last && all_in) {
+        if (seg0 + AM_SEG - 1 <= p_first && seg0 >= lo_last && missing == 0) {
             segment_softmax<false>(s, 0xffffffffu, a.scale, m, l, pf);   // every key counts for every column
         } else {
-            // (a tile without a page lies wholly at or after key_end, which the mask leaves out)
+            // (a tile without a page lies wholly at or after key_end, or before the window, which the mask leaves out)
             segment_softmax<true>(s, segment_mask(seg0, g, col_ok, lo_col, p_col, key_end), a.scale, m, l, pf);
         }
         f32x4_t o[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        __builtin_amdgcn_sched_barrier(0);
         chunk_values<DT>(vf_a, pf[0], o);
+        __builtin_amdgcn_sched_barrier(0);
         load_values(pages, subs, 2, vf_a);
+        __builtin_amdgcn_sched_barrier(0);
         chunk_values<DT>(vf_b, pf[1], o);
+        __builtin_amdgcn_sched_barrier(0);
         load_values(pages, subs, 3, vf_b);
+        __builtin_amdgcn_sched_barrier(0);
         chunk_values<DT>(vf_a, pf[2], o);
         chunk_values<DT>(vf_b, pf[3], o);
         if constexpr (PARTIAL) {
@@ -360,12 +376,17 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
         } else {
             fold_segment<DT>(o, m, l, o_tot, m_tot, l_tot);
         }
+        if (LAST) return;
 #pragma unroll
         for (int tl = 0; tl < 8; ++tl) {
             pages[tl] = pages_next[tl];
             subs[tl] = subs_next[tl];
         }
-    }
+        missing = missing_next;
+    };
+    int seg0 = key_begin;
+    for (; seg0 + AM_SEG < key_end; seg0 += AM_SEG) segment(seg0, std::false_type{});
+    segment(seg0, std::true_type{});
     if constexpr (!PARTIAL) {
         if (col_ok) store_output<DT>(a.out + ((size_t)t * a.n_heads + h) * D, g, o_tot, l_tot, head_gate_factor(a.gate, a.gate_ld, a.gate_wide, t, h),
                                 value_gates(a.gate, a.gate_ld, a.gate_wide, t, h, D));
@@ -426,33 +447,31 @@ __global__ void __launch_bounds__(256) paged_attention_split4_kernel(AttnMfmaArg
         bf16x8_t kf[2][QS];
         bf16x8_t vf[4][2];
     };
+    const int own_page = table[p_last / bt];      // stands for a tile without one, as in the kernel above
     auto fetch = [&](int seg0, Loaded& x) {
         int pages[8], subs[8];
 #pragma unroll
         for (int tl = 0; tl < 8; ++tl) {
             const int key0 = seg0 + 16 * tl;
             const bool in = key0 < key_end;
-            pages[tl] = in ? table[key0 / bt] : -1;
+            const int page = table[in ? key0 / bt : 0];
+            pages[tl] = in && page >= 0 ? page : own_page;
             subs[tl] = key0 % bt;
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             // row c of score tile u of chunk `wave`: key chunk_key(u, c), in the chunk's first (rows below 8) or second
             // 16 keys; the page selected without indexing the arrays by a run-time value
-            int page = -1, sub = 0;
+            int page = own_page, sub = 0;
 #pragma unroll
             for (int tl = 0; tl < 8; ++tl)
                 if (tl == 2 * wave + (c >= 8 ? 1 : 0)) {
                     page = pages[tl];
                     sub = subs[tl];
                 }
-            const bf16_t* src = a.k_cache + (((size_t)(page < 0 ? 0 : page) * Hkv + kvh) * bt + sub + (chunk_key(u, c) & 15)) * D + 8 * g;
+            const bf16_t* src = a.k_cache + (((size_t)page * Hkv + kvh) * bt + sub + (chunk_key(u, c) & 15)) * D + 8 * g;
 #pragma unroll
-            for (int s = 0; s < QS; ++s) {
-                u32x4_t v = {0u, 0u, 0u, 0u};
-                if (page >= 0) v = *reinterpret_cast<const u32x4_t*>(src + 32 * s);
-                x.kf[u][s] = __builtin_bit_cast(bf16x8_t, v);
-            }
+            for (int s = 0; s < QS; ++s) x.kf[u][s] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(src + 32 * s));
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -461,10 +480,8 @@ __global__ void __launch_bounds__(256) paged_attention_split4_kernel(AttnMfmaArg
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int dim = 32 * wave + 16 * q + c;
-                const bf16_t* src = a.v_cache + (((size_t)(page < 0 ? 0 : page) * Hkv + kvh) * D + dim) * bt + sub + 8 * (g & 1);
-                u32x4_t both = {0u, 0u, 0u, 0u};
-                if (page >= 0) both = *reinterpret_cast<const u32x4_t*>(src);
-                x.vf[v][q] = __builtin_bit_cast(bf16x8_t, both);
+                const bf16_t* src = a.v_cache + (((size_t)page * Hkv + kvh) * D + dim) * bt + sub + 8 * (g & 1);
+                x.vf[v][q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(src));
             }
         }
     };
