@@ -165,68 +165,74 @@ __device__ __forceinline__ float strided_squares(const float* __restrict__ row, 
 // r = 1 / sqrt(mean(x^2) + eps).  The norm kernels use 1,024 threads: thread v adds the squares of elements v, v + 1024,
 // ... in this order with fmaf, each wave of 64 threads adds its threads' sums with wave_sum, and the 16 waves' sums are
 // added in wave order.  Here a workgroup of NW waves does the same: wave w stands for the waves w, w + NW, ... of that
-// block.  store(row, i, y) receives every element.  Rows of at most 4,096 values with at least 4 waves are kept in
-// registers, all asked for (with the weights) before anything is added, so the workgroup waits for memory once a row.
+// block.  store(row, i, y) receives every element.  Rows of at most 4,096 values with at least 4 waves, of 1,024 with fewer, are kept in
+// registers (256 values, one wave: a product's launch 8.5 -> 7.1 us), all asked for (with the weights) before anything is added, so the workgroup waits for memory once a row.
 // scratch32: 32 floats of LDS.  The caller puts a barrier between the stores and their first read.
 // meanwhile(): called once, when the first row's values are on their way (or before them, for rows that are not kept): what the caller
 // asks memory for beside the norm goes there, behind what the norm waits for.
 struct NothingMeanwhile {
     __device__ __forceinline__ void operator()() const {}
 };
-template <int NW, typename Store, typename Meanwhile = NothingMeanwhile>
-__device__ __forceinline__ void rms_rows_as_1024(const float* __restrict__ X, size_t ldx, int rows, int n, const float* __restrict__ w,
-                                                 float eps, float* scratch32, Store store, Meanwhile meanwhile = Meanwhile()) {
-    static_assert(NW == 1 || NW == 2 || NW == 4 || NW == 8 || NW == 16, "waves of the workgroup");
+template <int NW, int KEPT, typename Store, typename Meanwhile>
+__device__ __forceinline__ void rms_rows_kept(const float* __restrict__ X, size_t ldx, int rows, int n, const float* __restrict__ w,
+                                              float eps, float* scratch32, Store store, Meanwhile meanwhile) {
     constexpr int VW = 16 / NW;       // waves of the 1,024-thread block that one wave stands for
-    constexpr int KEPT = 4;
     const int wave = threadIdx.x / LLMX_WAVE, lane = threadIdx.x & (LLMX_WAVE - 1);
-    if (VW * KEPT <= 16 && n <= 1024 * KEPT) {
-        float nw[VW][KEPT];
+    float nw[VW][KEPT];
+#pragma unroll
+    for (int j = 0; j < VW; ++j)
+#pragma unroll
+        for (int e = 0; e < KEPT; ++e) {
+            const int i = (wave + j * NW) * LLMX_WAVE + lane + e * 1024;
+            nw[j][e] = i < n ? w[i] : 0.0f;
+        }
+    for (int row = 0; row < rows; ++row) {
+        const float* x = X + (size_t)row * ldx;
+        float* scratch = scratch32 + 16 * (row & 1);   // rows take turns in two sets, so one barrier a row is enough
+        float v[VW][KEPT];
 #pragma unroll
         for (int j = 0; j < VW; ++j)
 #pragma unroll
             for (int e = 0; e < KEPT; ++e) {
                 const int i = (wave + j * NW) * LLMX_WAVE + lane + e * 1024;
-                nw[j][e] = i < n ? w[i] : 0.0f;
+                v[j][e] = i < n ? x[i] : 0.0f;
             }
-        for (int row = 0; row < rows; ++row) {
-            const float* x = X + (size_t)row * ldx;
-            float* scratch = scratch32 + 16 * (row & 1);   // rows take turns in two sets, so one barrier a row is enough
-            float v[VW][KEPT];
-#pragma unroll
-            for (int j = 0; j < VW; ++j)
-#pragma unroll
-                for (int e = 0; e < KEPT; ++e) {
-                    const int i = (wave + j * NW) * LLMX_WAVE + lane + e * 1024;
-                    v[j][e] = i < n ? x[i] : 0.0f;
-                }
-            if (row == 0) {
-                __builtin_amdgcn_sched_barrier(0);
-                meanwhile();
-                __builtin_amdgcn_sched_barrier(0);
-            }
-#pragma unroll
-            for (int j = 0; j < VW; ++j) {
-                float sq = 0.0f;     // an element past the end adds fmaf(0, 0, s) = s
-#pragma unroll
-                for (int e = 0; e < KEPT; ++e) sq = fmaf(v[j][e], v[j][e], sq);
-                sq = wave_sum(sq);
-                if (lane == 0) scratch[wave + j * NW] = sq;
-            }
-            __syncthreads();
-            float s = scratch[0];
-#pragma unroll
-            for (int u = 1; u < 16; ++u) s += scratch[u];
-            const float scale = 1.0f / sqrtf(s / (float)n + eps);
-#pragma unroll
-            for (int j = 0; j < VW; ++j)
-#pragma unroll
-                for (int e = 0; e < KEPT; ++e) {
-                    const int i = (wave + j * NW) * LLMX_WAVE + lane + e * 1024;
-                    if (i < n) store(row, i, v[j][e] * (scale * nw[j][e]));
-                }
+        if (row == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            meanwhile();
+            __builtin_amdgcn_sched_barrier(0);
         }
-        return;
+#pragma unroll
+        for (int j = 0; j < VW; ++j) {
+            float sq = 0.0f;     // an element past the end adds fmaf(0, 0, s) = s
+#pragma unroll
+            for (int e = 0; e < KEPT; ++e) sq = fmaf(v[j][e], v[j][e], sq);
+            sq = wave_sum(sq);
+            if (lane == 0) scratch[wave + j * NW] = sq;
+        }
+        __syncthreads();
+        float s = scratch[0];
+#pragma unroll
+        for (int u = 1; u < 16; ++u) s += scratch[u];
+        const float scale = 1.0f / sqrtf(s / (float)n + eps);
+#pragma unroll
+        for (int j = 0; j < VW; ++j)
+#pragma unroll
+            for (int e = 0; e < KEPT; ++e) {
+                const int i = (wave + j * NW) * LLMX_WAVE + lane + e * 1024;
+                if (i < n) store(row, i, v[j][e] * (scale * nw[j][e]));
+            }
+    }
+}
+template <int NW, typename Store, typename Meanwhile = NothingMeanwhile>
+__device__ __forceinline__ void rms_rows_as_1024(const float* __restrict__ X, size_t ldx, int rows, int n, const float* __restrict__ w,
+                                                 float eps, float* scratch32, Store store, Meanwhile meanwhile = Meanwhile()) {
+    static_assert(NW == 1 || NW == 2 || NW == 4 || NW == 8 || NW == 16, "waves of the workgroup");
+    const int wave = threadIdx.x / LLMX_WAVE, lane = threadIdx.x & (LLMX_WAVE - 1);
+    if constexpr (NW >= 4) {
+        if (n <= 4096) return rms_rows_kept<NW, 4>(X, ldx, rows, n, w, eps, scratch32, store, meanwhile);
+    } else {
+        if (n <= 1024) return rms_rows_kept<NW, 1>(X, ldx, rows, n, w, eps, scratch32, store, meanwhile);
     }
     meanwhile();
     for (int row = 0; row < rows; ++row) {

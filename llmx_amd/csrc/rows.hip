@@ -102,13 +102,20 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(float* __restrict__ x,
     const float old = accumulate ? *o : 0.0f;
     float s = 0.0f;
     for (int j0 = 0; j0 < k; j0 += 8) {
-        // the slots' rows are asked for whether or not a slot has an expert (its row exists either way), so nothing waits for the ids
-        float yv[8];
+        // the slots' rows, ids and weights are asked for together, whether or not a slot has an expert (its row exists either way), a slot past
+        // the last as the last: nothing waits for anything else
+        float yv[8], wv[8];
+        int id[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) yv[u] = j0 + u < k ? y[((size_t)t * k + j0 + u) * width + i] : 0.0f;
+        for (int u = 0; u < 8; ++u) {
+            const int j = t * k + min(j0 + u, k - 1);
+            id[u] = ids[j];
+            wv[u] = w ? w[j] : 1.0f;
+            yv[u] = y[(size_t)j * width + i];
+        }
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            if (j0 + u < k && ids[t * k + j0 + u] >= 0) s += (w ? w[t * k + j0 + u] : 1.0f) * yv[u];
+            if (j0 + u < k && id[u] >= 0) s += wv[u] * yv[u];
     }
     *o = accumulate ? old + s : s;
 }
