@@ -447,31 +447,33 @@ __global__ void __launch_bounds__(256) paged_attention_split4_kernel(AttnMfmaArg
         bf16x8_t kf[2][QS];
         bf16x8_t vf[4][2];
     };
-    const int own_page = table[p_last / bt];      // stands for a tile without one, as in the kernel above
     auto fetch = [&](int seg0, Loaded& x) {
         int pages[8], subs[8];
 #pragma unroll
         for (int tl = 0; tl < 8; ++tl) {
             const int key0 = seg0 + 16 * tl;
             const bool in = key0 < key_end;
-            const int page = table[in ? key0 / bt : 0];
-            pages[tl] = in && page >= 0 ? page : own_page;
+            pages[tl] = in ? table[key0 / bt] : -1;
             subs[tl] = key0 % bt;
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             // row c of score tile u of chunk `wave`: key chunk_key(u, c), in the chunk's first (rows below 8) or second
             // 16 keys; the page selected without indexing the arrays by a run-time value
-            int page = own_page, sub = 0;
+            int page = -1, sub = 0;
 #pragma unroll
             for (int tl = 0; tl < 8; ++tl)
                 if (tl == 2 * wave + (c >= 8 ? 1 : 0)) {
                     page = pages[tl];
                     sub = subs[tl];
                 }
-            const bf16_t* src = a.k_cache + (((size_t)page * Hkv + kvh) * bt + sub + (chunk_key(u, c) & 15)) * D + 8 * g;
+            const bf16_t* src = a.k_cache + (((size_t)(page < 0 ? 0 : page) * Hkv + kvh) * bt + sub + (chunk_key(u, c) & 15)) * D + 8 * g;
 #pragma unroll
-            for (int s = 0; s < QS; ++s) x.kf[u][s] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(src + 32 * s));
+            for (int s = 0; s < QS; ++s) {
+                u32x4_t v = {0u, 0u, 0u, 0u};
+                if (page >= 0) v = *reinterpret_cast<const u32x4_t*>(src + 32 * s);
+                x.kf[u][s] = __builtin_bit_cast(bf16x8_t, v);
+            }
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -480,8 +482,10 @@ __global__ void __launch_bounds__(256) paged_attention_split4_kernel(AttnMfmaArg
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int dim = 32 * wave + 16 * q + c;
-                const bf16_t* src = a.v_cache + (((size_t)page * Hkv + kvh) * D + dim) * bt + sub + 8 * (g & 1);
-                x.vf[v][q] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(src));
+                const bf16_t* src = a.v_cache + (((size_t)(page < 0 ? 0 : page) * Hkv + kvh) * D + dim) * bt + sub + 8 * (g & 1);
+                u32x4_t both = {0u, 0u, 0u, 0u};
+                if (page >= 0) both = *reinterpret_cast<const u32x4_t*>(src);
+                x.vf[v][q] = __builtin_bit_cast(bf16x8_t, both);
             }
         }
     };
