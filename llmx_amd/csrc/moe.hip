@@ -514,7 +514,7 @@ __global__ void __launch_bounds__(1024) moe_chunk_scan_kernel(int n_chunks, int 
             experts += wave_active[w];
         }
         tiles128[0] = n128;
-        if (choice) *choice = tile_choice(n_pairs, n128, n64, experts);
+        if (choice) *choice = ticket ? tile_choice_tickets(n_pairs, n128, n64, experts) : tile_choice(n_pairs, n128, n64, experts);
     }
     for (int w = 0; w < wave; ++w) {
         before += wave_total[w];
@@ -557,11 +557,13 @@ __global__ void __launch_bounds__(1024) moe_chunk_place_kernel(const int* __rest
 }
 
 extern "C" int llmx_tile_choice(int n_pairs, int n128, int n64, int experts) { return tile_choice(n_pairs, n128, n64, experts); }
+extern "C" int llmx_tile_choice_tickets(int n_pairs, int n128, int n64, int experts) { return tile_choice_tickets(n_pairs, n128, n64, experts); }
 
 // counts [X], offsets [X+1], list [n_pairs], active [X], n_active [1]
 // scratch (optional): [ceil(n_pairs / 1024) * n_experts] ints for steps of many pairs
 // tiles128 (optional) [1]: with scratch and many pairs, the sum over experts of ceil(rows / 128); choice (optional, with tiles128):
-// which routed products take tiles of 128 rows, a bit a class of K (tile_choice.h); ticket (optional) [1], with scratch and many pairs: set to 0
+// which routed products take tiles of 128 rows, a bit a class of K (tile_choice.h); ticket (optional) [1], with scratch and many pairs: set to 0, and
+// the choice is the one for products that take tiles by it
 extern "C" int llmx_moe_align_ticket(const int* ids, int n_pairs, int n_experts, int* counts, int* offsets, int* list, int* active, int* n_active,
                                      int* scratch, int* tiles128, int* choice, int* ticket, hipStream_t stream) {
     if (n_pairs <= 0 || n_experts <= 0) return 0;

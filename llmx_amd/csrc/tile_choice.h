@@ -24,3 +24,12 @@ __host__ __device__ inline int tile_choice(long n_pairs, long n128, long n64, lo
     const bool wide = ratio || (weighed && n_pairs <= 132 * experts), four = 10 * n64 >= 16 * n128;
     return (wide ? 1 : 0) | (wide && experts <= 128 ? 2 : 0) | (four || (2 * n64 >= 3 * n128 && n_pairs <= 80 * experts) ? 4 : 0) | (four ? 8 : 0);
 }
+
+// The choice where the products' workgroups take tiles by tickets.  A tile of 128 then costs what it has rows for, in halves, and its
+// lookup and first loads are covered, so that it is the better one up to some 130 rows an expert, and for K of 1,536 on to 200 (256
+// experts, tiles of 128 and of 64, us: 3,072 features of 3,072 values, 16 rows an expert 756 and 762, 45 817 and 855, 60 853 and 970, 130
+// 1,345 and 1,420, but 170 1,654 and 1,592; of 1,536 values 32 rows 486 and 488, 52 504 and 540, 130 761 and 797, 170 923 and 907; 2,048 features
+// of 2,048 values 20 rows 447 and 467, 60 497 and 532).  Beyond that, and for shorter K, as above.
+__host__ __device__ inline int tile_choice_tickets(long n_pairs, long n128, long n64, long experts) {
+    return tile_choice(n_pairs, n128, n64, experts) | (n_pairs <= 132 * experts ? 7 : n_pairs <= 200 * experts ? 4 : 0);
+}

@@ -118,6 +118,7 @@ def _declare(h) -> None:
         "llmx_argmax_rows": [P, P, P, P, I, I, P],
         "llmx_gemm_skinny_f32": [P, P, P, I, I, I, I, I, I, I, I, L, P, F, P],
         "llmx_tile_choice": [I, I, I, I],
+        "llmx_tile_choice_tickets": [I, I, I, I],
         "llmx_gemm_tile": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_chosen": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_tickets": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, P, I, P, I, F, P, P, I, P],
@@ -1684,7 +1685,7 @@ def moe_align(ids: torch.Tensor, n_experts: int, counts: torch.Tensor, offsets: 
     steps of many pairs (made here when it is not given).  `tile_stats` int32 [1]: for TILE_STATS_MIN_PAIRS pairs or
     more it receives the sum over experts of ceil(rows / 128), by which grouped_gemm chooses its tile size; int32 [2]: behind it
     the choice itself, from the tiles of both sizes and the experts that have rows, a bit a class of K, which grouped_gemm then follows.
-    `ticket` int32 [1]: set to 0 for grouped_gemm where moe_align_scratch(...) is not 0."""
+    `ticket` int32 [1]: set to 0 for grouped_gemm where moe_align_scratch(...) is not 0; the choice is then the one for it."""
     n_pairs = ids.numel()
     need = moe_align_scratch(n_pairs, n_experts)
     if need and scratch is None:

@@ -24,10 +24,12 @@ def test_tickets_change_no_bit(counts, N, K):
         n[3], n[39] = 4095, 1
     P = sum(n)
     ids = torch.repeat_interleave(torch.arange(X), torch.tensor(n))[torch.randperm(P, generator=gen)].to(torch.int32).view(P, 1).to(DEV)
-    held, offsets, active = (torch.zeros(m, dtype=torch.int32, device=DEV) for m in (X, X + 1, X))
+    found, offsets, active = (torch.zeros(m, dtype=torch.int32, device=DEV) for m in (X, X + 1, X))
     pairs, n_active, ticket, stats = (torch.full((m,), -7, dtype=torch.int32, device=DEV) for m in (P, 1, 1, 2))
-    ops.moe_align(ids, X, held, offsets, pairs, active, n_active, tile_stats=stats, ticket=ticket)
+    ops.moe_align(ids, X, found, offsets, pairs, active, n_active, tile_stats=stats, ticket=ticket)
     assert int(ticket) == 0
+    held = [c for c in n if c]
+    assert int(stats[1]) == ops.lib().llmx_tile_choice_tickets(P, sum(-(-c // 128) for c in n), sum(-(-c // 64) for c in n), len(held))
     a = torch.randn(P, K, generator=gen).to(DEV, torch.bfloat16)
     w = (torch.randn(X, N, K, generator=gen) * 0.05).to(DEV, torch.bfloat16)
     for choice in (15, int(stats[1])):
