@@ -207,8 +207,9 @@ class RoutedExperts(FeedForward):
         scratch = step.buf("experts.align_scratch", (need,), torch.int32) if need else None
         # for steps of many pairs the grouping also counts the experts' tiles of 128 rows, by which the products choose their tiles
         tile_stats = step.buf("experts.tile_stats", (2,), torch.int32) if T * slots >= ops.TILE_STATS_MIN_PAIRS else None
-        # ... and readies the counter by which the products' workgroups take tile after tile
-        ticket = step.buf("experts.ticket", (1,), torch.int32) if tile_stats is not None and need else None
+        # ... and readies the counter by which the products' workgroups take tile after tile (both products can: silu(gate) * up, nothing on the input)
+        bare = self.plain_unit is None and self.unit == ops.GLU_SILU and self.weight_on == "output"
+        ticket = step.buf("experts.ticket", (1,), torch.int32) if tile_stats is not None and need and bare else None
         ops.route_topk_align(z, self.bias, ids, weights, k, self.score, self.normalize, self.scale, counts, offsets, pairs, active, n_active,
                              parts=parts, scratch=scratch, tile_stats=tile_stats, logit_bias=self.logit_bias, groups=self.groups, ticket=ticket)
         step.observe("routing", logits=z, ids=ids[:, :k], weights=weights[:, :k])
