@@ -277,8 +277,8 @@ struct StateScanArgs {
     int ldq, ldk, ldv, ldg;
     float* state;
     long state_stride;
-    const int* slot_read;
-    const int* slot_write;
+    const int* slot_read;      // where an entry's state is read, and where it is left: entries run in no order, so that no slot written may be
+    const int* slot_write;     // one that another entry reads
     const int* entry_rows;
     float* out;          // [T, H*V]
     float out_scale;

@@ -839,7 +839,8 @@ def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.T
     u = beta (v - S^T k) (u = v without beta); S <- S + k u^T; out = out_scale * S^T q.  q, k [T, qk_heads*D], v [T, H*V],
     decay [T, H*D] are float32 views whose rows may be columns of wider tensors; state [slots, width] float32 holds S at
     its start in tiles of 8 value channels ([H, ceil(V / 8), D, 8]: `state_matrix_size`, `state_matrix_tiled`), read at
-    slot_read[e], written at slot_write[e].  `max_rows`: the most rows an entry has, when the caller knows it (steps of
+    slot_read[e], written at slot_write[e]: entries are worked on in no order, so no entry may write a slot that another one reads
+    (so for everything below and above that takes both).  `max_rows`: the most rows an entry has, when the caller knows it (steps of
     single tokens stage smaller chunks; the results are the same).  `tail` = (source [T, C] view, taps, offset):
     the convolution tail [taps - 1, C] at `offset` of the state is handed on from the step's rows of `source`.  `operands`: what
     is made of q, k and v as they are read (None: nothing).  `max_rows_here` > 0: entries of more rows are left alone (another

@@ -94,6 +94,8 @@ def test_join_of_two_results_and_logit_cap():
 def _delta_case(seed, H, G, D, V, taps, entries, slots_read, slots_write, n_slots=6, max_rows=0):
     """Runs delta_prep + state_scan + head_norm_gate over a step whose entries have `entries` rows each, from random
     states; returns everything the plain functions need and what the kernels gave."""
+    # the entries of a launch are not ordered: a slot that one of them writes may be read by itself alone
+    assert all(r != w for i, r in enumerate(slots_read) for j, w in enumerate(slots_write) if i != j) and len(set(slots_write)) == len(slots_write)
     rng = np.random.default_rng(seed)
     o = ops()
     T = sum(entries)
@@ -156,7 +158,7 @@ def test_delta_rule_rows_states_slots_and_the_convolution_tail(sizes):
     """Entries of 1, 2 (fewer than the taps: the tail is shifted), 9 and 40 rows read their state and tail at one slot and
     write them at another (and in place); slots of no entry are untouched."""
     H, G, D, V, taps = sizes
-    whole = _delta_case(1, H, G, D, V, taps, [9, 1, 2, 40], [0, 2, 4, 5], [1, 3, 4, 0])
+    whole = _delta_case(1, H, G, D, V, taps, [9, 1, 2, 40], [0, 2, 4, 5], [1, 3, 4, 6], n_slots=8)
     # steps of one or two rows an entry take smaller chunks: the same bits as the rows get in the larger ones
     short = _delta_case(2, H, G, D, V, taps, [1, 2, 1], [0, 2, 4], [1, 3, 4], max_rows=2)
     assert torch.equal(short, _delta_case(2, H, G, D, V, taps, [1, 2, 1], [0, 2, 4], [1, 3, 4]))
