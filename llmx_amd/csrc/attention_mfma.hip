@@ -258,26 +258,27 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     float m_tot = -INFINITY, l_tot = 0.0f;   // the segments folded so far (slot < 0)
 
     // the pages of a segment's 8 tiles of 16 keys and the tiles' places in them; a cursor steps from tile to tile, so that nothing is divided.
-    // A tile that holds no key of the item (`missing`, a bit a tile) stands at the page of the request's last token instead: its keys
-    // do not count, and no load sits behind a condition (with one at each load a wave waited for all it had asked for before it went on: 64
-    // requests of 1,280 tokens, 512 waves, 84 us and now 74.5; many waves of a segment each hide that among themselves, 35.8 and 35.8)
-    const int own_page = table[p_last / bt];
+    // A tile that holds no key of the item (`missing`, a bit a tile) stands at the tile of the request's last token instead: its keys do not
+    // count, what is read was written by the request (0 times an infinity that an ended request left in a page's unwritten tiles would not be
+    // 0), and no load sits behind a condition (with one at each load a wave waited for all it had asked for before it went on: 64 requests of
+    // 1,280 tokens, 512 waves, 84 us and now 74.5; many waves of a segment each hide that among themselves, 35.8 and 35.8)
+    const int own_blk = p_last / bt, own_page = table[own_blk], own_sub = p_last % bt & ~15, own_key = p_last & ~15;
     int cur_blk = key_begin / bt, cur_sub = key_begin % bt, cur_key = key_begin;
     auto locate = [&](int (&pages)[8], int (&subs)[8], int& missing) {
         missing = 0;
 #pragma unroll
         for (int tl = 0; tl < 8; ++tl) {
-            const int page = table[cur_key < key_end ? cur_blk : 0];
-            const bool none = cur_key >= key_end || page < 0;
-            pages[tl] = none ? own_page : page;
-            missing |= none ? 1 << tl : 0;
-            subs[tl] = cur_sub;
-            cur_key += 16;
+            const bool past = cur_key > own_key;
+            const int page = table[past ? own_blk : cur_blk], sub = past ? own_sub : cur_sub;
+            pages[tl] = page < 0 ? own_page : page;
+            subs[tl] = page < 0 ? own_sub : sub;
+            missing |= past || page < 0 ? 1 << tl : 0;
             cur_sub += 16;
             if (cur_sub >= bt) {
                 cur_sub = 0;
                 ++cur_blk;
             }
+            cur_key += 16;
         }
     };
     // K fragments of chunk v of the segment: lane (row c of each score tile: key chunk_key(u, c) of the chunk, which
