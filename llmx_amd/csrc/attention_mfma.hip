@@ -262,17 +262,17 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     // count, what is read was written by the request (0 times an infinity that an ended request left in a page's unwritten tiles would not be
     // 0), and no load sits behind a condition (with one at each load a wave waited for all it had asked for before it went on: 64 requests of
     // 1,280 tokens, 512 waves, 84 us and now 74.5; many waves of a segment each hide that among themselves, 35.8 and 35.8)
-    const int own_blk = p_last / bt, own_page = table[own_blk], own_sub = p_last % bt & ~15, own_key = p_last & ~15;
+    const int own_blk = p_last / bt, own_page = table[own_blk], own_sub = p_last % bt & ~15;
     int cur_blk = key_begin / bt, cur_sub = key_begin % bt, cur_key = key_begin;
     auto locate = [&](int (&pages)[8], int (&subs)[8], int& missing) {
         missing = 0;
 #pragma unroll
         for (int tl = 0; tl < 8; ++tl) {
-            const bool past = cur_key > own_key;
-            const int page = table[past ? own_blk : cur_blk], sub = past ? own_sub : cur_sub;
-            pages[tl] = page < 0 ? own_page : page;
-            subs[tl] = page < 0 ? own_sub : sub;
-            missing |= past || page < 0 ? 1 << tl : 0;
+            const int page = table[min(cur_blk, own_blk)];
+            const bool none = cur_key >= key_end || page < 0;
+            pages[tl] = none ? own_page : page;
+            subs[tl] = none ? own_sub : cur_sub;
+            missing |= none ? 1 << tl : 0;
             cur_sub += 16;
             if (cur_sub >= bt) {
                 cur_sub = 0;
@@ -313,34 +313,44 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     locate(pages, subs, missing);
     // Two chunks' loads are always on their way: keys in two register sets that take turns, values in two more.  The
     // first two value chunks of a segment are asked for before its scores are formed, the first two key chunks of the
-    // next segment while its last values are multiplied.
+    // next segment while its last values are multiplied.  The order is held by barriers to the compiler.
+    // What the registers hold at once decides where a load may go.  Heads of 208 and more that walk their context (WIDE) ask for the second
+    // value chunk behind the scores and for the next segment's keys ahead of the last value chunk, and their last segment has no body of its
+    // own: asked for as the others do, up to 349 registers a lane went to memory (64 requests of 1,280 tokens, 8 KV heads, us: of 256
+    // 248 -> 131, of 240 209 -> 123, of 224 153 -> 116; narrower ones are slower this way where the context is shared out: of 192 49 and 56).  The
+    // partial form of 128 has 256 registers and the order left to the compiler (8 requests of 4,096 tokens 38.3 -> 37.2).
     bf16x8_t kf_a[2][QS], kf_b[2][QS];
     load_keys(pages, subs, 0, kf_a);
     load_keys(pages, subs, 1, kf_b);
+    constexpr bool WIDE = !PARTIAL && DT >= 13, ORDERED = !(PARTIAL && DT == 8);
+    auto keep_order = [&]() {
+        if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
+    };
     auto segment = [&](int seg0, auto is_last) {      // the last segment asks for no keys of a next one
         constexpr bool LAST = decltype(is_last)::value;
         if (!LAST) locate(pages_next, subs_next, missing_next);   // the next segment's pages are looked up while this one is worked on
         bf16x8_t vf_a[DT], vf_b[DT];
         load_values(pages, subs, 0, vf_a);
-        load_values(pages, subs, 1, vf_b);
+        if (!WIDE) load_values(pages, subs, 1, vf_b);
         f32x4_t s[8];
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         chunk_scores<DT>(kf_a, qf, s[0], s[1]);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         load_keys(pages, subs, 2, kf_a);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         chunk_scores<DT>(kf_b, qf, s[2], s[3]);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         load_keys(pages, subs, 3, kf_b);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         chunk_scores<DT>(kf_a, qf, s[4], s[5]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!LAST) load_keys(pages_next, subs_next, 0, kf_a);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
+        if (!LAST && !WIDE) load_keys(pages_next, subs_next, 0, kf_a);
+        keep_order();
         chunk_scores<DT>(kf_b, qf, s[6], s[7]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!LAST) load_keys(pages_next, subs_next, 1, kf_b);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
+        if (WIDE) load_values(pages, subs, 1, vf_b);
+        else if (!LAST) load_keys(pages_next, subs_next, 1, kf_b);
+        keep_order();
         float m, l;
         bf16x8_t pf[4];
         if (seg0 + AM_SEG - 1 <= p_first && seg0 >= lo_last && missing == 0) {
@@ -352,16 +362,22 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
         f32x4_t o[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         chunk_values<DT>(vf_a, pf[0], o);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         load_values(pages, subs, 2, vf_a);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         chunk_values<DT>(vf_b, pf[1], o);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         load_values(pages, subs, 3, vf_b);
-        __builtin_amdgcn_sched_barrier(0);
+        keep_order();
         chunk_values<DT>(vf_a, pf[2], o);
+        if (WIDE) {
+            keep_order();
+            load_keys(pages_next, subs_next, 0, kf_a);
+            load_keys(pages_next, subs_next, 1, kf_b);
+            keep_order();
+        }
         chunk_values<DT>(vf_b, pf[3], o);
         if constexpr (PARTIAL) {
             if (col_ok) {
@@ -386,8 +402,12 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
         missing = missing_next;
     };
     int seg0 = key_begin;
-    for (; seg0 + AM_SEG < key_end; seg0 += AM_SEG) segment(seg0, std::false_type{});
-    segment(seg0, std::true_type{});
+    if constexpr (WIDE) {
+        for (; seg0 < key_end; seg0 += AM_SEG) segment(seg0, std::false_type{});
+    } else {
+        for (; seg0 + AM_SEG < key_end; seg0 += AM_SEG) segment(seg0, std::false_type{});
+        segment(seg0, std::true_type{});
+    }
     if constexpr (!PARTIAL) {
         if (col_ok) store_output<DT>(a.out + ((size_t)t * a.n_heads + h) * D, g, o_tot, l_tot, head_gate_factor(a.gate, a.gate_ld, a.gate_wide, t, h),
                                 value_gates(a.gate, a.gate_ld, a.gate_wide, t, h, D));

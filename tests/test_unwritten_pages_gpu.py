@@ -12,7 +12,7 @@ DEV = "cuda:0"
 # few requests (contexts shared out over many waves or workgroups) and many (a wave walks its context); contexts that end in a page's first
 # tile, in its last, at a segment's and a page's edge
 @pytest.mark.parametrize("requests,Hkv", [(3, 2), (40, 8)])
-@pytest.mark.parametrize("D,page,window", [(64, 32, 0), (128, 64, 0), (128, 48, 200), (160, 64, 0), (224, 64, 0), (256, 32, 100)])
+@pytest.mark.parametrize("D,page,window", [(64, 32, 0), (128, 64, 0), (128, 48, 200), (160, 64, 0), (208, 16, 0), (224, 64, 0), (240, 16, 0), (256, 32, 100)])
 def test_keys_past_the_end_are_not_numbers(requests, Hkv, D, page, window):
     from llmx_amd import ops
     contexts = [(1, 15, 17, 33, 96, 128, 129, 250, 257, 400, 513)[i % 11] for i in range(requests)] if requests > 3 else [5, 145, 390]
@@ -44,3 +44,8 @@ def test_keys_past_the_end_are_not_numbers(requests, Hkv, D, page, window):
     ran = ops.take_launches()
     assert ran.get("attention.direct", 0) == (2 if requests > 3 else 0), ran
     assert bool(out[0].isfinite().all()) and torch.equal(out[1], out[0])
+    for i in range(0, requests, 7):         # alone a request's context is shared out: the same bits
+        one = torch.empty_like(q[:1])
+        ops.paged_attention(q[i:i + 1].contiguous(), k.to(DEV), v.to(DEV), i32([contexts[i] - 1]), i32([0]), tables[i:i + 1].contiguous().to(DEV), one,
+                            1.0 / math.sqrt(D), 2 * Hkv, window, plan=ops.attention_plan([1], [contexts[i]], 2 * Hkv, Hkv, DEV, window))
+        assert torch.equal(one[0], out[0][i]), f"request {i}"
