@@ -1066,7 +1066,7 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
                w_group_stride, up_offset, 0, ks, 64, nullptr, -1, 0, 0, 0, epi != TL_SWIGLU ? act : LLMX_ACT_NONE, act_params,
                GluArgs{epi == TL_SWIGLU ? glu_kind : LLMX_GLU_SILU, glu_limit, epi == TL_SWIGLU ? glu_row_scale : nullptr,
                        epi == TL_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld},
-               ticket};
+               grouped ? ticket : nullptr};
     if (!llmx_act_fits(act, act_params, epi == TL_STORE, epi == TL_ADD)) return -2;
     auto launch = [&](int form, int tiles_y, bool short_k = false) -> int {      // short_k: 128-row tiles of short K, whichever kernel has them
         g.bm = form_rows(form);

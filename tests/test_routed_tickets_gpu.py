@@ -47,3 +47,19 @@ def test_tickets_change_no_bit(counts, N, K):
                 exact = a[rows].double() @ w[3].double().T
                 # float32 sums of K exact products of random sign
                 assert (got[rows].double() - exact).abs().max() <= 4 * 2.0 ** -24 * K ** 0.5 * exact.abs().max() * 4
+
+
+def test_a_dense_product_takes_no_tickets():
+    """The entry point that takes a ticket, called for a dense product of more tiles than there are CUs: every tile is stored."""
+    from llmx_amd import ops
+    M, N, K = 2568, 4104, 128
+    gen = torch.Generator().manual_seed(1)
+    a, w = (torch.randn(n, K, generator=gen).to(DEV, torch.bfloat16) for n in (M, N))
+    want, got = (torch.full((M, N), float("nan"), device=DEV) for _ in range(2))
+    ticket = torch.zeros(1, dtype=torch.int32, device=DEV)
+    ops.gemm(a, w, want)
+    args = (M, N, K, K, N, ops.EPI_STORE, ops._split_k(-(-N // 16), K), 0, 0, 0, 0, 1, 0, 0, 0, 0)
+    assert ops.lib().llmx_gemm_tile_tickets(a.data_ptr(), w.data_ptr(), got.data_ptr(), ops._code(got.dtype), *args, ticket.data_ptr(), 0, 0, 0, 0, 0.0, 0, 0, 0,
+                                            torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert bool(want.isfinite().all()) and torch.equal(got, want) and int(ticket) == 0
