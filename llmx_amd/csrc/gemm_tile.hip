@@ -568,9 +568,10 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
 // So, for routed products whose caller brings a ticket counter, a workgroup stays on its CU and takes tile after tile: the next one is
 // looked up while this one is multiplied, and its first K tiles are asked for as stages of LDS fall free; only the stores and one wait stand
 // between two tiles.  The tiles are handed out in order by tickets, not in strides: the row tiles of one expert have to stay close in
-// time for its weights to be found in the caches (strides, 256 experts of 300 rows, 3,072 features of 3,072 values: 2,423 -> 2,664 us).
-// A workgroup a tile and tickets, 256 experts: 64 rows an expert 940 -> 864 us, 100 1,038 -> 954, 130 1,427 -> 1,345, 170 1,701 -> 1,654; 55
-// experts of 300 519 -> 526.
+// time for its weights to be found in the caches (strides, 256 experts of 300 rows, 3,072 features of 3,072 values: 2,423 -> 2,664 us), and
+// a tile is drawn as late as it can be, when the one before the present is done (drawn a tile earlier 2,333 -> 2,436).
+// A workgroup a tile and tickets, gate_up of these sizes, 256 experts: 64 rows an expert 865 -> 839 us, 100 941 -> 893, 130 1,287 -> 1,260,
+// 170 1,599 -> 1,555, but 300 2,079 -> 2,333; 55 experts of 130 302 -> 294, of 200 395 -> 364, but of 100 211 -> 220, of 300 461 -> 497.
 // BARE: nothing is applied to the sums but, gated, silu(gate) * up.  With the other units and activations in the loop over tiles their
 // constants take the registers the sums need; those products launch a workgroup a tile, and dense ones too (nothing gained).
 #define WD_MAX_GROUPS 1536      // groups whose row tiles and places are kept in LDS beside the stages
@@ -581,7 +582,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
     __shared__ int tiles_before[GROUPED ? WD_MAX_GROUPS + 1 : 1], places[GROUPED ? WD_MAX_GROUPS + 1 : 1];
     __shared__ int pairs[3][GROUPED ? WD_BM : 1];        // of the tile before (its sums may still be stored), this one and the next
     __shared__ int scan_waves[8];
-    __shared__ int drawn[2];                             // the next tile and the one after it, taking turns
+    __shared__ int drawn;                                // the tile after this one
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const bool runs = !GROUPED || tile_launch_runs(g);   // looked at below, once the first offsets are asked for too
@@ -754,20 +755,12 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
     // barrier tile t's stage takes tile t+3 (past K's end: the next tile of the product's first ones), and tile t+1
     // (awaited before the barrier) can be read by everybody.
     if ((int)blockIdx.x >= total) return;
-    // A workgroup's first tile is its number's; the others it draws, two ahead, until the next one is none.  So every workgroup with a first
-    // tile draws two that are none, and who draws the last of all puts the counter back.
-    const bool tickets = BARE && GROUPED && g.ticket != nullptr;       // (K of at least four K tiles: TILE_TICKETS_MIN_K)
+    // A workgroup's first tile is its number's; the others it draws, each when the tile before the present is stored, until one is none.  So every
+    // workgroup draws one that is none, and who draws the last of all puts the counter back.
+    const bool tickets = BARE && GROUPED && g.ticket != nullptr && total > (int)gridDim.x;       // (K of at least four K tiles: TILE_TICKETS_MIN_K)
     const int firsts = min((int)gridDim.x, total);
-    auto tile_of = [&](int n) {
-        if (n == total + firsts - 1) atomicExch(g.ticket, 0);
-        return firsts + n;
-    };
-    if (tid == 0) {
-        for (int i = 0; i < 2; ++i) drawn[i] = tickets ? tile_of(atomicAdd(g.ticket, 1)) : total;
-    }
-    __syncthreads();
-    int turn = 0, ticket = 0;
-    bool drew = false;
+    int ticket = 0;
+    if (tid == 0 && tickets) ticket = atomicAdd(g.ticket, 1);
     Tile tile = tile_at(blockIdx.x), next = tile;
     int stage = 0, slot = 0;
     ask_pairs(tile, 0);
@@ -777,7 +770,13 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
     for (;;) {
         const int rows_here = tile.row_end - tile.row_begin;
         const bool works = 64 * wm < rows_here;
-        const int following = __builtin_amdgcn_readfirstlane(drawn[turn]);
+        __builtin_amdgcn_s_waitcnt(0x0070);     // the first three K tiles, the stores of the tile before, the ticket
+        if (tid == 0) {
+            if (tickets && ticket == total - 1) atomicExch(g.ticket, 0);
+            drawn = tickets ? firsts + ticket : total;
+        }
+        __syncthreads();
+        const int following = __builtin_amdgcn_readfirstlane(drawn);
         const bool more = BARE && GROUPED && following < total;
         const bool brings_now = brings_rows;
         const int slot_next = slot == 2 ? 0 : slot + 1;
@@ -806,12 +805,6 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
             ask(n_tiles + 2, stage);
             stage = stage == 2 ? 0 : stage + 1;
         };
-        __builtin_amdgcn_s_waitcnt(0x0070);     // the first three K tiles, and the stores of the tile before
-        if (tid == 0 && drew) drawn[1 - turn] = tile_of(ticket);
-        turn = 1 - turn;
-        __syncthreads();
-        drew = more;
-        if (tid == 0 && more) ticket = atomicAdd(g.ticket, 1);      // travels while the tile is multiplied, and is looked at behind the next wait for everything
         if (!works) {
             for (int t = 0; t < last; ++t) {
                 wait_but(t + 2);
@@ -918,6 +911,7 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
             }
         }
         if (!BARE || !more) return;
+        if (tid == 0) ticket = atomicAdd(g.ticket, 1);
         tile = next;
         slot = slot_next;
     }
