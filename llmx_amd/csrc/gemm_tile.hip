@@ -108,6 +108,7 @@ struct TileArgs {
     int bm;       // rows a workgroup covers: 64 or 128
     const int* tile_stats;  // grouped, optional: the sum over groups of ceil(rows / 128); with choice_bit >= 0 the grouping's choice
     int choice_bit;         // ... whose bit this is: set where this product takes tiles of 128 rows
+    int choice_without;     // ... where the grouping chose for tickets and this product takes none
     int run_if_big;         // with tile_stats: 1: this launch works only if the product takes tiles of 128 rows, 0: only if not
     int strip_runs;         // dense: XCDs take contiguous runs of tiles, strip after strip (see tile_place)
     int run_tiles;          // dense lean form, > 0: workgroup z multiplies only K's run z (this many 64-wide tiles) and stores its sums at C + z * M * ldc
@@ -124,7 +125,7 @@ struct TileArgs {
 __device__ __forceinline__ bool tile_launch_runs(const TileArgs& g) {
     if (!g.tile_stats) return true;
     const int stat = g.tile_stats[0];
-    const bool big = g.choice_bit >= 0 ? (stat >> g.choice_bit) & 1 : (long)stat * 128 * 5 <= (long)g.M * 8;
+    const bool big = g.choice_bit >= 0 ? ((g.choice_without ? stat ^ stat >> 4 : stat) >> g.choice_bit) & 1 : (long)stat * 128 * 5 <= (long)g.M * 8;
     return big == (g.run_if_big != 0);
 }
 
@@ -920,18 +921,21 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
 // form: which kernel takes the product.  The lean forms need whole 64-wide tiles of K, runs that end on them, and
 // operands whose byte offsets fit 32 bits (llmx_gemm_tile_offsets_fit).
 enum : int { FORM_64 = 0, FORM_128 = 1, FORM_WIDE = 2, FORM_BOUNDED = 3, FORM_64_DEEP = 4 };
-// Routed products' tiles of 128 rows: the wide form for long K, and with tickets for shorter K too while a group has some 200 rows at most
-// (256 experts, 3,072 features of 1,536 values, four waves a tile and the wide form, us: 64 rows an expert 563 and 525, 100 647 and 605, 130 770
-// and 761, 300 1,357 and 1,411; 2,048 features, 100 rows, of 1,024 315 and 270, of 512 194 and 170, but 64 experts of 150 rows, 512 76 and 79).
-#define TILE_TICKETS_MIN_K 1024
-static bool wide_routed(int K, long pairs, int groups, const int* ticket) { return K >= 2048 || (ticket && K >= TILE_TICKETS_MIN_K && pairs <= 200L * groups); }
+// Routed products' tiles of 128 rows: the wide form for long K and wherever tiles are taken by tickets (256 experts, 3,072 features of 1,536 values, four
+// waves a tile and the wide form, us: 64 rows an expert 558 and 524, 100 612 and 575, 130 731 and 709, 170 855 and 861; of 1,792 170 964 and
+// 998, 199 1,024 and 1,004; 55 experts of 300 rows, some 60 a group, 281 and 287; 2,048 features of 1,024 values, 100 rows 319 and 277).
+static bool wide_routed(int K, const int* ticket) { return K >= 2048 || ticket; }
+
+// The sums are stored as they are or, gated, as silu(gate) * up.
+static bool nothing_applied(const TileArgs& g, int epi) {
+    return epi == TL_SWIGLU ? g.glu.kind == LLMX_GLU_SILU && !g.glu.row_scale && !g.glu.row_gate : g.act == LLMX_ACT_NONE;
+}
 
 template <int EPI, typename TC, bool GROUPED, bool SPLIT>
 static void tile_launch_form(const TileArgs& g, int form, dim3 grid, hipStream_t stream) {
     if (form == FORM_WIDE) {
         const unsigned tiles = grid.x * grid.y;
-        const bool bare = EPI == TL_SWIGLU ? g.glu.kind == LLMX_GLU_SILU && !g.glu.row_scale && !g.glu.row_gate : g.act == LLMX_ACT_NONE;
-        if (bare) hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT, true>), dim3(g.ticket && tiles > TILE_CUS ? TILE_CUS : tiles), dim3(512), 0, stream, g);
+        if (nothing_applied(g, EPI)) hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT, true>), dim3(g.ticket && tiles > TILE_CUS ? TILE_CUS : tiles), dim3(512), 0, stream, g);
         else hipLaunchKernelGGL((gemm_wide_kernel<EPI, TC, GROUPED, SPLIT, false>), dim3(tiles), dim3(512), 0, stream, g);
         return;
     }
@@ -1057,10 +1061,11 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
     const int steps = (K + 31) / 32, per = (steps + ks - 1) / ks;
     const bool lean = K % TL_BK == 0 && (ks == 1 || per % 2 == 0) && llmx_gemm_tile_offsets_fit(M, N, K, lda, epi, n_groups, a_div, up_offset);
     TileArgs g{(const bf16_t*)A, (const bf16_t*)W, C, M, N, K, lda, ldc, group_offsets, list, n_groups, a_div > 0 ? a_div : 1,
-               w_group_stride, up_offset, 0, ks, 64, nullptr, -1, 0, 0, 0, epi != TL_SWIGLU ? act : LLMX_ACT_NONE, act_params,
+               w_group_stride, up_offset, 0, ks, 64, nullptr, -1, 0, 0, 0, 0, epi != TL_SWIGLU ? act : LLMX_ACT_NONE, act_params,
                GluArgs{epi == TL_SWIGLU ? glu_kind : LLMX_GLU_SILU, glu_limit, epi == TL_SWIGLU ? glu_row_scale : nullptr,
                        epi == TL_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld},
-               grouped ? ticket : nullptr};
+               nullptr};
+    if (grouped && nothing_applied(g, epi) && tile_takes_tickets(K, (N + form_feats(FORM_WIDE, epi) - 1) / form_feats(FORM_WIDE, epi), M, n_groups)) g.ticket = ticket;
     if (!llmx_act_fits(act, act_params, epi == TL_STORE, epi == TL_ADD)) return -2;
     auto launch = [&](int form, int tiles_y, bool short_k = false) -> int {      // short_k: 128-row tiles of short K, whichever kernel has them
         g.bm = form_rows(form);
@@ -1115,8 +1120,9 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
         const int big_tiles = (n_groups < M ? n_groups : M) + M / 128;
         g.tile_stats = tile_stats;
         g.choice_bit = stats_choose ? tile_k_class(K) : -1;
+        g.choice_without = ticket && !g.ticket;
         g.run_if_big = 1;
-        rc = launch(wide_routed(K, M, n_groups, g.ticket) ? FORM_WIDE : FORM_128, big_tiles < max_tiles ? big_tiles : max_tiles, K < 2048);
+        rc = launch(wide_routed(K, g.ticket) ? FORM_WIDE : FORM_128, big_tiles < max_tiles ? big_tiles : max_tiles, K < 2048);
         if (rc == 0) {
             g.run_if_big = 0;
             rc = launch(FORM_64, max_tiles);

@@ -557,6 +557,7 @@ __global__ void __launch_bounds__(1024) moe_chunk_place_kernel(const int* __rest
 }
 
 extern "C" int llmx_tile_choice(int n_pairs, int n128, int n64, int experts) { return tile_choice(n_pairs, n128, n64, experts); }
+extern "C" int llmx_tile_takes_tickets(int K, int strips, int n_pairs, int n_groups) { return tile_takes_tickets(K, strips, n_pairs, n_groups) ? 1 : 0; }
 extern "C" int llmx_tile_choice_tickets(int n_pairs, int n128, int n64, int experts) { return tile_choice_tickets(n_pairs, n128, n64, experts); }
 
 // counts [X], offsets [X+1], list [n_pairs], active [X], n_active [1]

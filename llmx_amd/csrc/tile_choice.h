@@ -25,11 +25,27 @@ __host__ __device__ inline int tile_choice(long n_pairs, long n128, long n64, lo
     return (wide ? 1 : 0) | (wide && experts <= 128 ? 2 : 0) | (four || (2 * n64 >= 3 * n128 && n_pairs <= 80 * experts) ? 4 : 0) | (four ? 8 : 0);
 }
 
-// The choice where the products' workgroups take tiles by tickets.  A tile of 128 then costs what it has rows for, in halves, and its
-// lookup and first loads are covered, so that it is the better one up to some 130 rows an expert, and for K of 1,536 on to 200 (256
-// experts, tiles of 128 and of 64, us: 3,072 features of 3,072 values, 16 rows an expert 756 and 762, 45 817 and 855, 60 853 and 970, 130
-// 1,345 and 1,420, but 170 1,654 and 1,592; of 1,536 values 32 rows 486 and 488, 52 504 and 540, 130 761 and 797, 170 923 and 907; 2,048 features
-// of 2,048 values 20 rows 447 and 467, 60 497 and 532).  Beyond that, and for shorter K, as above.
+// Which routed products take tiles by tickets, of those whose caller brings a counter: `strips` strips of weights of K values, n_pairs rows of n_groups
+// experts (on the host, which does not know how many of them have rows).  Where an expert has few rows a workgroup that stays on its CU gains by what
+// it does not wait for.  Where it has several tiles, one a workgroup finds its weights nearer: launched in order the row tiles of a strip go to one
+// XCD if the strips are a multiple of 8, and the more so the longer they are.  Tickets and a workgroup a tile, us: 12 strips of 3,072
+// values, 256 experts of 64 rows 839 and 865, of 130 1,260 and 1,287, 55 experts of 200 364 and 395, but 256 of 300 2,333 and 2,079; 8 strips of
+// 2,048, 256 of 100 543 and 577, of 170 767 and 821, of 300 1,130 and 1,003.  8 and 16 strips of 3,072, 256 of 130 912 and 890, 1,724 and
+// 1,662, 55 of 300 367 and 331, 688 and 588; of 4,096 1,180 and 1,134, 2,253 and 2,106, 468 and 412, 896 and 730; 12 strips of 3,584 and
+// 4,096, 256 of 64 1,054 and 1,069, 1,336 and 1,387, but 55 of 300 612 and 567, 691 and 641.
+// K from 1,024 on: there the other 128-row form has four waves a tile (wide_routed); 12 strips of 1,536, 256 of 100 575 and 612.
+#define TILE_TICKETS_MIN_K 1024
+inline int tile_takes_tickets(int K, int strips, long n_pairs, long n_groups) {
+    return K >= TILE_TICKETS_MIN_K && K <= 3072 && (K < 2560 || strips % 8 != 0) && n_pairs <= 200 * n_groups;
+}
+
+// The choice for a step whose products bring a counter.  By tickets a tile of 128 costs what it has rows for, in halves, and its lookup and first loads
+// are covered, so that it is the better one up to some 130 rows an expert, and for K of 1,536 on to 200 (256 experts, tiles of 128 and of 64, us:
+// 3,072 features of 3,072 values, 16 rows an expert 756 and 762, 45 808 and 854, 64 839 and 1,028, 130 1,260 and 1,404, but 170 1,555 and
+// 1,561; of 1,536 values 45 503 and 518, 130 709 and 776, 170 861 and 886; 2,048 features of 2,048 values 45 497 and 501, 64 510 and 564, 170
+// 767 and 758).  Beyond that, and for shorter K, as above.  Bits 4 to 7: where the choice above is another one, for the products of the step
+// that take no tickets.
 __host__ __device__ inline int tile_choice_tickets(long n_pairs, long n128, long n64, long experts) {
-    return tile_choice(n_pairs, n128, n64, experts) | (n_pairs <= 132 * experts ? 7 : n_pairs <= 200 * experts ? 4 : 0);
+    const int without = tile_choice(n_pairs, n128, n64, experts), with = without | (n_pairs <= 132 * experts ? 7 : n_pairs <= 200 * experts ? 4 : 0);
+    return with | (with ^ without) << 4;
 }

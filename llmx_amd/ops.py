@@ -119,6 +119,7 @@ def _declare(h) -> None:
         "llmx_gemm_skinny_f32": [P, P, P, I, I, I, I, I, I, I, I, L, P, F, P],
         "llmx_tile_choice": [I, I, I, I],
         "llmx_tile_choice_tickets": [I, I, I, I],
+        "llmx_tile_takes_tickets": [I, I, I, I],
         "llmx_gemm_tile": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_chosen": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_tickets": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, P, I, P, I, F, P, P, I, P],
