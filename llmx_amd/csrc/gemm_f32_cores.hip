@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(64 * KS, MT == 1 ? 4 : 1) gemm_f32_stream_kern
     constexpr int NS = EPI == EPI_SWIGLU ? 2 : 1;                  // weight strips: the features', and the up rows' of the same features
     constexpr int UN = NS * MT == 1 ? 4 : 2;    // steps of a round: its loads travel together (a wave has two rounds on their way, a SIMD four waves)
     __shared__ __attribute__((aligned(16))) float red[KS > 1 ? KS : 1][NS * MT][256];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;     // known to be one for the wave: else every load of weights is a loop over its lanes
     const int r = lane & 15, kg = lane >> 4;
     const int n0 = blockIdx.x * 16, K = g.K;
     const float* A = (const float*)g.A;
