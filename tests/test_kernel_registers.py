@@ -53,6 +53,14 @@ def test_decode_attention_keeps_its_registers(kernels):
         assert kernel[0][".private_segment_fixed_size"] == 0, (name, kernel[0][".vgpr_spill_count"])
 
 
+# the streaming products: those that add or have a bias a feature kept up to 20 registers a lane in memory
+@pytest.mark.parametrize("kernel", ["gemm_skinny_kernel", "gemm_f32_stream_kernel"])
+def test_streaming_products_keep_their_registers(kernel, kernels):
+    found = {n: k for n, k in kernels.items() if kernel in n}
+    assert len(found) > 20
+    assert {n: k[".vgpr_spill_count"] for n, k in found.items() if k[".private_segment_fixed_size"]} == {}
+
+
 # weights are asked for from a place the wave shares; where the compiler does not know it for one, each load becomes a loop over the lanes' places
 @pytest.mark.parametrize("kernel", ["gemm_f32_stream_kernel", "gemm_skinny_kernel"])
 def test_streamed_weights_are_asked_for_once(kernel, library, tmp_path):
