@@ -1144,20 +1144,11 @@ extern "C" int llmx_gemm_tile_tickets(const void* A, const void* W, void* C, int
                      stats_choose, runs_scratch, act, act_params, glu_kind, glu_limit, glu_row_scale, glu_row_gate, glu_row_gate_ld, ticket, stream);
 }
 
-// ... without one.
-extern "C" int llmx_gemm_tile_chosen(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldc, int epi, int ks,
-                                     int n_groups, int max_tiles, const int* group_offsets, const int* list, int a_div, long w_group_stride,
-                                     int up_offset, const int* tile_stats, int stats_choose, float* runs_scratch, int act, const float* act_params, int glu_kind,
-                                     float glu_limit, const float* glu_row_scale, const float* glu_row_gate, int glu_row_gate_ld, hipStream_t stream) {
-    return gemm_tile(A, W, C, c_dtype, M, N, K, lda, ldc, epi, ks, n_groups, max_tiles, group_offsets, list, a_div, w_group_stride, up_offset, tile_stats,
-                     stats_choose, runs_scratch, act, act_params, glu_kind, glu_limit, glu_row_scale, glu_row_gate, glu_row_gate_ld, nullptr, stream);
-}
-
-// ... with the bare count in tile_stats, or none.
+// ... without one, and with the bare count in tile_stats, or none.
 extern "C" int llmx_gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, int N, int K, int lda, int ldc, int epi, int ks,
                               int n_groups, int max_tiles, const int* group_offsets, const int* list, int a_div, long w_group_stride,
                               int up_offset, const int* tile_stats, float* runs_scratch, int act, const float* act_params, int glu_kind,
                               float glu_limit, const float* glu_row_scale, const float* glu_row_gate, int glu_row_gate_ld, hipStream_t stream) {
-    return llmx_gemm_tile_chosen(A, W, C, c_dtype, M, N, K, lda, ldc, epi, ks, n_groups, max_tiles, group_offsets, list, a_div, w_group_stride, up_offset,
-                                 tile_stats, 0, runs_scratch, act, act_params, glu_kind, glu_limit, glu_row_scale, glu_row_gate, glu_row_gate_ld, stream);
+    return gemm_tile(A, W, C, c_dtype, M, N, K, lda, ldc, epi, ks, n_groups, max_tiles, group_offsets, list, a_div, w_group_stride, up_offset, tile_stats,
+                     0, runs_scratch, act, act_params, glu_kind, glu_limit, glu_row_scale, glu_row_gate, glu_row_gate_ld, nullptr, stream);
 }

@@ -585,10 +585,6 @@ extern "C" int llmx_moe_align_ticket(const int* ids, int n_pairs, int n_experts,
     hipLaunchKernelGGL(moe_place_kernel, dim3(n_experts), dim3(64), 0, stream, ids, n_pairs, n_experts, counts, offsets, list, active, n_active);
     return LLMX_CHECK_LAUNCH();
 }
-extern "C" int llmx_moe_align(const int* ids, int n_pairs, int n_experts, int* counts, int* offsets, int* list, int* active, int* n_active,
-                              int* scratch, int* tiles128, int* choice, hipStream_t stream) {
-    return llmx_moe_align_ticket(ids, n_pairs, n_experts, counts, offsets, list, active, n_active, scratch, tiles128, choice, nullptr, stream);
-}
 
 // ---------------------------------------------------------------------------
 // A decode step's routing in one launch: top-k of every row (one wave a row, values in registers: at most 256 experts,

@@ -109,7 +109,6 @@ def _declare(h) -> None:
         "llmx_memory_prep": [P, I, I, I, I, I, P, P, F, P, L, I, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
         "llmx_paged_attention_mfma": [P, P, P, P, P, P, P, I, I, I, P, I, P, P, P, F, I, I, I, I, I, I, I, P, I, I, P],
         "llmx_route_topk": [P, P, I, L, P, P, P, I, I, I, I, I, F, P, I, I, I, P],
-        "llmx_moe_align": [P, I, I, P, P, P, P, P, P, P, P, P],
         "llmx_moe_align_ticket": [P, I, I, P, P, P, P, P, P, P, P, P, P],
         "llmx_route_topk_align": [P, P, I, L, P, P, P, I, I, I, I, I, F, I, I, I, P, P, P, P, P, P],
         "llmx_gemm_skinny": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, P, P, I, L, I, P, P, F, I, P, I, P, I, F, P, P, I, P],
@@ -121,7 +120,6 @@ def _declare(h) -> None:
         "llmx_tile_choice_tickets": [I, I, I, I],
         "llmx_tile_takes_tickets": [I, I, I, I],
         "llmx_gemm_tile": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, P, I, P, I, F, P, P, I, P],
-        "llmx_gemm_tile_chosen": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_tickets": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_offsets_fit": [I, I, I, I, I, I, I, I],
         "llmx_sample_all": [P, P, P, P, P, P, I, I, P, P],
@@ -1695,11 +1693,11 @@ def moe_align(ids: torch.Tensor, n_experts: int, counts: torch.Tensor, offsets: 
     if scratch is not None and scratch.numel() < need:
         raise KernelError(f"moe_align: scratch of {scratch.numel()} ints, {need} needed")
     _check(lib().llmx_moe_align_ticket(_dev(ids, "ids", torch.int32), n_pairs, n_experts, _dev(counts, "counts", torch.int32, (n_experts,)),
-                                _dev(offsets, "offsets", torch.int32, (n_experts + 1,)), _dev(pairs, "pairs", torch.int32, (n_pairs,)),
-                                _dev(active, "active", torch.int32, (n_experts,)), _dev(n_active, "n_active", torch.int32, (1,)),
-                                _dev(scratch if need else None, "scratch", torch.int32),
-                                *(_tile_stats(tile_stats) + [0])[:2] if need and n_pairs >= TILE_STATS_MIN_PAIRS else (0, 0),
-                                _dev(ticket if need else None, "ticket", torch.int32, (1,)), _stream()), "moe_align")
+                                       _dev(offsets, "offsets", torch.int32, (n_experts + 1,)), _dev(pairs, "pairs", torch.int32, (n_pairs,)),
+                                       _dev(active, "active", torch.int32, (n_experts,)), _dev(n_active, "n_active", torch.int32, (1,)),
+                                       _dev(scratch if need else None, "scratch", torch.int32),
+                                       *(_tile_stats(tile_stats) + [0])[:2] if need and n_pairs >= TILE_STATS_MIN_PAIRS else (0, 0),
+                                       _dev(ticket if need else None, "ticket", torch.int32, (1,)), _stream()), "moe_align")
 
 
 def route_topk_align(z: torch.Tensor, bias: Optional[torch.Tensor], ids: torch.Tensor, weights: torch.Tensor, k: int, score: int,

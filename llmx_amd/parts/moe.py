@@ -217,7 +217,7 @@ class RoutedExperts(FeedForward):
         on_input = self.weight_on == "input"
         if self.plain_unit is not None:
             ops.grouped_gemm(h, self.w_gate_up, act, offsets, pairs, slots, ops.EPI_STORE, active, n_active, token_rows=T, tile_stats=tile_stats,
-                             act=(self.plain_unit, None), ticket=ticket)
+                             act=(self.plain_unit, None))
         else:
             glu = ops.Glu(self.unit, self.limit, weights.view(T * slots) if on_input else None)
             ops.grouped_gemm(h, self.w_gate_up, act, offsets, pairs, slots, ops.EPI_SWIGLU, active, n_active, token_rows=T, tile_stats=tile_stats,
