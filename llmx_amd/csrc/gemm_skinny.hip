@@ -37,7 +37,7 @@ struct SkinnyArgs {
     int M, N, K;
     int lda, ldc;
     // grouped
-    const int* active;         // [n_active] group ids that have rows (blockIdx.y indexes it)
+    const int* active;         // [max_active] group ids (blockIdx.y indexes it), the first n_active those that have rows; the others are read, not used
     const int* n_active;       // device scalar
     const int* group_offsets;  // [G+1]
     const int* list;           // expert-sorted pair ids
@@ -308,8 +308,8 @@ __global__ void __launch_bounds__(64 * KS, MT > 1 || NORM == SK_LAYER ? 1 : EPI 
 
 // Dense products of 17 to 64 rows: two strips of 16 features a workgroup.  With several tiles of rows a step fetches
 // more bytes of rows (from the caches, again for every strip) than of weights; a workgroup that multiplies the rows'
-// fragments into two strips fetches them half as often.  A wave's steps, their rounds of four and the order in which
-// the waves' sums are added are those of the kernel above: the same bits.
+// fragments into two strips fetches them half as often.  A wave's steps and the order in which the waves' sums are added are
+// those of the kernel above: the same bits.
 template <int KS, int MT, int EPI, typename TC, bool BIASED>
 __global__ void __launch_bounds__(64 * KS) gemm_skinny_two_strips_kernel(SkinnyArgs g) {
     static_assert(EPI != SK_SWIGLU, "one weight strip a feature strip");

@@ -44,10 +44,12 @@ def test_rows_have_the_bits_the_tiles_give(M, N, K):
     if N % 2 == 0:
         gated = torch.full((M, N // 2), float("nan"), device=DEV)
         ops.gemm(a[:M].contiguous(), w, gated, ops.EPI_SWIGLU)
-        gate, up = c[:, :N // 2].double(), c[:, N // 2:].double()
+        both = a[:M].double() @ w.double().T
+        gate, up = both[:, :N // 2], both[:, N // 2:]
         want = gate * torch.sigmoid(gate) * up
-        # the gated product's own split of K may differ from the plain one's: both are K-term float32 sums
-        assert (gated.double() - want).abs().max() <= 64 * 2.0 ** -24 * math.sqrt(K) * max(1.0, want.abs().max().item()) * K ** 0.5
+        # the two sums' errors (see close), carried on by |silu'| <= 1.1 and |silu(g)| <= |g|, and the unit's own float32 roundings
+        bound = 4 * 2.0 ** -24 * math.sqrt(K) * both.abs().max() * (1.1 * up.abs() + gate.abs()) + 2.0 ** -21 * want.abs() + 1e-6
+        assert ((gated.double() - want).abs() <= bound).all()
     if M <= 4 and K % 8 == 0 and M * K * 2 <= 32768:
         x, nw = rnd(M, K, seed=3, dtype=torch.float32), rnd(K, seed=4, dtype=torch.float32)
         h, formed = torch.empty(M, K, dtype=torch.bfloat16, device=DEV), torch.full((M, N), float("nan"), device=DEV)
@@ -66,7 +68,7 @@ def test_grouped_rows_are_the_dense_ones(N, K):
     w, a = rnd(G, N, K, seed=1), rnd(P, K)
     offsets = torch.tensor([0] + torch.tensor(counts).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
     pairs = torch.randperm(P, generator=torch.Generator().manual_seed(5)).to(DEV, torch.int32)
-    active = torch.tensor([0, 2, 3, 5, 77777, -5], dtype=torch.int32, device=DEV)      # what lies beyond the groups that have rows is not read
+    active = torch.tensor([0, 2, 3, 5, 77777, -5], dtype=torch.int32, device=DEV)      # what lies beyond the groups that have rows is not used
     n_active = torch.tensor([4], dtype=torch.int32, device=DEV)
     c = torch.full((P, N), float("nan"), device=DEV)
     ops.take_launches()
