@@ -230,7 +230,6 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     const int p_col = a.pos[t];
     const int p_first = __builtin_amdgcn_readfirstlane(a.pos[row0]), p_last = __builtin_amdgcn_readfirstlane(a.pos[row0 + n_rows - 1]);
     const int* table = a.tables + (size_t)__builtin_amdgcn_readfirstlane(a.row_entry[row0]) * a.max_blocks;
-    const int lo_col = (a.window > 0 && p_col - a.window + 1 > 0) ? p_col - a.window + 1 : 0;
     const int lo_first = (a.window > 0 && p_first - a.window + 1 > 0) ? p_first - a.window + 1 : 0;
     const int lo_last = (a.window > 0 && p_last - a.window + 1 > 0) ? p_last - a.window + 1 : 0;
     // the item's keys: the segments seg_first .. p_last / 128 of the row, cut into n_splits runs of whole segments
@@ -317,15 +316,11 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
     // What the registers hold at once decides where a load may go.  Heads of 208 and more that walk their context (WIDE) ask for the second
     // value chunk behind the scores and for the next segment's keys ahead of the last value chunk, and their last segment has no body of its
     // own: asked for as the others do, up to 349 registers a lane went to memory (64 requests of 1,280 tokens, 8 KV heads, us: of 256
-    // 248 -> 131, of 240 209 -> 123, of 224 153 -> 116; narrower ones are slower this way where the context is shared out: of 192 49 and 56).  The
-    // partial form of 128 has 256 registers and the order left to the compiler (8 requests of 4,096 tokens 38.3 -> 37.2).
+    // 248 -> 131, of 240 209 -> 123, of 224 153 -> 116; narrower ones are slower this way where the context is shared out: of 192 49 and 56).
     bf16x8_t kf_a[2][QS], kf_b[2][QS];
     load_keys(pages, subs, 0, kf_a);
     load_keys(pages, subs, 1, kf_b);
-    constexpr bool WIDE = !PARTIAL && DT >= 13, ORDERED = !(PARTIAL && DT == 8);
-    auto keep_order = [&]() {
-        if constexpr (ORDERED) __builtin_amdgcn_sched_barrier(0);
-    };
+    constexpr bool WIDE = !PARTIAL && DT >= 13;
     auto segment = [&](int seg0, auto is_last) {      // the last segment asks for no keys of a next one
         constexpr bool LAST = decltype(is_last)::value;
         if (!LAST) locate(pages_next, subs_next, missing_next);   // the next segment's pages are looked up while this one is worked on
@@ -333,55 +328,58 @@ __global__ void __launch_bounds__(256, (PARTIAL && DT <= 8) ? 2 : 1) paged_atten
         load_values(pages, subs, 0, vf_a);
         if (!WIDE) load_values(pages, subs, 1, vf_b);
         f32x4_t s[8];
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_a, qf, s[0], s[1]);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         load_keys(pages, subs, 2, kf_a);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_b, qf, s[2], s[3]);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         load_keys(pages, subs, 3, kf_b);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_a, qf, s[4], s[5]);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         if (!LAST && !WIDE) load_keys(pages_next, subs_next, 0, kf_a);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_scores<DT>(kf_b, qf, s[6], s[7]);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         if (WIDE) load_values(pages, subs, 1, vf_b);
         else if (!LAST) load_keys(pages_next, subs_next, 1, kf_b);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         float m, l;
         bf16x8_t pf[4];
         if (seg0 + AM_SEG - 1 <= p_first && seg0 >= lo_last && missing == 0) {
             segment_softmax<false>(s, 0xffffffffu, a.scale, m, l, pf);   // every key counts for every column
         } else {
             // (a tile without a page lies wholly at or after key_end, or before the window, which the mask leaves out)
+            const int lo_col = (a.window > 0 && p_col - a.window + 1 > 0) ? p_col - a.window + 1 : 0;
             segment_softmax<true>(s, segment_mask(seg0, g, col_ok, lo_col, p_col, key_end), a.scale, m, l, pf);
         }
         f32x4_t o[DT];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_values<DT>(vf_a, pf[0], o);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         load_values(pages, subs, 2, vf_a);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_values<DT>(vf_b, pf[1], o);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         load_values(pages, subs, 3, vf_b);
-        keep_order();
+        __builtin_amdgcn_sched_barrier(0);
         chunk_values<DT>(vf_a, pf[2], o);
         if (WIDE) {
-            keep_order();
+            __builtin_amdgcn_sched_barrier(0);
             load_keys(pages_next, subs_next, 0, kf_a);
             load_keys(pages_next, subs_next, 1, kf_b);
-            keep_order();
+            __builtin_amdgcn_sched_barrier(0);
         }
         chunk_values<DT>(vf_b, pf[3], o);
         if constexpr (PARTIAL) {
             if (col_ok) {
-                const size_t at = (size_t)slot * 16 + (size_t)c * slots + (seg0 / AM_SEG - seg_first);
+                // heads of 128, whose registers are full: the lane's column formed again (kept since the kernel's start, two registers went to memory)
+                const int col = DT == 8 ? (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) & 15 : c;
+                const size_t at = (size_t)slot * 16 + (size_t)col * slots + (seg0 / AM_SEG - seg_first);
                 float* dst = a.part_o + at * D;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4_t*>(dst + 16 * dt + 4 * g) = o[dt];
