@@ -92,6 +92,32 @@ __device__ __forceinline__ void store_quad(TC* crow, int n, int N, bool rows_ali
     }
 }
 
+// Sixteen rows of two neighbouring tiles of 16 features, float32 (a lane: row lane % 16, features 4 (lane / 16) .. of either), stored as whole
+// lines of 128 bytes that the caches do not keep: lanes 8 apart exchange quads (as weight_lines.h's do), so that an instruction stores 32
+// features of eight rows.  line(0) and line(8) are the lane's rows lane % 8 and 8 + lane % 8 of C, null where the tile has none; n: of the even tile.
+// Kept, results of many megabytes are written back from the caches between the weights' reads and cost several times their bytes (down of 256
+// experts, 3,072 features of 1,536 values, us, half lines kept, whole lines kept, half lines streamed, whole lines streamed: 52 rows an expert 511,
+// 510, 493, 477; 100 rows 608, 606, 575, 542).  From TILE_STREAM_OUT bytes on, which the caches would not hold for the reader anyway; below, it
+// gains nothing (product and a pass over its results, kept and streamed: 2,048 features of 2,048 values, 768 rows 21.8 and 22.3, 2,048 rows
+// 31.6 and 30.0; 8,192 of 3,072, 128 rows 24.7 and 25.3, 256 rows 27.9 and 27.4, 600 rows 48.3 and 47.4; 200,064 of 3,072, 8 rows 219.5 and
+// 218.8, 16 rows 228.6 and 222.9, 64 rows 263 and 253).
+#define TILE_STREAM_OUT (6L << 20)
+template <typename Line>
+__device__ __forceinline__ void store_lines(const f32x4_t& even, const f32x4_t& odd, int n, int N, Line line) {
+    f32x4_t lo, hi;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        lo[i] = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(even[i]), (int)__float_as_uint(odd[i]), 0x128, 0xf, 0xc, false));
+        hi[i] = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(odd[i]), (int)__float_as_uint(even[i]), 0x128, 0xf, 0x3, false));
+    }
+    n += 2 * (threadIdx.x & 8);
+    if (n >= N) return;
+    float* const first = line(0);
+    float* const second = line(8);
+    if (first) __builtin_nontemporal_store(lo, reinterpret_cast<f32x4_t*>(first + n));
+    if (second) __builtin_nontemporal_store(hi, reinterpret_cast<f32x4_t*>(second + n));
+}
+
 struct TileArgs {
     const bf16_t* A;
     const bf16_t* W;
@@ -115,6 +141,7 @@ struct TileArgs {
     int act;                // TL_STORE, TL_ADD: an activation applied to the product (LLMX_ACT_*; a launch of runs' sums leaves it to the kernel that adds them)
     const float* act_params;
     GluArgs glu;            // TL_SWIGLU: the gated unit and its per-row values
+    int stream_out;         // float32 results that go past the caches (see store_lines)
     int* ticket;            // grouped wide form, optional: 0, and 0 again afterwards; workgroups take tile after tile by it
 };
 
@@ -516,6 +543,22 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(TileArgs g) {
     const int fq = 4 * (lane >> 4);
     const bool rows_aligned = g.ldc % 4 == 0 && ((uintptr_t)g.C & 15) == 0;   // a lane's four features make one access
     const ActFn act(EPI == TL_STORE ? g.act : LLMX_ACT_NONE, g.act_params);      // formed once, as in the wide form
+    if constexpr (FAST && EPI == TL_STORE && std::is_same<TC, float>::value) {
+        if (g.stream_out) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                float* at[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int rc = rows_c[BM / 2 * wm + 16 * t + 8 * h + (lr & 7)];
+                    at[h] = rc >= 0 ? (float*)g.C + (size_t)rc * g.ldc : nullptr;
+                }
+#pragma unroll
+                for (int f = 0; f < 4; f += 2) store_lines(acc[f][t], acc[f + 1][t], n0 + 64 * wn + 16 * f + fq, g.N, [&](int d) { return at[d >> 3]; });
+            }
+            return;
+        }
+    }
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
         const int rc = rows_c[BM / 2 * wm + 16 * t + lr];
@@ -876,8 +919,34 @@ __global__ void __launch_bounds__(512) gemm_wide_kernel(TileArgs g) {
             last_stage_read();
 
             // acc[f][q][i]: feature (tile f) 4*(lane/16) + i, row 64*wm + 16*q + lane%16
+            const bool lines = BARE && EPI == TL_STORE && std::is_same<TC, float>::value && g.stream_out;
+            if (lines) {
+#pragma unroll
+                for (int q = 0; q < TT; ++q) {
+                    float* at[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int m = 64 * wm + 16 * q + 8 * h + (lr & 7);
+                        at[h] = m < rows_here ? (float*)g.C + (size_t)row_of(tile, slot, m) * g.ldc : nullptr;
+                    }
+#pragma unroll
+                    for (int f = 0; f < 4; f += 2) {
+                        // (copies, as below)
+                        f32x4_t even = acc[f][q], odd = acc[f + 1][q];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float x = even[i], y = odd[i];
+                            asm volatile("" : "+v"(x), "+v"(y));
+                            even[i] = x;
+                            odd[i] = y;
+                        }
+                        store_lines(even, odd, tile.n0 + 64 * wn + 16 * f + fq, g.N, [&](int d) { return at[d >> 3]; });
+                    }
+                }
+            }
 #pragma unroll
             for (int q = 0; q < TT; ++q) {
+                if (lines) break;
                 if (64 * wm + 16 * q + lr >= rows_here) continue;
                 const int rc = row_of(tile, slot, 64 * wm + 16 * q + lr);
                 TC* crow = (TC*)g.C + (size_t)rc * g.ldc;
@@ -1064,7 +1133,9 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
                w_group_stride, up_offset, 0, ks, 64, nullptr, -1, 0, 0, 0, 0, epi != TL_SWIGLU ? act : LLMX_ACT_NONE, act_params,
                GluArgs{epi == TL_SWIGLU ? glu_kind : LLMX_GLU_SILU, glu_limit, epi == TL_SWIGLU ? glu_row_scale : nullptr,
                        epi == TL_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld},
-               nullptr};
+               0, nullptr};
+    g.stream_out = lean && epi == TL_STORE && c_dtype == LLMX_F32 && nothing_applied(g, epi) && N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0 &&
+                   (long)M * N * (long)sizeof(float) >= TILE_STREAM_OUT;
     if (grouped && nothing_applied(g, epi) && tile_takes_tickets(K, (N + form_feats(FORM_WIDE, epi) - 1) / form_feats(FORM_WIDE, epi), M, n_groups)) g.ticket = ticket;
     if (!llmx_act_fits(act, act_params, epi == TL_STORE, epi == TL_ADD)) return -2;
     auto launch = [&](int form, int tiles_y, bool short_k = false) -> int {      // short_k: 128-row tiles of short K, whichever kernel has them
@@ -1096,6 +1167,7 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
         part.m_tiles = (M + 63) / 64;
         part.run_tiles = tiles_per_run;
         part.strip_runs = llmx_gemm_tile_strip_runs((N + TL_BN - 1) / TL_BN, part.m_tiles, 0);
+        part.stream_out = 0;
         part.act = LLMX_ACT_NONE;       // the runs' sums are stored bare; the kernel that adds them applies the activation
         llmx_note_launch(LK_GEMM_TILE_RUNS_APART);
         hipLaunchKernelGGL((gemm_tile_kernel<TL_STORE, float, false, false, true, 64>), dim3((N + TL_BN - 1) / TL_BN, part.m_tiles, runs), dim3(256), 0,
