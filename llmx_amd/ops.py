@@ -1371,7 +1371,11 @@ class AttentionPlan:
 
 
 _PLAN_CACHE: dict = {}
-ATTENTION_TARGET_WAVES = 2048   # work items wanted before long contexts stop being split further
+# Work items wanted before long contexts stop being split further; half as many again where each segment is an item of its own then: they are on the
+# chip together, and no item has two segments while others have one (us a step of four layers, 2,048 items and an item a segment: 2 requests of
+# 20,011 tokens 970 -> 949, 4 of 8,000 1,269 -> 1,248, 8 of 4,096 1,720 -> 1,703, 16 of 2,000 2,540 -> 2,521).  Beyond, more items lose (2,048 and 3,072
+# items: 2 of 40,000 tokens 2,300 and 2,383, 8 of 9,000 3,590 and 3,660, 30 of 2,500 7,391 and 7,447).
+ATTENTION_TARGET_WAVES = 2048
 ATTENTION_WHOLE_ITEMS = 320     # from this many items on (rows x KV heads) no context is split: one wave an item walks its context (up to 512 items a workgroup each, over all the chip) at 5-6 TB/s, and sharing out would cost the partial results and their merge (4,096 tokens: 40 rows 163 -> 152 us a layer, 48 rows 190 -> 154, 64 rows 227 -> 176, 128 rows 447 -> 348; 32 rows are faster split: 114 against 139)
 ATTENTION_SEGMENT = 128         # keys in a segment: the unit contexts are split in (the kernel's AM_SEG)
 ATTENTION_WIDE_ITEMS = 1024     # up to this many decoding items a step, an item gets a workgroup of 4 waves instead of one wave
@@ -1395,6 +1399,8 @@ def attention_plan(row_counts, contexts, n_heads: int, n_kv_heads: int, device, 
         seg_cap = -(-longest // ATTENTION_SEGMENT) + 1
         seg_cap = -(-seg_cap // 8) * 8       # in steps of 8, so a growing context reuses a plan for 1,024 tokens
         n_splits = max(1, min(-(-ATTENTION_TARGET_WAVES // base), seg_cap))
+        if 2 * base * seg_cap <= 3 * ATTENTION_TARGET_WAVES:
+            n_splits = seg_cap
         if base >= ATTENTION_WHOLE_ITEMS:     # enough items as they are: sharing out would cost the partial results and their merge
             n_splits = 1
     key = (tuple(row_counts), n_heads, n_kv_heads, n_splits, seg_cap, str(device))
