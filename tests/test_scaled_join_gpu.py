@@ -1,0 +1,31 @@
+"""x += s1 * y1 (+ s2 * y2): four values a thread where the rows allow it, with the bits of one a thread."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rnd(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+# four values a thread, and one where a row's are no multiple of 4 or do not begin on 16 bytes
+@pytest.mark.parametrize("rows,n", [(1, 4), (3, 2048), (129, 1028), (2, 6)])
+@pytest.mark.parametrize("two,scaled,copied", [(True, True, torch.bfloat16), (True, False, None), (False, True, torch.float32), (False, False, torch.bfloat16)])
+def test_the_scaled_join_of_any_place(rows, n, two, scaled, copied):
+    from llmx_amd import ops
+    got = []
+    for shift in (0, 1):
+        place = lambda seed, *shape: rnd(*shape, seed=seed) if not shift else torch.cat([torch.zeros(1, device=DEV), rnd(*shape, seed=seed).flatten()])[1:].view(*shape)
+        x, y1, y2, s1, s2 = place(1, rows, n), place(2, rows, n), place(3, rows, n), place(4, n), place(5, n)
+        copy = torch.full((rows, n), float("nan"), dtype=copied, device=DEV) if copied is not None else None
+        ops.scale_add(x, y1, s1 if scaled else None, y2 if two else None, s2 if scaled and two else None, copy)
+        got.append((x.clone(), None if copy is None else copy.float()))
+    assert torch.equal(got[0][0], got[1][0]) and (copied is None or torch.equal(got[0][1], got[1][1]))
+    want = rnd(rows, n, seed=1).double() + rnd(rows, n, seed=2).double() * (rnd(n, seed=4).double() if scaled else 1.0)
+    if two:
+        want = want + rnd(rows, n, seed=3).double() * (rnd(n, seed=5).double() if scaled else 1.0)
+    # two products and two sums, each rounded once
+    assert (got[0][0].double() - want).abs().max() <= 4 * 2.0 ** -24 * 60
