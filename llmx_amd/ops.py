@@ -1371,19 +1371,38 @@ class AttentionPlan:
 
 
 _PLAN_CACHE: dict = {}
-# Work items wanted before long contexts stop being split further; half as many again where each segment is an item of its own then: they are on the
-# chip together, and no item has two segments while others have one (us a step of four layers, 2,048 items and an item a segment: 2 requests of
-# 20,011 tokens 970 -> 949, 4 of 8,000 1,269 -> 1,248, 8 of 4,096 1,720 -> 1,703, 16 of 2,000 2,540 -> 2,521).  Beyond, more items lose (2,048 and 3,072
-# items: 2 of 40,000 tokens 2,300 and 2,383, 8 of 9,000 3,590 and 3,660, 30 of 2,500 7,391 and 7,447).
+# Work items wanted before long contexts stop being split further: what the chip holds of them at once (head sizes to 128; above, half as many).
 ATTENTION_TARGET_WAVES = 2048
+# An item a segment instead, where that many items leave an eighth and more of the segments to items that have one already: the launch then takes as long
+# as two segments, while items of one each give their places to the rest as they end.  us a layer with the join, 48 query and 8 KV heads of 128, equal
+# rows, 2,048 items and an item a segment: 2 of 20,460 tokens 46.8 and 43.0, 4 of 9,196 45.6 and 40.1, 8 of 5,356 47.0 and 42.8, 16 of 2,668 48.1 and
+# 44.7; heads of 256 (16 and 8) 2 of 20,460 81.5 and 72.9, 8 of 5,356 83.1 and 73.7; 130 drawn batches of equal and unequal rows, head sizes 128, 192
+# and 256, gain 4-22%.  The limits, each with what lies beyond it:
+ATTENTION_EACH_ITEMS = 3072     # items in all: 2 of 31,980 59.5 and 60.6; of 256, 2 of 24,812 87.6 and 92.1
+ATTENTION_EACH_SECOND = 8       # the part (1 / this) of the segments that would be an item's second: 16 of 2,156 37.9 and 41.7, 8 of 4,076 (none) 32.6 and 36.3
+# Items to segments with keys: a plan has items for the longest context and up to 1,024 tokens more, and those without keys stand between the others
+# (8 of 2,797 to 6,007, 1.31 items a segment: 39.9 and 41.4; 2 of 17,178 about, 1.25: 38.3 and 39.4; one of 16,000 beside 7 of 1,000 45 and 65)
+ATTENTION_EACH_SPARE = 1.15
+ATTENTION_EACH_SEGMENTS = 256   # segments of a context: 2 of 75,480, 86,020 and 91,072 with 12 and 2 heads 54.5 and 55.5, 56.5 and 57.0, 58.1 and 62.6
+ATTENTION_EACH_MIN_DIM = 128    # head size: of 64 (32 and 8 heads), 1 of 48,876 36.0 and 37.2, 2 of 24,428 32.8 and 33.1, 8 of 5,356 28.2 and 26.5
 ATTENTION_WHOLE_ITEMS = 320     # from this many items on (rows x KV heads) no context is split: one wave an item walks its context (up to 512 items a workgroup each, over all the chip) at 5-6 TB/s, and sharing out would cost the partial results and their merge (4,096 tokens: 40 rows 163 -> 152 us a layer, 48 rows 190 -> 154, 64 rows 227 -> 176, 128 rows 447 -> 348; 32 rows are faster split: 114 against 139)
 ATTENTION_SEGMENT = 128         # keys in a segment: the unit contexts are split in (the kernel's AM_SEG)
 ATTENTION_WIDE_ITEMS = 1024     # up to this many decoding items a step, an item gets a workgroup of 4 waves instead of one wave
 
 
-def attention_plan(row_counts, contexts, n_heads: int, n_kv_heads: int, device, window: int = 0) -> AttentionPlan:
+def _item_a_segment(contexts, head_chunks: int, n_splits: int, seg_cap: int, head_dim: int, reach: int) -> bool:
+    """Whether the decoding rows' segments get an item each, where n_splits items a row and head would leave some items two (the constants above say why)."""
+    items = len(contexts) * seg_cap
+    if n_splits >= seg_cap or seg_cap > ATTENTION_EACH_SEGMENTS or items * head_chunks > ATTENTION_EACH_ITEMS or head_dim < ATTENTION_EACH_MIN_DIM:
+        return False
+    segments = [-(-min(context, reach) // ATTENTION_SEGMENT) for context in contexts]
+    second = sum(max(0, n - n_splits) for n in segments)
+    return ATTENTION_EACH_SECOND * second >= sum(segments) and items <= ATTENTION_EACH_SPARE * sum(segments)
+
+
+def attention_plan(row_counts, contexts, n_heads: int, n_kv_heads: int, device, window: int = 0, head_dim: int = 128) -> AttentionPlan:
     """row_counts[i]: rows of entry i in the step (entries' rows are consecutive, in order); contexts[i]: tokens the
-    entry holds after the step.  Single-row entries become items per KV head (columns = its query heads) that share out
+    entry holds after the step; head_dim: the heads' size, by which the sharing out is chosen.  Single-row entries become items per KV head (columns = its query heads) that share out
     the context's 128-key segments when there are few rows; longer entries become tiles of 16 rows of one head, 12 tiles
     that read the same KV head to a workgroup (three workgroups of 4 for head sizes other than 128).  How the context is shared out changes no result: segments are folded in
     key order either way."""
@@ -1394,12 +1413,11 @@ def attention_plan(row_counts, contexts, n_heads: int, n_kv_heads: int, device, 
     if single:
         base = len(single) * len(head_chunks)
         longest = max(contexts[i] for i in single)
-        if window > 0:
-            longest = min(longest, window + ATTENTION_SEGMENT)
-        seg_cap = -(-longest // ATTENTION_SEGMENT) + 1
+        reach = window + ATTENTION_SEGMENT if window > 0 else longest
+        seg_cap = -(-min(longest, reach) // ATTENTION_SEGMENT) + 1
         seg_cap = -(-seg_cap // 8) * 8       # in steps of 8, so a growing context reuses a plan for 1,024 tokens
         n_splits = max(1, min(-(-ATTENTION_TARGET_WAVES // base), seg_cap))
-        if 2 * base * seg_cap <= 3 * ATTENTION_TARGET_WAVES:
+        if _item_a_segment([contexts[i] for i in single], len(head_chunks), n_splits, seg_cap, head_dim, reach):
             n_splits = seg_cap
         if base >= ATTENTION_WHOLE_ITEMS:     # enough items as they are: sharing out would cost the partial results and their merge
             n_splits = 1

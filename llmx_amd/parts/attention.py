@@ -206,11 +206,11 @@ class Attention(Mixer):
 
     def _plan(self, step):
         """The matrix-core attention kernel's work items for this step's rows: made once a step and shared by every
-        layer with the same heads and window."""
+        layer with the same heads, head size and window."""
         window = int(self.window or 0)
-        return step.shared(("attention.plan", self.heads, self.kv_heads, window),
+        return step.shared(("attention.plan", self.heads, self.kv_heads, window, self.head_dim),
                            lambda: ops.attention_plan([e.n for e in step.entries], [e.past + e.n for e in step.entries], self.heads,
-                                                      self.kv_heads, step.device, window))
+                                                      self.kv_heads, step.device, window, self.head_dim))
 
     def _rules_plan(self, step):
         """The work items of the matrix-core kernel for rules, made once a step and shared by every layer with the same
