@@ -92,16 +92,36 @@ __device__ __forceinline__ void store_quad(TC* crow, int n, int N, bool rows_ali
     }
 }
 
+// Which float32 results leave past the caches.  Kept, they are written back between the reads of weights that stream from memory and cost several times
+// their bytes (down of 256 experts, 3,072 features of 1,536 values, us, half lines kept, whole lines kept, half lines streamed, whole lines streamed:
+// 52 rows an expert 511, 510, 493, 477; 100 rows 608, 606, 575, 542).  Streamed, their reader finds them in memory instead of the last cache (256 MB), so
+// both count.
+// Routed, from 8 MB on.  Down and combine together, kept and streamed, us: 256 experts 6 MB 328 and 326, 8 MB 368 and 366, 31 MB 435 and 417, 60 MB 472 and
+// 453, 117 MB 514 and 491, 156 MB 537 and 508 (503 + 34 and 470 + 38), 309 MB 658 and 611; 55 of 256 experts 60 MB 149 and 143, 192 MB 332 and 333;
+// 64 experts (2,048 of 512) 12 MB 44 and 42, 48 MB 67 and 64, 96 MB 105 and 104; 16 experts (4,096 of 2,048) 8 MB 73 and 74; 8 experts nothing.
+// Dense, where the results are a fifth of the last cache (48 MB), or the weights twice as large as it and the results 10 MB.  Whole passes of a model with
+// its other results as they are, kept and streamed, us: 8,192 features of 3,072 values in four layers, 2,048 rows (64 MB) 6,267 and 6,195,
+// 1,745 rows 7,163 and 7,132; 9,216 of 2,048 (72 MB) 5,477 and 5,373, but 900 rows (32 MB) 3,428 and 3,446; 3,072 of 2,048, 900 and 1,999
+// rows 3,374 and 3,388, 5,532 and 5,538; 2,048 of 2,048, 1,999 rows 5,532 and 5,546; smaller results go either way (520 rows of 8,192 of 3,072 4,103
+// and 4,088, 900 rows of 4,096 of 128 3,374 and 3,390).  A product and a copy of its results: 65,536 features of 2,048 values 25 MB 74 and 76, 50 MB
+// 159 and 135; 28,672 of 4,096 22 MB 79 and 82, 56 MB 162 and 153, 224 MB 554 and 568; 16,384 of 8,192 32 MB 147 and 149, 64 MB 290 and 287; a
+// head of 200,064 of 3,072 (1.2 GB) 13 MB 229 and 223, 49 MB 264 and 254, 76 MB 295 and 269, of 151,936 of 2,048 (0.6 GB) 7 MB 122 and 124,
+// 14 MB 135 and 131, of 131,072 of 2,048 (0.54 GB) 5 MB 129 and 130, 12 MB 139 and 138.
+// Only whole lines: rows that begin within one lose (9,220 of 3,072, 1,024 rows 99 and 106; 256 experts, 3,076 features, 192 MB 585 and 614).
+#define TILE_STREAM_ROUTED (8L << 20)
+#define TILE_STREAM_DENSE (48L << 20)
+#define TILE_STREAM_HEAD (10L << 20)
+#define TILE_STREAM_HEAD_WEIGHTS (512L << 20)
+extern "C" int llmx_gemm_tile_streams_out(const void* C, int M, int N, int K, int ldc, int n_groups) {
+    const long results = (long)M * N * (long)sizeof(float), weights = (long)N * K * (long)sizeof(bf16_t);
+    if (N % 4 || ldc % 32 || ((uintptr_t)C & 127)) return 0;
+    if (n_groups > 0) return results >= TILE_STREAM_ROUTED;
+    return results >= TILE_STREAM_DENSE || (results >= TILE_STREAM_HEAD && weights >= TILE_STREAM_HEAD_WEIGHTS);
+}
+
 // Sixteen rows of two neighbouring tiles of 16 features, float32 (a lane: row lane % 16, features 4 (lane / 16) .. of either), stored as whole
 // lines of 128 bytes that the caches do not keep: lanes 8 apart exchange quads (as weight_lines.h's do), so that an instruction stores 32
 // features of eight rows.  line(0) and line(8) are the lane's rows lane % 8 and 8 + lane % 8 of C, null where the tile has none; n: of the even tile.
-// Kept, results of many megabytes are written back from the caches between the weights' reads and cost several times their bytes (down of 256
-// experts, 3,072 features of 1,536 values, us, half lines kept, whole lines kept, half lines streamed, whole lines streamed: 52 rows an expert 511,
-// 510, 493, 477; 100 rows 608, 606, 575, 542).  From TILE_STREAM_OUT bytes on, which the caches would not hold for the reader anyway; below, it
-// gains nothing (product and a pass over its results, kept and streamed: 2,048 features of 2,048 values, 768 rows 21.8 and 22.3, 2,048 rows
-// 31.6 and 30.0; 8,192 of 3,072, 128 rows 24.7 and 25.3, 256 rows 27.9 and 27.4, 600 rows 48.3 and 47.4; 200,064 of 3,072, 8 rows 219.5 and
-// 218.8, 16 rows 228.6 and 222.9, 64 rows 263 and 253).
-#define TILE_STREAM_OUT (6L << 20)
 template <typename Line>
 __device__ __forceinline__ void store_lines(const f32x4_t& even, const f32x4_t& odd, int n, int N, Line line) {
     f32x4_t lo, hi;
@@ -1134,8 +1154,7 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
                GluArgs{epi == TL_SWIGLU ? glu_kind : LLMX_GLU_SILU, glu_limit, epi == TL_SWIGLU ? glu_row_scale : nullptr,
                        epi == TL_SWIGLU ? glu_row_gate : nullptr, glu_row_gate_ld},
                0, nullptr};
-    g.stream_out = lean && epi == TL_STORE && c_dtype == LLMX_F32 && nothing_applied(g, epi) && N % 4 == 0 && ldc % 4 == 0 && ((uintptr_t)C & 15) == 0 &&
-                   (long)M * N * (long)sizeof(float) >= TILE_STREAM_OUT;
+    g.stream_out = lean && epi == TL_STORE && c_dtype == LLMX_F32 && nothing_applied(g, epi) && llmx_gemm_tile_streams_out(C, M, N, K, ldc, n_groups);
     if (grouped && nothing_applied(g, epi) && tile_takes_tickets(K, (N + form_feats(FORM_WIDE, epi) - 1) / form_feats(FORM_WIDE, epi), M, n_groups)) g.ticket = ticket;
     if (!llmx_act_fits(act, act_params, epi == TL_STORE, epi == TL_ADD)) return -2;
     auto launch = [&](int form, int tiles_y, bool short_k = false) -> int {      // short_k: 128-row tiles of short K, whichever kernel has them

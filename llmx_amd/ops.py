@@ -122,6 +122,7 @@ def _declare(h) -> None:
         "llmx_gemm_tile": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_tickets": [P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, I, L, I, P, I, P, P, I, P, I, F, P, P, I, P],
         "llmx_gemm_tile_offsets_fit": [I, I, I, I, I, I, I, I],
+        "llmx_gemm_tile_streams_out": [P, I, I, I, I, I],
         "llmx_sample_all": [P, P, P, P, P, P, I, I, P, P],
         "llmx_sample_topk": [P, P, P, P, P, P, P, P, I, I, P, I, P],
         "llmx_sample_ranked": [P, P, P, P, P, P, P, P, I, I, P, P],

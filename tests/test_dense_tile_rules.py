@@ -1,5 +1,5 @@
 """The host's rules for dense tiled products, asked of the built library: which of them multiply K's runs in workgroups of their own, and
-which hand their strips to XCDs in runs."""
+which hand their strips to XCDs in runs; and which tiled products, dense or routed, send float32 results past the caches."""
 
 import pytest
 
@@ -33,3 +33,16 @@ def test_runs_apart(M, N, K, apart):
 def test_strips_handed_to_xcds_in_runs(strips, row_tiles, wide, runs):
     from llmx_amd import ops
     assert ops.lib().llmx_gemm_tile_strip_runs(strips, row_tiles, int(wide)) == int(runs)
+
+
+# both sides of every line: bytes of the results (8 MB routed, 48 MB dense, 10 MB beside weights of 512 MB), rows of whole lines
+@pytest.mark.parametrize("at,M,N,K,ldc,groups,streams", [
+    (0, 683, 3072, 1536, 3072, 256, True), (0, 682, 3072, 1536, 3072, 256, False), (0, 4096, 512, 128, 512, 24, True), (0, 4095, 512, 128, 512, 24, False),
+    (0, 8192, 3076, 1536, 3076, 256, False), (0, 8192, 3076, 1536, 3104, 256, True), (0, 8192, 3074, 1536, 3104, 256, False), (64, 8192, 3072, 1536, 3072, 256, False),
+    (128, 8192, 3072, 1536, 3072, 256, True), (16, 64, 200064, 3072, 200064, 0, False),
+    (0, 14, 200064, 3072, 200064, 0, True), (0, 13, 200064, 3072, 200064, 0, False), (0, 20, 131072, 2048, 131072, 0, True), (0, 90, 131040, 2048, 131040, 0, False),
+    (0, 1536, 8192, 3072, 8192, 0, True), (0, 1535, 8192, 3072, 8192, 0, False), (0, 96, 131072, 64, 131072, 0, True), (0, 768, 2048, 2048, 2048, 0, False),
+    (0, 400, 8192, 32768, 8192, 0, True), (0, 64, 200068, 3072, 200068, 0, False), (0, 2048, 9220, 2048, 9220, 0, False)])
+def test_results_past_the_caches(at, M, N, K, ldc, groups, streams):
+    from llmx_amd import ops
+    assert ops.lib().llmx_gemm_tile_streams_out(4096 + at, M, N, K, ldc, groups) == int(streams)
