@@ -1165,6 +1165,7 @@ static int gemm_tile(const void* A, const void* W, void* C, int c_dtype, int M, 
         if (grid.y > 65535) return -2;
         g.strip_runs = grouped ? 0 : llmx_gemm_tile_strip_runs((int)grid.x, (int)grid.y, form == FORM_WIDE);
         if (form == FORM_64_DEEP) llmx_note_launch(LK_GEMM_TILE_64_DEEP);
+        if (g.stream_out) llmx_note_launch(LK_GEMM_TILE_LINES);
         llmx_note_launch(short_k ? LK_GEMM_TILE_GROUPED_128
                          : form == FORM_WIDE ? (grouped ? LK_GEMM_TILE_GROUPED_WIDE : LK_GEMM_TILE_WIDE)
                          : form == FORM_128 ? LK_GEMM_TILE_GROUPED_128

@@ -7,6 +7,8 @@
 // Some kinds name a path with several forms, each with a kind of its own beside it: gemm_generic (products outside the bfloat16 matrix
 // cores) is gemm_universal, gemm_generic.stream or gemm_generic.tiles; attention.generic is attention_universal or attention_f32;
 // gemm_tile.64 counts gemm_tile.64_deep too, delta_prep counts delta_prep.rows.
+// A kind whose name has a + is a detail of launches that are counted under their own kind too (how a kernel stores its results): ops.take_launches gives
+// details only where they are asked for.
 // The reference keeps the same kind of record for its tests (/root/reference/src/backends/backend.hpp:96-112).
 #pragma once
 
@@ -34,6 +36,7 @@
     X(GEMM_TILE_GROUPED_128, "gemm_tile.grouped_128")                                                                     \
     X(GEMM_TILE_GROUPED_WIDE, "gemm_tile.grouped_wide")                                                                   \
     X(GEMM_TILE_GROUPED_BOUNDED, "gemm_tile.grouped_bounded")                                                             \
+    X(GEMM_TILE_LINES, "gemm_tile+lines")                                                                                 \
     X(GEMM_F32_SKINNY, "gemm_f32.skinny")                                                                                 \
     X(GEMM_F32_NORMED, "gemm_f32.normed")                                                                                 \
     X(GEMM_F32_ROWS, "gemm_f32.rows")                                                                                     \

@@ -198,16 +198,17 @@ def launch_kinds() -> list:
     return [h.llmx_launch_name(i).decode() for i in range(h.llmx_launch_kinds())]
 
 
-def take_launches() -> dict:
+def take_launches(details: bool = False) -> dict:
     """Which kernel forms were launched since the last call, by name, with their counts (forms that were not are
-    left out); the counts are cleared.  The library counts on the host at every launch site, so this tells a test which
+    left out); the counts are cleared.  `details`: with the names that have a +, which say how launches counted under another name did their work.  The library counts on the host at every launch site, so this tells a test which
     of several kernels with equal results ran (/root/reference/src/backends/backend.hpp:96-112 keeps such a record for
     the same purpose).  A launch recorded into a HIP graph counts once, at the recording, not at replays."""
     h = lib()
     n = h.llmx_launch_kinds()
     counts = (c_long * n)()
     h.llmx_take_launches(counts, n)
-    return {h.llmx_launch_name(i).decode(): int(counts[i]) for i in range(n) if counts[i]}
+    names = [h.llmx_launch_name(i).decode() for i in range(n)]
+    return {name: int(count) for name, count in zip(names, counts) if count and (details or "+" not in name)}
 
 
 # ---------------------------------------------------------------------------
