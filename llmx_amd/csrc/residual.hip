@@ -88,6 +88,7 @@ extern "C" int llmx_scale_add(float* x, const float* y1, const float* s1, const 
     const size_t total = (size_t)rows * n;
     const uintptr_t bits = (uintptr_t)x | (uintptr_t)y1 | (uintptr_t)s1 | (uintptr_t)y2 | (uintptr_t)s2 | (uintptr_t)copy;
     if (n % 4 == 0 && bits % 16 == 0) {
+        llmx_note_launch(LK_SCALE_ADD_FOUR);
         const dim3 grid((unsigned)((total / 4 + 255) / 256));
         if (copy_dtype == LLMX_F32)
             hipLaunchKernelGGL(scale_add4_kernel<float>, grid, dim3(256), 0, stream, x, y1, s1, y2, s2, (float*)copy, n, total);

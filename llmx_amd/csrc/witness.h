@@ -66,6 +66,7 @@
     X(RMSNORM_PAIR, "rmsnorm_pair")                                                                                       \
     X(RMSNORM_ADD, "rmsnorm_add")                                                                                         \
     X(SCALE_ADD, "scale_add")                                                                                             \
+    X(SCALE_ADD_FOUR, "scale_add+four")                                                                                   \
     X(ACT_XIELU, "act.xielu")                                                                                             \
     X(ACT_GELU_GATHER, "act.gelu_gather")                                                                                 \
     X(GATED_SCAN, "gated_scan")                                                                                           \

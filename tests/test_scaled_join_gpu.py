@@ -29,3 +29,33 @@ def test_the_scaled_join_of_any_place(rows, n, two, scaled, copied):
         want = want + rnd(rows, n, seed=3).double() * (rnd(n, seed=5).double() if scaled else 1.0)
     # two products and two sums, each rounded once
     assert (got[0][0].double() - want).abs().max() <= 4 * 2.0 ** -24 * 60
+
+
+# four values a thread only where every operand lies on 16 bytes: each of them moved by one value, alone
+@pytest.mark.parametrize("n", [1028, 1030])
+@pytest.mark.parametrize("copied", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("moved", [None, "x", "y1", "s1", "y2", "s2", "copy"])
+def test_four_values_a_thread(moved, copied, n):
+    from llmx_amd import ops
+    rows, got = 3, []
+    for name in (None, moved):
+        held = {}
+
+        def place(which, values):
+            space = torch.full((values.numel() + 8,), float("nan"), dtype=values.dtype, device=DEV)
+            at = 1 if which == name else 0
+            held[which] = (space, at, values.numel())
+            view = space[at:at + values.numel()].view(values.shape)
+            view.copy_(values)
+            return view
+
+        x, y1, y2 = (place(which, rnd(rows, n, seed=i)) for i, which in enumerate(("x", "y1", "y2")))
+        s1, s2 = place("s1", rnd(n, seed=3)), place("s2", rnd(n, seed=4))
+        copy = place("copy", torch.zeros(rows, n, dtype=copied, device=DEV))
+        ops.take_launches()
+        ops.scale_add(x, y1, s1, y2, s2, copy)
+        assert ops.take_launches(details=True) == {"scale_add": 1, **({"scale_add+four": 1} if name is None and n % 4 == 0 else {})}
+        got.append((x.clone(), copy.clone()))
+        for space, at, size in held.values():       # nothing beside an operand is touched
+            assert bool(space[:at].isnan().all()) and bool(space[at + size:].isnan().all())
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
