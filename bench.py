@@ -5,7 +5,7 @@
 
 A step is one decode step of the whole batch: B requests, each at a context that reaches C tokens at the last timed
 step, one new token each, logits -> greedy token on the device -> ids read back (the reference's batched `tg`,
-/root/reference/src/cli/main.cpp:1246-1254, reads each pass's results before the next; it reports every test it times,
+src/cli/main.cpp:1246-1254, reads each pass's results before the next; it reports every test it times,
 :1192-1287, and so does this line).  Prints one JSON line:
   value, ms_per_step   decoded tokens a second and the step's time at the default batch;
   roofline             bytes the decode step has to read (every weight it uses once, with the measured number of

@@ -3,7 +3,7 @@
 Layers with the same need (kv heads, head width, all keys or a window of them) form a group with a pool of its own.
 A step first reserves (`prepare`) the pages its rows will write, in every group or in none; after the step ran it
 commits, which also gives back the pages of a windowed group that no later row can read; a failed step aborts and
-returns exactly the pages the attempt took (/root/reference/src/model/kv_cache.hpp:71-179).  `truncate` takes a request
+returns exactly the pages the attempt took (src/model/kv_cache.hpp:71-179).  `truncate` takes a request
 back to a shorter length and returns the pages beyond it (:126-134).  Ending a request gives everything back.
 
 State slots and a failing step: with `shadow_slots` a step writes each request's fixed-size state into a second slot

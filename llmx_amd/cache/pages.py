@@ -1,7 +1,7 @@
 """Page ids and per-request state slots: the logical side of the cache, host only.
 
 The pool hands out ids dense from zero, reuses the most recently freed id first, counts references, and refuses a
-double release, a retain of a free page and an empty pool (/root/reference/src/model/kv_cache.hpp:14-67).
+double release, a retain of a free page and an empty pool (src/model/kv_cache.hpp:14-67).
 """
 
 from __future__ import annotations

@@ -1,4 +1,4 @@
-"""The command line, in the reference's manner (/root/reference/src/cli/main.cpp): `llmx generate MODEL [PROMPT]`.
+"""The command line, in the reference's manner (src/cli/main.cpp): `llmx generate MODEL [PROMPT]`.
 
 Flags keep the reference's names and meanings where it has them (main.cpp:2018-2038 sampling, :541-574 execution):
 --max-tokens/-n, --temp, --topk, --topp, --min-p, --penalty, --presence-penalty, --frequency-penalty, --seed,
@@ -7,7 +7,7 @@ perplexity: --ctx-size/-c, --chunks, --per-token.  There is no tokenizer here: a
 (comma or space separated), given on the line, with --file, or made up with --prompt-len; a stop text is a sequence
 of token ids.  Instead of a model folder, `--config JSON --random SEED` runs the configuration with weights generated
 on the device from the seed (the reference builds its file-less model the same way for its bench,
-/root/reference/src/model/arch/registry.hpp:144-152): `llmx generate --config cfg.json --random 0 "1 2 3"`.
+src/model/arch/registry.hpp:144-152): `llmx generate --config cfg.json --random 0 "1 2 3"`.
 A usage error exits with status 2 (main.cpp:100-103); a flag given twice is refused (:129-159).
 """
 
@@ -285,7 +285,7 @@ def bench_model_parser() -> argparse.ArgumentParser:
 
 def cmd_bench_model(argv) -> int:
     """`llmx bench --model DIR [--p 64] [--n 64] [--r 3] [--seqs 1] [--depth 0]`, the reference's model bench
-    (/root/reference/src/cli/main.cpp:67-75,1192-1287): the rate of a prompt of p tokens after `depth` tokens of
+    (src/cli/main.cpp:67-75,1192-1287): the rate of a prompt of p tokens after `depth` tokens of
     history, and of n decoded tokens (one sequence after the history; or `seqs` sequences together, each after the
     prompt, with each step's logits read on the host as a server would), as mean and standard deviation over r runs
     after one run that is not counted.  `--config JSON --random SEED` stands for the folder as elsewhere."""

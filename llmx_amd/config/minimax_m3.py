@@ -5,8 +5,8 @@ q and the whole k projection and a partial NeoX rotary embedding, then a
 sigmoid-scored top-k router with a per-expert correction bias over SwiGLU
 experts (no shared expert, every layer routed).  Key names are the ones the
 reference's fixture writes for this family
-(/root/reference/tests/fixture_minimax.py:26-38); the checks are those of
-/root/reference/src/model/arch/minimax_m3.hpp:38-52.
+(tests/fixture_minimax.py:26-38); the checks are those of
+src/model/arch/minimax_m3.hpp:38-52.
 """
 
 from __future__ import annotations

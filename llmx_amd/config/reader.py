@@ -4,8 +4,8 @@ Every key that changes the arithmetic must be present and in range; a key the
 architecture does not read is refused by name unless it is on the
 architecture's list of keys without effect.  The two refusal texts follow the
 reference's discipline for model metadata ("missing metadata K" /
-"unsupported metadata K": /root/reference/src/model/arch/minimax_m3.hpp:58-63,
-typed getters in /root/reference/src/model/arch/metadata.hpp:17-77), spelled
+"unsupported metadata K": src/model/arch/minimax_m3.hpp:58-63,
+typed getters in src/model/arch/metadata.hpp:17-77), spelled
 with config.json's own key names.
 """
 

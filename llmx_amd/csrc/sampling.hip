@@ -1,6 +1,6 @@
 // Sampling kernels: arg-max and the temperature draw over the whole row.
 //
-// Semantics follow the reference's host sampler (/root/reference/src/inference/sampler.hpp:88-132,258-378):
+// Semantics follow the reference's host sampler (src/inference/sampler.hpp:88-132,258-378):
 // greedy takes the largest score, the lowest id on ties, a NaN only as the leader; the weight of a token is
 // exp((score - best) / temp); sums are double; the draw r * sum walks ids in increasing order and returns the first id
 // whose running sum exceeds it, else the best id.  `skip` (>= n for none) is an id no path gives.

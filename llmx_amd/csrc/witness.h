@@ -9,7 +9,7 @@
 // gemm_tile.64 counts gemm_tile.64_deep too, delta_prep counts delta_prep.rows.
 // A kind whose name has a + is a detail of launches that are counted under their own kind too (how a kernel stores its results): ops.take_launches gives
 // details only where they are asked for.
-// The reference keeps the same kind of record for its tests (/root/reference/src/backends/backend.hpp:96-112).
+// The reference keeps the same kind of record for its tests (src/backends/backend.hpp:96-112).
 #pragma once
 
 #define LLMX_LAUNCH_KINDS(X)                                                                                              \

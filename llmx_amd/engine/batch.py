@@ -1,6 +1,6 @@
 """One step's rows as the parts see them: the row plan on the device and scratch storage.
 
-The row plan follows the reference's `begin` (/root/reference/src/model/passes.hpp:369-392): token ids, positions that
+The row plan follows the reference's `begin` (src/model/passes.hpp:369-392): token ids, positions that
 continue each request's length, the rows whose logits are wanted; it is uploaded in one copy.
 """
 
@@ -38,7 +38,7 @@ class StepError(ValueError):
 
 
 def check_entries(entries: Sequence[StepEntry], cache, max_positions: int, vocab: int) -> List[EntryView]:
-    """The refusals that come before anything is reserved (/root/reference/src/model/passes.hpp:271-413): an empty
+    """The refusals that come before anything is reserved (src/model/passes.hpp:271-413): an empty
     batch, a request named twice or not open, an entry without tokens, a context that would be exceeded, a token id
     outside the embedding's rows, a wanted place outside the entry, more rows than a step takes.  Returns the entries'
     views (slot, first row, rows, tokens held before)."""

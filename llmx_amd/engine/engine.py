@@ -2,7 +2,7 @@
 
 `step` takes a batch of (request, its next tokens): portions of prompts beside single decoded tokens, cut anywhere.
 It runs only the tokens it is given, as one batch, from the cache earlier steps left, and returns the logits at the
-wanted places.  The transaction follows the reference's pass (/root/reference/src/model/passes.hpp:271-413 refusals
+wanted places.  The transaction follows the reference's pass (src/model/passes.hpp:271-413 refusals
 before anything is reserved, :633-653 reserve pages, :771-830 run, :1007-1032 commit, :1124-1134 roll back).
 """
 
@@ -89,7 +89,7 @@ class Engine:
         self._workspace = Workspace(self.device)
         self._uploader = RowPlanUploader(self.device)
         #: callable(step, kind, **tensors): sees what parts show of a step (the reference's route hook,
-        #: /root/reference/src/model/arch/blocks.hpp:118-138); None in serving
+        #: src/model/arch/blocks.hpp:118-138); None in serving
         self.observer = None
         self._make_cache()
         self.graphs = bool(graphs) and all(getattr(p, "graph_safe", False) for p in self.model.parts()) \
@@ -241,7 +241,7 @@ class Engine:
         """Takes the request back to its first `length` tokens (its pages beyond them are given back), so that it can go
         on from that prefix: scoring another continuation, dropping a rejected draft.  A model that keeps fixed-size
         state per request can only be taken back to nothing (the state is cleared) or left as it is: a state cannot be
-        unwound.  The reference's rule: /root/reference/src/model/kv_cache.hpp:126-134, history.hpp:58-59."""
+        unwound.  The reference's rule: src/model/kv_cache.hpp:126-134, history.hpp:58-59."""
         held = self.cache.length(request)
         if self._stateful and 0 < length < held:
             raise StepError(f"truncate: request {request!r} keeps a state of fixed size, which cannot be taken back to {length} of {held} tokens")

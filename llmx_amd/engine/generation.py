@@ -1,6 +1,6 @@
 """Generation: the scheduler driving the engine's step function and the device sampler.
 
-The loop is the reference's generate (/root/reference/src/inference/generate.hpp:19-124) for many requests at once:
+The loop is the reference's generate (src/inference/generate.hpp:19-124) for many requests at once:
 the first token comes from the logits of the prompt's last row, every later one from a one-token step; an end token is
 neither kept nor fed; at max_tokens the request ends.
 """

@@ -1,6 +1,6 @@
 """Perplexity of a sequence of token ids, in windows that each start from an empty history.
 
-Follows the reference's definition (/root/reference/src/inference/perplexity.hpp:41-90): a window of `context` tokens
+Follows the reference's definition (src/inference/perplexity.hpp:41-90): a window of `context` tokens
 scores every token but its first (which is only context) with -(logit[target] - log sum exp(logits)) in double; a
 rest shorter than two tokens is left out; windows run through the prompt path (portions of a step) or, with
 `per_token`, one token a step through the decode path.

@@ -10,10 +10,10 @@ Policy (decisions only; it owns no model and is tested with a simulated executor
   * A request finishes on its end token (not kept, unless ignore_eos), when its generated ids end with one of its
     stop sequences, or at max_tokens; its pages and slot go back at once.  The last token that max_tokens allows is
     fed in the next step, without logits, before the request ends, so that what the cache holds is the whole reply
-    (/root/reference/src/inference/generate.hpp:28-45: an end token and the token completing a stop text are not fed,
+    (src/inference/generate.hpp:28-45: an end token and the token completing a stop text are not fed,
     the last token the limit allows is); `feed_last=False` skips that step.
-The shape follows the reference's scheduler (/root/reference/src/server/scheduler.hpp:1187-1376 form, :752-766 admission,
-:2514-2571 retire; reservation: /root/reference/src/server/policy.hpp:153-158).
+The shape follows the reference's scheduler (src/server/scheduler.hpp:1187-1376 form, :752-766 admission,
+:2514-2571 retire; reservation: src/server/policy.hpp:153-158).
 """
 
 from __future__ import annotations

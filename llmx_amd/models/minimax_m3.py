@@ -2,7 +2,7 @@
 
 E0 embedding; per layer: RMSNorm, attention (GQA, RMSNorm over the whole q and k projections, partial NeoX rotary),
 RMSNorm, sigmoid-routed SwiGLU experts with a correction bias; final RMSNorm and an untied or tied head.  Tensor names
-are the ones the reference's fixture gives this family (/root/reference/tests/fixture_minimax.py:48-67), minus the
+are the ones the reference's fixture gives this family (tests/fixture_minimax.py:48-67), minus the
 index, shared-expert and dense-layer tensors this variant does not have.
 """
 

@@ -1,7 +1,7 @@
 """One registry from an architecture's name (config.json `architectures[0]`, or `architecture`) to its typed configuration and its model.
 
 An entry holds the configuration class (`from_json(dict)`, `to_json()`) and the function that turns a configuration
-into a `ModelSpec`.  The lookup follows /root/reference/src/model/arch/registry.hpp:25-60: an unknown name is refused
+into a `ModelSpec`.  The lookup follows src/model/arch/registry.hpp:25-60: an unknown name is refused
 by name.
 """
 

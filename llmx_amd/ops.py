@@ -201,7 +201,7 @@ def launch_kinds() -> list:
 def take_launches(details: bool = False) -> dict:
     """Which kernel forms were launched since the last call, by name, with their counts (forms that were not are
     left out); the counts are cleared.  `details`: with the names that have a +, which say how launches counted under another name did their work.  The library counts on the host at every launch site, so this tells a test which
-    of several kernels with equal results ran (/root/reference/src/backends/backend.hpp:96-112 keeps such a record for
+    of several kernels with equal results ran (src/backends/backend.hpp:96-112 keeps such a record for
     the same purpose).  A launch recorded into a HIP graph counts once, at the recording, not at replays."""
     h = lib()
     n = h.llmx_launch_kinds()

@@ -3,9 +3,9 @@
 Per row: q, k, v projections of the normed input (biases optional); an optional RMSNorm over the whole q and the whole k
 projection, or over every q and k head by itself with one weight of head_dim values for all heads; rotation of the first `rotary_dim` values of each head at the row's position; k and v written to the
 request's pages; softmax(q.k * head_dim^-1/2) over keys 0..p (or the last `window`) of the same request, head h reading
-KV head h / (heads / kv_heads); output projection.  Formula order: /root/reference/src/backends/cpu/cpu_backend.hpp:971-1104
+KV head h / (heads / kv_heads); output projection.  Formula order: src/backends/cpu/cpu_backend.hpp:971-1104
 (attention), :1461-1480 (rotation); the norm over the whole projection is this architecture's variant of the
-reference's per-head norm (/root/reference/src/model/arch/minimax_m3.hpp:258-259).
+reference's per-head norm (src/model/arch/minimax_m3.hpp:258-259).
 """
 
 from __future__ import annotations

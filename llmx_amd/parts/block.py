@@ -1,7 +1,7 @@
 """The arrangements of a layer's parts.
 
 "prenorm": x += mixer(norm(x)); x += ffn(norm(x)) with the residual x in float32 (the second optional): the arrangement of
-/root/reference/src/model/arch/minimax_m3.hpp:247-287 (norm, mixer joined into the residual, norm, feed-forward joined).
+src/model/arch/minimax_m3.hpp:247-287 (norm, mixer joined into the residual, norm, feed-forward joined).
 "parallel": x += s1 * mixer(norm1(x)) + s2 * ffn(norm2(x)) with both norms of the same x, learned factors s1, s2 a
 coordinate (or constants), and an optional per-layer token input after the sum; without a second norm both sublayers read
 norm1's rows.  Without factors each result is added to x where it is formed: (x + mixer(h)) + ffn(h).

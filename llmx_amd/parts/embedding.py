@@ -1,6 +1,6 @@
 """Token embedding and the language-model head.
 
-x[t] = table[id[t]] widened to float32, times the embedding's scale where the model has one (/root/reference/src/model/arch/blocks.hpp:95-97); logits = rows . W^T in
+x[t] = table[id[t]] widened to float32, times the embedding's scale where the model has one (src/model/arch/blocks.hpp:95-97); logits = rows . W^T in
 float32 for the wanted rows only (:267-272).  A tied head reads the embedding's table.  A bigram embedding adds a second
 table's row, chosen by the token and the one before it.
 """

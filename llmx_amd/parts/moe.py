@@ -1,11 +1,11 @@
 """Feed-forward parts: routed SwiGLU experts behind a scored top-k router, a dense SwiGLU, and a dense layer with one
 activation between its two products.
 
-Router: z = h.Wr^T in float32 on unrounded rows (/root/reference/src/backends/backend.hpp:944-947); score sigmoid(z);
+Router: z = h.Wr^T in float32 on unrounded rows (src/backends/backend.hpp:944-947); score sigmoid(z);
 the pick key is score + correction bias, k picks, the lowest id on ties; weight = the unbiased score, divided by the
-picks' sum when normalizing, times the scale (/root/reference/src/backends/cpu/cpu_backend.hpp:2774-2819).
+picks' sum when normalizing, times the scale (src/backends/cpu/cpu_backend.hpp:2774-2819).
 Experts: a = silu(h.Wg_e^T) * (h.Wu_e^T), y = a.Wd_e^T (:3003-3010); the row's result is sum_j w_j * y_j in slot order
-(:2840-2867).  The fused gate_up tensor holds gate rows first (/root/reference/tests/fixture_minimax.py:153-155).
+(:2840-2867).  The fused gate_up tensor holds gate rows first (tests/fixture_minimax.py:153-155).
 """
 
 from __future__ import annotations

@@ -1,7 +1,7 @@
 """Norms of float32 rows.  RMSNorm: y = x * (r * w), r = 1/sqrt(mean(x^2) + eps); LayerNorm (a weight, a bias if there is one):
 y = (x - mean) / sqrt(var + eps) * w (+ b), var the mean of the squared deviations.  All in float32.
 
-Order of operations as the reference computes it (/root/reference/src/backends/cpu/cpu_backend.hpp:1437-1459): the
+Order of operations as the reference computes it (src/backends/cpu/cpu_backend.hpp:1437-1459): the
 reciprocal root times the weight is formed first, then multiplied into x.
 """
 

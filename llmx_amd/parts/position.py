@@ -1,6 +1,6 @@
 """Position encodings.
 
-Rotary tables follow the reference's float32 arithmetic (/root/reference/src/model/rope.hpp:25-28,203-210):
+Rotary tables follow the reference's float32 arithmetic (src/model/rope.hpp:25-28,203-210):
 freq_i = 1.0f / powf(theta, 2.0f*i/R), angle = (float)pos * freq_i, cos and sin of that angle, one table for all
 layers, pairs (i, i + R/2) of each head rotated (NeoX halves).
 """

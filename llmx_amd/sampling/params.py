@@ -1,6 +1,6 @@
 """Sampling settings, their defaults and ranges, and the generator each request owns.
 
-Names, defaults and ranges are the reference's (/root/reference/src/inference/sampler.hpp:43-65); the generator is its
+Names, defaults and ranges are the reference's (src/inference/sampler.hpp:43-65); the generator is its
 xorshift64 (:21-32).
 """
 
@@ -65,7 +65,7 @@ MAX_STOPS, MAX_STOP_TOKENS = 16, 256
 def normalize_stop(stop) -> tuple:
     """A tuple of tuples of token ids from one sequence of ids or several.
 
-    The reference stops on a text (/root/reference/src/inference/generate.hpp:33, at most 16 of 256 bytes each on its
+    The reference stops on a text (src/inference/generate.hpp:33, at most 16 of 256 bytes each on its
     server); without a tokenizer a sequence of token ids stands for the text.
     """
     if not stop:

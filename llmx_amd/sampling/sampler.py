@@ -1,6 +1,6 @@
 """Draws the next token of each wanted row on the device.
 
-Order of operations as the reference's sampler (/root/reference/src/inference/sampler.hpp:258-378): penalties from the
+Order of operations as the reference's sampler (src/inference/sampler.hpp:258-378): penalties from the
 raw logit, then greedy, or top-k, top-p, min-p and the draw; one uniform number is taken from the request's generator
 per sampled (non-greedy) row, before the branch.
 """

@@ -12,9 +12,9 @@ OUT/<step>.f32 as little-endian float32 [wanted, vocab], in the order of the ent
 `done <step>` is printed and flushed.  Requests named in `end` give back what they hold after the step.
 With --routing the routed layers' expert picks and router logits of every step's rows are written beside the logits
 (OUT/<step>.picks.i32 [routed layers, rows, k], OUT/<step>.router.f32 [routed layers, rows, experts]), as the reference's
-route hook shows them (/root/reference/src/model/arch/blocks.hpp:118-138).
-Modelled on the reference's captures (/root/reference/tools/model_logits.cpp:82-109) and its replay of recorded passes
-(/root/reference/src/server/scheduler.hpp:860-868).
+route hook shows them (src/model/arch/blocks.hpp:118-138).
+Modelled on the reference's captures (tools/model_logits.cpp:82-109) and its replay of recorded passes
+(src/server/scheduler.hpp:860-868).
 """
 
 from __future__ import annotations

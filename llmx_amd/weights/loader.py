@@ -2,8 +2,8 @@
 
 The file's tensors must be exactly the ones the model's parts name, each with the shape its part expects; otherwise
 one error lists every missing tensor, every unexpected tensor and every wrong shape, and nothing is loaded
-(the reference validates headers and the plan before any byte streams: /root/reference/src/inference/load.hpp:316-422,
-/root/reference/src/model/runtime.hpp:582-653).
+(the reference validates headers and the plan before any byte streams: src/inference/load.hpp:316-422,
+src/model/runtime.hpp:582-653).
 
 Types on the device: matrices and tables stay bfloat16 when stored so (a tensor stored in 32 bits stays 32 bits; half
 precision is widened to 32 bits); the 32-bit path widens everything to float32, which is exact.  Norm weights, biases
@@ -51,7 +51,7 @@ class ModelFiles:
             for tensor, file_name in weight_map.items():
                 if not isinstance(file_name, str):
                     raise WeightsError(f"weights: {index}: the weight_map value of {tensor} is not a file name")
-                # a file named by an index sits beside it (/root/reference/src/format/safetensors.hpp:134-137)
+                # a file named by an index sits beside it (src/format/safetensors.hpp:134-137)
                 if file_name in ("", ".", "..") or any(c in file_name for c in "/\\:"):
                     raise WeightsError(f"weights: {index} names a file outside its directory: {file_name}")
             names = sorted(set(weight_map.values()))

@@ -3,7 +3,7 @@
 A counter-based generator: element i of tensor `name` under `seed` is a function of (seed, name, i) only, so the host
 (model folders for tests) and the device (in-place fill of models too large to stage) compute the same values up to the
 rounding of log/cos.  Per-tensor streams keyed by name follow the reference's fixtures
-(/root/reference/tests/fixture_minimax.py:42-83); the distributions are run options, not configuration.
+(tests/fixture_minimax.py:42-83); the distributions are run options, not configuration.
 """
 
 from __future__ import annotations

@@ -2,7 +2,7 @@
 
 The container: an 8-byte little-endian header length, a JSON header whose
 entries hold exactly `dtype`, `shape` and `data_offsets`, then the data area.
-The reader keeps the reference's rules (/root/reference/src/format/safetensors.hpp:
+The reader keeps the reference's rules (src/format/safetensors.hpp:
 dtype map :52-64, entry rules :66-86, file rules :107-130): no key twice in the
 header or in an entry, `__metadata__` an object of strings, offsets span the
 shape, tensors tile the data area without gap or overlap, each at a file offset
@@ -39,7 +39,7 @@ class SafetensorsError(ValueError):
 
 def parse_json_unique(text: str, what: str):
     """json.loads that refuses an object that holds a key twice (the standard parser silently keeps the last one;
-    the reference refuses: /root/reference/src/format/safetensors.hpp:40-44,109)."""
+    the reference refuses: src/format/safetensors.hpp:40-44,109)."""
     def pairs(items):
         seen = {}
         for k, v in items:

@@ -2,7 +2,7 @@
 
 Whole sequences, no cache, no batching, one function for each part, torch on the CPU used as a calculator (float64 by
 default).  It shares no code with llmx_amd: it reads config.json with `json` and the weights with the `safetensors`
-package.  Every function cites the lines of /root/reference it was written from.
+package.  Every function cites the lines of the reference it was written from.
 
 `round_to=torch.bfloat16` rounds the inputs of weight products, the cached keys and values, and the attention output to
 bfloat16 (and widens them again), the places where the serving path stores bfloat16; every sum, norm, softmax, rotation,

@@ -1,6 +1,6 @@
 """A slow, sort-everything transcription of the reference's sampler for one row, with the uniform number given.
 
-Written from /root/reference/src/inference/sampler.hpp:258-378: keep = top_k when 0 < top_k < m else m; weight =
+Written from src/inference/sampler.hpp:258-378: keep = top_k when 0 < top_k < m else m; weight =
 exp((score - best) / temp) in float32; sums in double; all kept and no top-p: walk ids in increasing order; top-k
 without top-p: walk the kept ids in increasing order (weights below min_p count 0); top-p: the shortest ranked prefix
 (best first; ties to the lower id, :76-82) whose weight reaches top_p of the kept weight, min_p cuts its tail, the draw

@@ -1,5 +1,5 @@
 """The cache manager: no page lost, held twice or freed twice, under random orders of requests; windows; slots.
-Rules of the pool follow /root/reference/tests/kv_cache.cpp:42-120 (ids dense from zero, the freed id reused first,
+Rules of the pool follow tests/kv_cache.cpp:42-120 (ids dense from zero, the freed id reused first,
 double release / retain of a free page / exhaustion refused, a failed prepare leaves the request unchanged)."""
 
 import random
@@ -168,7 +168,7 @@ def test_random_orders_never_lose_or_share_a_page(seed):
 
 
 def test_truncate_returns_the_pages_beyond_the_new_length():
-    """/root/reference/src/model/kv_cache.hpp:126-134: the history is rolled back to `length` and the blocks beyond it
+    """src/model/kv_cache.hpp:126-134: the history is rolled back to `length` and the blocks beyond it
     go back; reset is truncate(0)."""
     m = CacheManager([GroupSpec("kv", 4, 10)], max_requests=2)
     m.open("a")
@@ -215,7 +215,7 @@ def test_truncate_inside_a_window_that_gave_pages_back_is_refused():
 
 def test_shadow_slots_keep_the_committed_state_apart_from_a_running_step():
     """With shadow slots a step writes a second slot; commit makes it the request's, abort drops it (the reference keeps
-    the live slot as a mark while a pass writes another: /root/reference/src/model/kv_cache.hpp:216-266)."""
+    the live slot as a mark while a pass writes another: src/model/kv_cache.hpp:216-266)."""
     m = CacheManager([GroupSpec("kv", 4, 8)], max_requests=2, shadow_slots=True)
     assert m.slots.capacity == 4
     a = m.open("a")

@@ -1,5 +1,5 @@
 """The command line's handling of its own arguments (no GPU): usage errors exit with status 2 and say what is wrong
-(the reference's flag discipline: /root/reference/src/cli/main.cpp:100-284)."""
+(the reference's flag discipline: src/cli/main.cpp:100-284)."""
 
 import json
 
@@ -79,7 +79,7 @@ def test_config_and_random_name_a_model_without_a_folder(tmp_path, capsys):
 
 def test_cache_types_and_device_are_the_reference_flags_with_this_engines_limits(tmp_path, capsys):
     """`--cache-type-k/-ctk`, `--cache-type-v/-ctv` and `--device` exist as in the reference
-    (/root/reference/src/cli/main.cpp:120,544-555); the cache has the activations' type and the device is a GPU, and
+    (src/cli/main.cpp:120,544-555); the cache has the activations' type and the device is a GPU, and
     anything else is a usage error before a model is read."""
     rc, _, err = run(["generate", str(tmp_path), "1,2", "-ctk", "f32"], capsys)
     assert rc == 2 and "--cache-type-k f32" in err and "--dtype bf16" in err

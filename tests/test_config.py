@@ -1,5 +1,5 @@
 """Configuration and registry: every key read and checked, each refusal by name (method of
-/root/reference/tests/arch_minimax_m3.cpp:140-193: remove each key in turn, match the refusal text)."""
+tests/arch_minimax_m3.cpp:140-193: remove each key in turn, match the refusal text)."""
 
 import copy
 import json

@@ -3,7 +3,7 @@
 Seventeen, thirty-three and sixty-four requests of different lengths are decoded together for 40 steps with graph
 replays on; some of them pass a block table's width of 64 pages on the way and some the 896 tokens where the split
 contexts' partial results get more slots.  Every request's rows must be the bits of its run alone (the reference's
-"two sequences batched == each alone", /root/reference/tests/kv_cache.cpp, docs/TESTS.md:863-866).  Such steps take
+"two sequences batched == each alone", tests/kv_cache.cpp, docs/TESTS.md:863-866).  Such steps take
 kernels that steps of a few requests do not: the weight-streaming product with two and four tiles of rows and with two
 strips, routed products through the tiled kernels from 17 token rows on, routing and grouping as two launches, more
 attention items than one plan splits.  The launch witness (ops.take_launches) says which forms ran, so that a dispatch

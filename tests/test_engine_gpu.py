@@ -153,7 +153,7 @@ def test_truncate_takes_a_request_back_to_a_prefix(setup):
 
 def test_the_router_reads_unrounded_rows_in_bfloat16():
     """The router's logits come from the float32 normed rows, not from their bfloat16 roundings
-    (/root/reference/src/backends/backend.hpp:943-947: the router's product is F32 whatever the step's type).  Eight
+    (src/backends/backend.hpp:943-947: the router's product is F32 whatever the step's type).  Eight
     one-token requests in one step: with a single key the softmax weight is exactly 1, so everything before the router is
     the plain implementation's arithmetic up to the order of float32 sums, and the engine's logits can be told apart from
     the logits a router reading rounded rows would give."""

@@ -202,7 +202,7 @@ def test_command_line_runs_a_configuration_with_random_weights(tmp_path):
 
 def test_command_line_bench_of_a_model(tmp_path):
     """`llmx bench --model DIR --p --n --r --seqs --depth` prints the reference's lines (`bench: pp16 ...`,
-    `bench: tg8 ...`, `bench: x3 tg8 ...`, ` @ d40` after a history; /root/reference/src/cli/main.cpp:1261-1270) and
+    `bench: tg8 ...`, `bench: x3 tg8 ...`, ` @ d40` after a history; src/cli/main.cpp:1261-1270) and
     leaves no request open between its runs (every run opens its requests anew in a pool made for one run)."""
     import re
     exe = os.path.join(ROOT, "bin", "llmx")

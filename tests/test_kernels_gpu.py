@@ -905,7 +905,7 @@ def test_attention_finds_a_far_key():
 # ---------------------------------------------------------------------------
 def test_route_topk_vectors():
     """Levels with ties, infinities and a NaN; k in {1, 8, 24}; bias on/off; normalize on/off.  The method (not the
-    data) follows /root/reference/tests/minimax_ops.cpp:74-139: ids equal a stable sort by float(s)+bias descending,
+    data) follows tests/minimax_ops.cpp:74-139: ids equal a stable sort by float(s)+bias descending,
     weights close to s/sum*scale, a row with a non-finite key gives no expert, a row alone equals the row in a batch."""
     o = ops()
     X = 24
@@ -1036,7 +1036,7 @@ def test_route_matches_plain_and_invariants():
 
 # ---------------------------------------------------------------------------
 def test_argmax_rows_vectors():
-    """Vectors the reference's own sampler test holds (/root/reference/tests/sampler.cpp:95-98) and the NaN rules."""
+    """Vectors the reference's own sampler test holds (tests/sampler.cpp:95-98) and the NaN rules."""
     o = ops()
     cases = [([0.5, 2.0, -1.0, 1.5], 1), ([-2.0, -0.5, -1.0], 1), ([1.0, 3.0, 0.0, 3.0], 1), ([3.0, 3.0, 3.0], 0),
              ([float("nan"), 5.0, 1.0], 0), ([1.0, float("nan"), 5.0], 2), ([float("-inf")] * 3, 0)]
@@ -1404,7 +1404,7 @@ def test_sampling_frequencies():
 
 
 def test_penalties():
-    """The reference's penalty cases (/root/reference/tests/sampler.cpp:101-113): a seen positive leader is divided, a
+    """The reference's penalty cases (tests/sampler.cpp:101-113): a seen positive leader is divided, a
     negative one multiplied, once however often it was seen."""
     o = ops()
 

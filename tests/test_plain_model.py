@@ -241,7 +241,7 @@ def _attention_weights(scale=1.0):
 
 def test_queries_and_keys_are_normed_and_values_are_not():
     """The norm (with the rotation) is applied to the q and k rows only; v goes to the cache as projected
-    (/root/reference/src/model/arch/minimax_m3.hpp:258-259 norm q and k, :264 writes v_rows untouched).  A norm's output
+    (src/model/arch/minimax_m3.hpp:258-259 norm q and k, :264 writes v_rows untouched).  A norm's output
     does not change when its input is scaled, so scaling W_q or W_k changes nothing (up to eps), while the output is
     linear in W_v: scaling W_v by c scales it by c, and W_v = 0 gives exactly 0.  Norming v as well, or forgetting the
     norm of q or k, breaks one of the three."""
@@ -266,7 +266,7 @@ def test_queries_and_keys_are_normed_and_values_are_not():
 
 
 def _bf16_by_hand(v: float) -> float:
-    """Round to nearest, ties to even, on the bits (/root/reference/src/core/bf16.hpp:5-11), without torch's conversion."""
+    """Round to nearest, ties to even, on the bits (src/core/bf16.hpp:5-11), without torch's conversion."""
     import struct
     u = struct.unpack("<I", struct.pack("<f", v))[0]
     u = (u + 0x7FFF + ((u >> 16) & 1)) & 0xFFFF0000
@@ -275,7 +275,7 @@ def _bf16_by_hand(v: float) -> float:
 
 def test_where_the_bfloat16_path_rounds():
     """The bfloat16 path rounds the inputs of weight products and what the cache stores, nothing else: sums, norms, the
-    softmax, the router's logits and the residual stay wide (/root/reference/src/backends/backend.hpp:943-962: the
+    softmax, the router's logits and the residual stay wide (src/backends/backend.hpp:943-962: the
     router's product is F32 whatever the step's dtype, the experts' three products read their inputs in the step's dtype
     and sum in F32).  Each site is fixed by a vector whose rounding is worked out by hand on the bits."""
     bf = torch.bfloat16

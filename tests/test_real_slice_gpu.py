@@ -1,8 +1,8 @@
 """The real layer sizes (hidden 3072, 48 query / 8 KV heads of 128, rotary 64, 256 experts top-8 of intermediate 1536,
 vocabulary 200,064) with random weights: against the plain implementation, and the cuttings against each other.
 
-Method of the reference's own parity runs (/root/reference/tests/minimax.py:63-90: the module's logits beside a
-straightforward forward pass; /root/reference/tools/model_logits.cpp:82-109: the same tokens whole and step by step).
+Method of the reference's own parity runs (tests/minimax.py:63-90: the module's logits beside a
+straightforward forward pass; tools/model_logits.cpp:82-109: the same tokens whole and step by step).
 Weights are generated on the device from (seed, tensor name); the plain implementation reads the same tensors by name,
 copied to the host as it touches them (only the experts a row picked), and a sample far into the largest tensor is
 checked against the generator's formula written out here.

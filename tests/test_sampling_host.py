@@ -7,7 +7,7 @@ from llmx_amd.sampling import SamplingParams, XorShift64
 
 
 def test_generator_follows_the_xorshift_definition():
-    """First outputs recomputed from the definition (/root/reference/src/inference/sampler.hpp:21-32)."""
+    """First outputs recomputed from the definition (src/inference/sampler.hpp:21-32)."""
     def step(x):
         m = (1 << 64) - 1
         x ^= (x << 13) & m
@@ -43,7 +43,7 @@ def test_defaults_and_ranges():
 
 
 def test_reference_transcription_on_small_rows():
-    """The slow sampler the GPU tests compare with: greedy vectors of /root/reference/tests/sampler.cpp:95-98 and simple draws."""
+    """The slow sampler the GPU tests compare with: greedy vectors of tests/sampler.cpp:95-98 and simple draws."""
     s = sampler_reference.sample
     assert s([0.5, 2.0, -1.0, 1.5], 0.0, 0, 1.0, 0.0, 0.3) == 1
     assert s([1.0, 3.0, 0.0, 3.0], 0.0, 0, 1.0, 0.0, 0.3) == 1

@@ -1,5 +1,5 @@
 """The scheduler's decisions, without a model: a simulated executor feeds it tokens
-(the reference tests its policy the same way: /root/reference/docs/TESTS.md:829)."""
+(the reference tests its policy the same way: docs/TESTS.md:829)."""
 
 import random
 
@@ -76,7 +76,7 @@ def test_eos_and_ignore_eos():
 
 def test_stop_sequences():
     """Generation ends when the generated ids end with a stop sequence; the completing token is kept (the reference
-    keeps the token that completes its stop text and does not feed it: /root/reference/src/inference/generate.hpp:29-36)."""
+    keeps the token that completes its stop text and does not feed it: src/inference/generate.hpp:29-36)."""
     s = Scheduler([GroupSpec("kv", 4, 100)], 3, 16, eos_token_id=EOS)
     seq = [5, 6, 7, 6, 7, 8, 9]
     s.submit(Request("one", [1, 2], SamplingParams(max_tokens=7, temp=0.0, stop=(7, 8))))
@@ -162,7 +162,7 @@ def test_random_loads_finish_and_return_everything(seed):
 
 def test_the_last_token_the_limit_allows_is_fed_without_logits():
     """At max_tokens the last token goes into the cache in the next step (no logits wanted) and then the request ends;
-    an end token and a token completing a stop sequence are never fed (/root/reference/src/inference/generate.hpp:28-45)."""
+    an end token and a token completing a stop sequence are never fed (src/inference/generate.hpp:28-45)."""
     groups = [GroupSpec("kv", 4, 100)]
     cache = CacheManager(groups, max_requests=3)
     s = Scheduler(groups, 3, 16, eos_token_id=EOS)

@@ -55,7 +55,7 @@ def test_reader_refusals(tmp_path, header, data, text):
 
 def test_a_key_twice_in_the_header_is_refused(tmp_path):
     """The standard JSON parser would silently keep the last of two equal keys
-    (/root/reference/src/format/safetensors.hpp:40-44,69,109 refuse them)."""
+    (src/format/safetensors.hpp:40-44,69,109 refuse them)."""
     entry = '{"dtype": "F32", "shape": [2], "data_offsets": [0, 8]}'
     raw_file(tmp_path / "twice.safetensors", '{"t": %s, "t": %s}' % (entry, entry), b"\0" * 8)
     with pytest.raises(SafetensorsError, match="header of .*twice.safetensors repeats key t"):
@@ -77,7 +77,7 @@ def test_metadata_must_be_an_object_of_strings(tmp_path):
 
 def test_a_tensor_at_an_unaligned_file_offset_is_refused(tmp_path):
     """Elements must lie at multiples of their size (of 4 bytes at most) in the file, so that the map can be read in place
-    (/root/reference/src/format/safetensors.hpp:123-126)."""
+    (src/format/safetensors.hpp:123-126)."""
     # a bfloat16 tensor of 3 elements pushes the float32 tensor behind it to an offset of 6
     header = {"h": {"dtype": "BF16", "shape": [3], "data_offsets": [0, 6]}, "f": {"dtype": "F32", "shape": [2], "data_offsets": [6, 14]}}
     raw_file(tmp_path / "odd.safetensors", header, b"\0" * 14)
@@ -95,7 +95,7 @@ def test_a_tensor_at_an_unaligned_file_offset_is_refused(tmp_path):
 
 
 def test_an_index_that_names_a_file_outside_its_folder_is_refused(tmp_path):
-    """/root/reference/src/format/safetensors.hpp:134-137: a file named by an index sits beside it."""
+    """src/format/safetensors.hpp:134-137: a file named by an index sits beside it."""
     write_safetensors(tmp_path / "part.safetensors", {"t": torch.zeros(2)})
     for bad in ("../part.safetensors", "sub/part.safetensors", "..", ""):
         (tmp_path / "model.safetensors.index.json").write_text(json.dumps({"weight_map": {"t": bad}}))
